@@ -1802,7 +1802,8 @@ class MatrixPartitionedTyings(_Handle):
 
 class MatrixPartitionedTyingsSolver:
     """GooseFEM::MatrixPartitionedTyingsSolver (MatrixPartitionedTyings.h:527-675): x_u from the
-    condensed system by an FP64 Jacobi-PCG (tol relative), x_d from the tyings; K' must be SPD."""
+    condensed system by an FP64 PCG (tol relative; multigrid-preconditioned on a Regular Quad4 cell,
+    else Jacobi), x_d from the tyings; K' must be SPD."""
 
     def __init__(self, tol=1e-12, maxiter=None):
         self.tol = tol
@@ -1831,7 +1832,7 @@ class MatrixPartitionedTyingsSolver:
 
 class MatrixPartitionedSolver:
     """GooseFEM::MatrixPartitionedSolver (MatrixPartitioned.h:526-640) for a symmetric positive
-    definite A_uu: x_u = A_uu^-1 (b_u - A_up x_p) by an FP64 Jacobi-preconditioned CG on the GPU
+    definite A_uu: x_u = A_uu^-1 (b_u - A_up x_p) by an FP64 preconditioned CG on the GPU
     (relative residual tol) instead of a sparse LDLT factorisation."""
 
     def __init__(self, tol=1e-12, maxiter=None):

@@ -11,6 +11,7 @@
 // (e, m, i) order, which is also the order of MatrixDiagonalPartitioned::assemble per DOF).
 #include <algorithm>
 
+#include "gf_gridmg.hpp"
 #include "gf_internal.hpp"
 #include "gf_wave.hpp"
 
@@ -40,6 +41,7 @@ struct gf_matpart_s {
     DBuf<double> work; // x_u, x_p, b_u, b_p, then the PCG vectors
     DBuf<double> red;  // reduction partials and scalars
     DBuf<int32_t> state;
+    GridMGPtr mg; // multigrid on A_uu where the mesh is a Regular Quad4 grid (else null)
 };
 
 // MatrixPartitionedTyings: the unpartitioned CSR K over the tied DOF numbering [u | p | d] and the
@@ -53,6 +55,7 @@ struct gf_mattyings_s {
     DBuf<double> work; // x, r, z, p, q, invd, rhs [nnu]; xfull, yfull, kdiag [ndof]; p2 [nnu]
     DBuf<double> red;
     DBuf<int32_t> state;
+    GridMGPtr mg; // multigrid on the condensed operator where the cell is a Regular Quad4 grid (else null)
 };
 
 namespace {
@@ -209,7 +212,7 @@ __global__ void k_node_from_part_sel(int64_t n, int64_t nnu, int which, const in
 // Two launches per iteration: the product (which also forms the search direction from the
 // previous iteration's z and p) and the x / r / z update.
 // Deterministic two-stage reductions: NPB blocks each store one partial sum, every consumer sums
-// the NPB partials in index order.  scal: [0], [1] rz by iteration parity, [2] rr, [3] bb,
+// the NPB partials in the same fixed order.  scal: [0], [1] rz by iteration parity, [2] rr, [3] bb,
 // [4] tol^2 bb.  state: [0] done, [1] iterations, [2] iteration cap.  Every kernel returns at once
 // when done is set, so launches queued past convergence leave the result alone.
 constexpr int PB = 256, NPB = 256;
@@ -219,13 +222,6 @@ __device__ inline void block_sum_store(double v, double* out)
 {
     const double t = block_sum<PB>(v);
     if (threadIdx.x == 0) *out = t;
-}
-
-__device__ inline double sum_partials(const double* partial)
-{
-    double s = 0.0;
-    for (int b = 0; b < NPB; ++b) s += partial[b];
-    return s;
 }
 
 // The sum of count partials for a whole block: thread t adds partials t, t + PB, ... in turn, then
@@ -263,11 +259,12 @@ __global__ void __launch_bounds__(PB) k_cg_init(int64_t n, const int32_t* __rest
     block_sum_store(abb, partial + 2 * NPB + blockIdx.x);
 }
 
-__global__ void k_cg_init_scal(const double* __restrict__ partial, double* __restrict__ scal, int32_t* __restrict__ state,
-                               double tol, int32_t maxiter)
+__global__ void __launch_bounds__(PB) k_cg_init_scal(const double* __restrict__ partial, double* __restrict__ scal,
+                                                     int32_t* __restrict__ state, double tol, int32_t maxiter)
 {
+    const double rz = block_sum_partials(partial, NPB), rr = block_sum_partials(partial + NPB, NPB),
+                 bb = block_sum_partials(partial + 2 * NPB, NPB);
     if (threadIdx.x != 0) return;
-    const double rz = sum_partials(partial), rr = sum_partials(partial + NPB), bb = sum_partials(partial + 2 * NPB);
     scal[0] = rz;
     scal[2] = rr;
     scal[3] = bb;
@@ -413,11 +410,10 @@ __global__ void __launch_bounds__(PB) k_cg_residual(int64_t n, const int32_t* __
     block_sum_store(abb, partial + NPB + blockIdx.x);
 }
 
-__global__ void k_cg_relres(const double* __restrict__ partial, double* __restrict__ out)
+__global__ void __launch_bounds__(PB) k_cg_relres(const double* __restrict__ partial, double* __restrict__ out)
 {
-    if (threadIdx.x != 0) return;
-    const double rr = sum_partials(partial), bb = sum_partials(partial + NPB);
-    out[0] = sqrt(rr / (bb > 0.0 ? bb : 1.0));
+    const double rr = block_sum_partials(partial, NPB), bb = block_sum_partials(partial + NPB, NPB);
+    if (threadIdx.x == 0) out[0] = sqrt(rr / (bb > 0.0 ? bb : 1.0));
 }
 
 // inverse diagonal of a CSR block
@@ -950,13 +946,36 @@ void matpart_cg(gf_matpart A, const double* rhs, double* xu, bool warm, double t
     const int32_t *rp = A->rowptr[0].p, *cl = A->col[0].p;
     const double* vl = A->val[0].p;
     int32_t st[2] = {0, 0};
+    auto finish = [&](int64_t its) {
+        // the true residual ||rhs - A_uu x_u|| / ||rhs||
+        k_cg_residual<<<NPB, PB, 0, s>>>(n, rp, cl, vl, rhs, W.cx, partial);
+        k_cg_relres<<<1, PB, 0, s>>>(partial, scal + 5);
+        check_launch();
+        GF_HIP(hipMemcpyAsync(xu, W.cx, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+        double res = 0.0;
+        GF_HIP(hipMemcpyAsync(&res, scal + 5, sizeof(double), hipMemcpyDeviceToHost, s));
+        if (its < 0) GF_HIP(hipMemcpyAsync(st, state, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        GF_HIP(hipStreamSynchronize(s));
+        if (iterations) *iterations = its < 0 ? st[1] : its;
+        if (relres) *relres = res;
+        return res;
+    };
+    if (A->mg) {
+        // a Regular Quad4 grid: multigrid-preconditioned iterations, independent of the grid's size
+        if (warm) GF_HIP(hipMemcpyAsync(W.cx, xu, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+        int64_t its = 0;
+        const GridMGStatus g = gridmg_solve(A->mg.get(), vl, rhs, W.cx, warm, tol, maxiter, &its, s);
+        if (g == GRIDMG_BAD_RHS) throw Error(GF_EINVAL, "non-finite right-hand side");
+        // otherwise, and where rounding keeps the true residual from following, the Jacobi iteration below
+        if (g == GRIDMG_CONVERGED && finish(its) <= 10.0 * tol) return;
+    }
     auto init = [&](bool from_x) {
         if (from_x)
             GF_HIP(hipMemcpyAsync(W.cx, xu, n * sizeof(double), hipMemcpyDeviceToDevice, s));
         else
             k_zero<<<nblocks(n, BS), BS, 0, s>>>(n, W.cx);
         k_cg_init<<<NPB, PB, 0, s>>>(n, rp, cl, vl, rhs, W.cx, W.invd, W.cr, W.cz, W.cp, partial);
-        k_cg_init_scal<<<1, 64, 0, s>>>(partial, scal, state, tol, static_cast<int32_t>(maxiter));
+        k_cg_init_scal<<<1, PB, 0, s>>>(partial, scal, state, tol, static_cast<int32_t>(maxiter));
         check_launch();
         GF_HIP(hipMemcpyAsync(st, state, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
         GF_HIP(hipStreamSynchronize(s));
@@ -990,17 +1009,7 @@ void matpart_cg(gf_matpart A, const double* rhs, double* xu, bool warm, double t
         if (chunk > 0 && pipe.wait(chunk - 1)[0]) st[0] = 1;
         ++chunk;
     }
-    // the true residual ||rhs - A_uu x_u|| / ||rhs||
-    k_cg_residual<<<NPB, PB, 0, s>>>(n, rp, cl, vl, rhs, W.cx, partial);
-    k_cg_relres<<<1, 64, 0, s>>>(partial, scal + 5);
-    check_launch();
-    GF_HIP(hipMemcpyAsync(xu, W.cx, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-    double res = 0.0;
-    GF_HIP(hipMemcpyAsync(&res, scal + 5, sizeof(double), hipMemcpyDeviceToHost, s));
-    GF_HIP(hipMemcpyAsync(st, state, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    GF_HIP(hipStreamSynchronize(s));
-    if (iterations) *iterations = st[1];
-    if (relres) *relres = res;
+    const double res = finish(-1);
     if (!(res <= 10.0 * tol))
         throw Error(GF_ENOTCONV, "PCG on A_uu did not reach the tolerance (true residual " + std::to_string(res) + ")");
 }
@@ -1015,6 +1024,7 @@ void matpart_split(gf_matpart A, hipStream_t s)
         const int64_t n = A->nnz[b];
         if (n) k_take<<<nblocks(n, BS), BS, 0, s>>>(n, A->src[b].p, val, A->val[b].p);
     }
+    gridmg_invalidate(A->mg.get());
     const int64_t nu = A->nrows[0];
     if (nu) k_csr_invdiag<<<nblocks(nu, BS), BS, 0, s>>>(nu, A->rowptr[0].p, A->col[0].p, A->val[0].p, work_of(A).invd);
     check_launch();
@@ -1082,6 +1092,16 @@ int gf_matpart_create(gf_matpart* out, gf_vecpart p)
                 A->src[b].upload(bsrc[b]);
                 A->val[b].alloc(A->nnz[b]);
             }
+            std::vector<int64_t> same(nu);
+            for (int64_t u = 0; u < nu; ++u) same[u] = u;
+            const auto& dofs = p->v->dofs_h;
+            A->mg = gridmg_create(
+                p->v, nu,
+                [&](int64_t node, int c) {
+                    const int64_t r = renum[dofs[node * p->v->ndim + c]];
+                    return r < nu ? r : int64_t(-1);
+                },
+                brp[0], bcl[0], same);
             A->work.alloc(2 * (nu + np) + 8 * nu);
             A->red.alloc(3 * NPB + 8 + nblocks(LPR * nu, PB));
             A->state.alloc(4);
@@ -1292,6 +1312,28 @@ int gf_mattyings_create(gf_mattyings* out, gf_vector v, int64_t nnu, int64_t nnp
             A->ud_rp.upload(trp);
             A->ud_cl.upload(tcl);
             A->ud_v.upload(tv);
+            // the unknown that a DOF stands for in the condensed system: itself, its partner's if it is a
+            // copy of that one (plus prescribed terms), -1 for none, -2 for a combination
+            const int64_t nni = nnu + nnp;
+            std::vector<int64_t> u_of(A->ndof);
+            for (int64_t d = 0; d < A->ndof; ++d) {
+                if (d < nni) u_of[d] = d < nnu ? d : -1;
+                else {
+                    const int64_t k = du_rp[d - nni], cnt = du_rp[d - nni + 1] - k;
+                    u_of[d] = cnt == 0 ? -1 : cnt == 1 && du_v[k] == 1.0 ? du_cl[k] : -2;
+                }
+            }
+            int64_t knr = 0, knz = 0;
+            gf_matrix_sizes(A->K, &knr, &knz);
+            const int32_t *krp = nullptr, *kcl = nullptr;
+            const double* kv = nullptr;
+            gf_matrix_csr(A->K, &krp, &kcl, &kv);
+            rp.resize(knr + 1);
+            cl.resize(knz);
+            GF_HIP(hipMemcpy(rp.data(), krp, rp.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            if (knz) GF_HIP(hipMemcpy(cl.data(), kcl, cl.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            A->mg = gridmg_create(
+                v, nnu, [&](int64_t node, int c) { return u_of[v->dofs_h[node * v->ndim + c]]; }, rp, cl, u_of);
             A->work.alloc(8 * nnu + 3 * A->ndof);
             A->red.alloc(3 * NPB + 8 + nblocks(LPR * nnu, PB)); // + the fused product's p.q partials
             A->state.alloc(4);
@@ -1330,6 +1372,7 @@ int gf_mattyings_assemble(gf_mattyings A, const double* elemmat, void* stream)
         const double* val = nullptr;
         gf_matrix_csr(A->K, &rp, &cl, &val);
         hipStream_t s = S(stream);
+        gridmg_invalidate(A->mg.get());
         double* kd = A->work.p + 7 * A->nnu + 2 * A->ndof;
         double* invd = A->work.p + 5 * A->nnu;
         k_csr_diag<<<nblocks(A->ndof, BS), BS, 0, s>>>(A->ndof, rp, cl, val, kd);
@@ -1381,10 +1424,37 @@ int gf_mattyings_solve(gf_mattyings A, const double* b, double* x, double tol, i
         ty_product(A, nullptr, Xp, cq, nullptr, nullptr, s);
         if (nu) k_ty_rhs<<<nblocks(nu, BS), BS, 0, s>>>(nu, ni, bfull.p, A->ud_rp.p, A->ud_cl.p, A->ud_v.p, cq, rhs);
         check_launch();
+        // the true residual of the condensed system for the solution in cx
+        auto residual = [&] {
+            double res = 0.0;
+            ty_product(A, cx, nullptr, cq, nullptr, nullptr, s);
+            k_cg_residual_vec<<<NPB, PB, 0, s>>>(nu, rhs, cq, partial);
+            k_cg_relres<<<1, PB, 0, s>>>(partial, scal + 5);
+            check_launch();
+            GF_HIP(hipMemcpyAsync(&res, scal + 5, sizeof(double), hipMemcpyDeviceToHost, s));
+            GF_HIP(hipStreamSynchronize(s));
+            return res;
+        };
         int32_t st[2] = {0, 0};
-        if (nu) {
+        int64_t its = 0;
+        double res = 0.0;
+        bool solved = nu == 0;
+        if (A->mg) {
+            // a Regular Quad4 cell: multigrid-preconditioned iterations, independent of the grid's size
+            const int32_t *krp = nullptr, *kcl = nullptr;
+            const double* kv = nullptr;
+            gf_matrix_csr(A->K, &krp, &kcl, &kv);
+            const GridMGStatus g = gridmg_solve(A->mg.get(), kv, rhs, cx, false, tol, maxiter, &its, s);
+            if (g == GRIDMG_BAD_RHS) throw Error(GF_EINVAL, "non-finite right-hand side");
+            // otherwise, and where rounding keeps the true residual from following, the Jacobi iteration
+            if (g == GRIDMG_CONVERGED) {
+                res = residual();
+                solved = res <= 10.0 * tol;
+            }
+        }
+        if (!solved) {
             k_ty_init<<<NPB, PB, 0, s>>>(nu, rhs, invd, cx, cr, cz, cp, partial);
-            k_cg_init_scal<<<1, 64, 0, s>>>(partial, scal, state, tol, static_cast<int32_t>(maxiter));
+            k_cg_init_scal<<<1, PB, 0, s>>>(partial, scal, state, tol, static_cast<int32_t>(maxiter));
             check_launch();
             GF_HIP(hipMemcpyAsync(st, state, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
             GF_HIP(hipStreamSynchronize(s));
@@ -1425,11 +1495,9 @@ int gf_mattyings_solve(gf_mattyings A, const double* b, double* x, double tol, i
                 if (chunk > 0 && pipe.wait(chunk - 1)[0]) st[0] = 1;
                 ++chunk;
             }
-            // true residual of the condensed system
-            ty_product(A, cx, nullptr, cq, nullptr, nullptr, s);
-            k_cg_residual_vec<<<NPB, PB, 0, s>>>(nu, rhs, cq, partial);
-            k_cg_relres<<<1, 64, 0, s>>>(partial, scal + 5);
-            check_launch();
+            res = residual();
+            GF_HIP(hipMemcpy(st, state, 2 * sizeof(int32_t), hipMemcpyDeviceToHost));
+            its = st[1];
         }
         // x = AsNode(X_u, X_p, C_du X_u + C_dp X_p): u and d entries solved, p entries as given
         k_ty_expand<<<nblocks(nd, BS), BS, 0, s>>>(nu, A->nnp, A->nnd, cx, Xp, A->du_rp.p, A->du_cl.p, A->du_v.p,
@@ -1437,11 +1505,8 @@ int gf_mattyings_solve(gf_mattyings A, const double* b, double* x, double tol, i
         check_launch();
         rc = gf_vector_as_node_dofval(A->v, xfull, x, stream);
         if (rc != GF_OK) throw Error(rc, gf_last_error());
-        double res = 0.0;
-        if (nu) GF_HIP(hipMemcpyAsync(&res, scal + 5, sizeof(double), hipMemcpyDeviceToHost, s));
-        GF_HIP(hipMemcpyAsync(st, state, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        GF_HIP(hipStreamSynchronize(s));
-        if (iterations) *iterations = nu ? st[1] : 0;
+        GF_HIP(hipStreamSynchronize(s)); // xin and bfull are released here
+        if (iterations) *iterations = its;
         if (relres) *relres = res;
         if (!(res <= 10.0 * tol))
             throw Error(GF_ENOTCONV, "PCG on the condensed system did not reach the tolerance (true residual " +

@@ -1605,7 +1605,7 @@ private:
 };
 
 /* MatrixPartitionedSolver  (MatrixPartitioned.h:526-640): x_u = A_uu^-1 (b_u - A_up x_p) by an FP64
- * Jacobi-preconditioned CG on the device (A_uu symmetric positive definite) in place of the
+ * preconditioned CG on the device (A_uu symmetric positive definite) in place of the
  * reference's SimplicialLDLT.  Throws if the true relative residual exceeds 10 tol. */
 class MatrixPartitionedSolver {
 public:
@@ -1760,7 +1760,7 @@ private:
 // =================================================================================================
 // MatrixPartitionedTyings + MatrixPartitionedTyingsSolver (include/GooseFEM/MatrixPartitionedTyings.h)
 // for any element matrices: K as one CSR over the tied numbering [u | p | d], the condensed system
-// solved by a matrix-free FP64 Jacobi-PCG (K' symmetric positive definite) instead of LDLT
+// solved by a matrix-free FP64 PCG (K' symmetric positive definite) instead of LDLT
 // =================================================================================================
 
 class MatrixPartitionedTyings {

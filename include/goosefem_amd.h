@@ -280,8 +280,10 @@ int gf_material_elastic_tangent_f32(int64_t nq, int tdim, const double* K_q, con
  * numbering [u | p | d] (a gf_matrix over v, whose dofs are Tyings::Periodic's dofs()); the
  * condensed operator K'_uu = K_uu + K_ud C_du + C_ud K_du + C_ud K_dd C_du (:661-663) is applied
  * matrix-free (expand x_d = C_du x_u + C_dp x_p, one CSR product, fold y_u + C_ud y_d) inside an
- * FP64 Jacobi-preconditioned CG instead of an LDLT factorisation, so K'_uu must be symmetric
- * positive definite.  C_du [nnd, nnu] and C_dp [nnd, nnp] are host CSR (int64 rowptr / col, FP64
+ * FP64 preconditioned CG instead of an LDLT factorisation, so K'_uu must be symmetric positive
+ * definite.  The preconditioner is a multigrid V-cycle where the cell is a Regular Quad4 grid of at
+ * least 64 nodes whose dependent DOFs are copies of u DOFs (plus prescribed terms), which makes the
+ * iteration count independent of the grid, else (and should that not converge) the diagonal.  C_du [nnd, nnu] and C_dp [nnd, nnp] are host CSR (int64 rowptr / col, FP64
  * values), as Tyings::Periodic::Cdu() / Cdp() (TyingsPeriodic.h:244-256).
  * ============================================================================================== */
 int gf_mattyings_create(gf_mattyings* out, gf_vector v, int64_t nnu, int64_t nnp, int64_t nnd, const int64_t* du_rowptr,
@@ -290,7 +292,7 @@ int gf_mattyings_create(gf_mattyings* out, gf_vector v, int64_t nnu, int64_t nnp
 int gf_mattyings_destroy(gf_mattyings A);
 /* the unpartitioned CSR (Todense via gf_matrix_todense) */
 int gf_mattyings_matrix(gf_mattyings A, gf_matrix* K);
-/* assemble(elemmat)  (MatrixPartitionedTyings.h:210-305): K, and the Jacobi diagonal of K' */
+/* assemble(elemmat)  (MatrixPartitionedTyings.h:210-305): K, and the diagonal of K' */
 int gf_mattyings_assemble(gf_mattyings A, const double* elemmat, void* stream);
 /* MatrixPartitionedTyingsSolver::solve(A, b, x)  (:540-564) on nodevecs: B_u = b_u + C_ud b_d,
  * X_u = K'^-1 (B_u - K'_up X_p), X_d = C_du X_u + C_dp X_p; writes x's u and d entries, keeps its
@@ -464,9 +466,11 @@ int gf_matrix_todense(gf_matrix A, double* out, void* stream);
  * (e, m, i, n, j) order as setFromTriplets (:156-210): assembly is bit-exact.  Products run one
  * sum per row over ascending columns of the first block, then of the second: the order Eigen
  * evaluates "A_uu X_u + A_up X_p" for a column-major matrix (dst = A X_u; dst += B X_p).
- * Solve factorises nothing: x_u = A_uu^-1 (b_u - A_up x_p) by a Jacobi-preconditioned CG on A_uu
+ * Solve factorises nothing: x_u = A_uu^-1 (b_u - A_up x_p) by a preconditioned CG on A_uu
  * (FP64, deterministic reductions), so A_uu must be symmetric positive definite (the reference's
- * SimplicialLDLT also takes indefinite symmetric matrices).  set() / add() of dense sub-matrices
+ * SimplicialLDLT also takes indefinite symmetric matrices).  The preconditioner is a multigrid V-cycle
+ * where the mesh is a Regular Quad4 grid of at least 64 nodes with one DOF per node and component
+ * (opposite edges may share theirs), else (and should that not converge) the diagonal.  set() / add() of dense sub-matrices
  * are not provided (the sparsity pattern is the mesh's).
  * ============================================================================================== */
 

@@ -1,0 +1,166 @@
+"""The multigrid-preconditioned solve of the partitioned and the tied sparse matrices on Regular Quad4
+grids (goosefem_amd/csrc/gf_gridmg.hip): against a sparse direct solve of the same CSR, at grid sizes
+around the edges of its tiles (20 x 4 and 22 x 6 owned nodes), its coarse kernel (256 nodes) and its
+threshold (64 nodes), on elongated, wrapped, renumbered and prescribed-inside grids; what it hands back
+to the Jacobi iteration; bad input."""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as sl
+
+import oracle
+from oracle import QUAD4_PLANAR
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gf():
+    import torch
+
+    import goosefem_amd
+
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    goosefem_amd.lib()
+    return goosefem_amd
+
+
+def host(t):
+    import torch
+
+    torch.cuda.synchronize()
+    return t.detach().cpu().numpy()
+
+
+def stiffness(conn, coor, rng, contrast=0.4):
+    q = oracle.Quadrature(QUAD4_PLANAR, oracle.Vector(conn, np.arange(coor.size).reshape(coor.shape)).AsElement(coor))
+    G = np.exp(contrast * rng.standard_normal((q.nelem, q.nip)))
+    return q.Int_gradN_dot_tensor4_dot_gradNT_dV(oracle.elastic_tangent(np.full_like(G, 10.0), G))
+
+
+def check(gf, A, b_u, x_u, tol):
+    """x_u solves A_uu x_u = b_u to the solver's contract, and equals the direct solution to the condition
+    of the system: |x - y| <= |A^-1| |r|, |r| <= 10 tol |b|, with |A^-1| |b| / |x| below 1e5 for elastic
+    plates of these sizes (their lowest mode is resolved by 250 elements at most)."""
+    rp, cl, v = (host(t) for t in A.csr(0))
+    M = sp.csr_matrix((v, cl, rp), shape=(A.nnu, A.nnu))
+    assert np.linalg.norm(b_u - M @ x_u) <= 10 * tol * np.linalg.norm(b_u)
+    y = sl.spsolve(M.tocsc(), b_u)
+    assert np.linalg.norm(x_u - y) <= 1e6 * tol * np.linalg.norm(y)
+    return M
+
+
+GRIDS = [(7, 7), (8, 6), (7, 6), (15, 15), (16, 15), (16, 16), (19, 3), (20, 4), (21, 5), (22, 6), (23, 11), (40, 8),
+         (41, 9), (43, 37), (64, 31), (65, 66), (250, 5), (5, 120)]
+
+
+@pytest.mark.parametrize("nx,ny", GRIDS)
+def test_plate(gf, nx, ny):
+    rng = np.random.default_rng(nx * 1000 + ny)
+    coor, conn = oracle.quad4_regular(nx, ny)
+    coor = coor + rng.uniform(-0.1, 0.1, coor.shape)
+    dofs = rng.permutation(coor.size).reshape(coor.shape)  # any numbering
+    fixed = np.concatenate((dofs[: nx + 1].ravel(), dofs[rng.choice(np.arange(nx + 1, coor.shape[0]), 3, False), 0]))
+    A = gf.MatrixPartitioned(conn, dofs, fixed)
+    solver = gf.MatrixPartitionedSolver()
+    for k in range(2):  # a second assembly is seen by the next solve
+        A.assemble(stiffness(conn, coor, rng))
+        b_u, x_p = rng.standard_normal(A.nnu), np.zeros(A.nnp)
+        x = host(solver.Solve_u(A, b_u, x_p))
+        M = check(gf, A, b_u, x, solver.tol)
+        assert solver.relres <= 10 * solver.tol
+        if (nx + 1) * (ny + 1) >= 64 and max(nx, ny) >= 6:
+            assert solver.iterations <= 60  # the Jacobi iteration takes more on all but the smallest
+        again = host(solver.Solve_u(A, b_u, x_p))
+        assert np.array_equal(x, again)
+    # a start: the solution itself needs no iteration, one that is not finite is replaced by zero
+    it = solver.iterations
+    loose = gf.MatrixPartitionedSolver(tol=1e-9)
+    warm = host(loose.Solve_u(A, M @ x, x_p, x_u0=x))
+    assert loose.iterations == 0 and np.array_equal(warm, x)
+    assert np.array_equal(host(solver.Solve_u(A, b_u, x_p, x_u0=np.full(A.nnu, np.nan))), x) and solver.iterations == it
+    with pytest.raises(gf.GooseFEMError) as e:
+        solver.Solve_u(A, np.where(np.arange(A.nnu) == 1, np.nan, b_u), x_p)
+    assert e.value.code == gf.GF_EINVAL
+
+
+@pytest.mark.parametrize("nx,ny,px,py", [(9, 9, 1, 0), (6, 12, 1, 0), (31, 20, 0, 1), (5, 40, 1, 0), (37, 6, 1, 1),
+                                         (40, 40, 1, 1)])
+def test_wrapped_numbering(gf, nx, ny, px, py):
+    # DOFs shared by opposite edges; (5, 40, 1, 0) wraps too few elements and takes the Jacobi iteration
+    rng = np.random.default_rng(nx + 100 * ny)
+    coor, conn = oracle.quad4_regular(nx, ny)
+    dofs = np.arange(coor.size).reshape(ny + 1, nx + 1, 2)
+    if px:
+        dofs[:, nx] = dofs[:, 0]
+    if py:
+        dofs[ny] = dofs[0]
+    _, dofs = np.unique(dofs.ravel(), return_inverse=True)
+    dofs = dofs.reshape(-1, 2)
+    fixed = np.unique(dofs[0] if px and py else dofs[: nx + 1] if px else dofs[:: nx + 1])
+    A = gf.MatrixPartitioned(conn, dofs, fixed)
+    A.assemble(stiffness(conn, coor, rng))
+    b_u = rng.standard_normal(A.nnu)
+    solver = gf.MatrixPartitionedSolver(tol=1e-11)
+    check(gf, A, b_u, host(solver.Solve_u(A, b_u, np.zeros(A.nnp))), solver.tol)
+    assert nx < 6 or solver.iterations <= 60
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_matrices_the_cycle_is_not_made_for(gf, sign):
+    # symmetric positive definite but random: solved; negative definite: the cycle's scaling is positive,
+    # so the method breaks down at once and the Jacobi iteration, which does not mind, solves it
+    rng = np.random.default_rng(5)
+    coor, conn = oracle.quad4_regular(17, 13)
+    dofs = np.arange(coor.size).reshape(coor.shape)
+    a = rng.random((conn.shape[0], 8, 8))
+    A = gf.MatrixPartitioned(conn, dofs, dofs[:18].ravel())
+    A.assemble(sign * (a @ a.transpose(0, 2, 1) + np.eye(8)))
+    b_u = rng.standard_normal(A.nnu)
+    solver = gf.MatrixPartitionedSolver(tol=1e-12)
+    check(gf, A, b_u, host(solver.Solve_u(A, b_u, np.zeros(A.nnp))), solver.tol)
+
+
+def test_iteration_cap(gf):
+    coor, conn = oracle.quad4_regular(30, 30)
+    dofs = np.arange(coor.size).reshape(coor.shape)
+    A = gf.MatrixPartitioned(conn, dofs, dofs[:31].ravel())
+    A.assemble(stiffness(conn, coor, np.random.default_rng(0)))
+    with pytest.raises(gf.GooseFEMError) as e:
+        gf.MatrixPartitionedSolver(maxiter=3).Solve_u(A, np.ones(A.nnu), np.zeros(A.nnp))
+    assert e.value.code == gf.GF_ENOTCONV
+
+
+@pytest.mark.parametrize("nx,ny", [(6, 11), (7, 7), (17, 16), (25, 41), (64, 6)])
+def test_tied_cell(gf, nx, ny):
+    # the condensed solve of a periodic cell against a sparse direct condensation
+    rng = np.random.default_rng(nx + 100 * ny)
+    mesh = gf.Mesh.Quad4.Regular(nx, ny)
+    control = gf.Tyings.Control(mesh.coor, mesh.dofs)
+    iip = np.concatenate((control.controlDofs.ravel(), control.dofs[mesh.nodesOrigin].ravel()))
+    ty = gf.Tyings.Periodic(control.coor, control.dofs, control.controlDofs, mesh.nodesPeriodic, iip)
+    A = gf.MatrixPartitionedTyings(mesh.conn, ty.dofs, ty.Cdu_csr, ty.Cdp_csr)
+    em = stiffness(mesh.conn, mesh.coor, rng)
+    A.assemble(em)
+    dof = ty.dofs[mesh.conn].reshape(mesh.nelem, 8)
+    K = sp.csr_matrix((em.ravel(), (np.repeat(dof, 8, axis=1).ravel(), np.tile(dof, (1, 8)).ravel())),
+                      shape=(A.ndof, A.ndof))
+    T = sp.vstack((sp.identity(A.nni), sp.hstack((sp.csr_matrix(ty.Cdu), sp.csr_matrix(ty.Cdp))))).tocsr()
+    Kc = (T.T @ K @ T).tocsr()
+    b = rng.standard_normal(control.coor.shape)
+    x = np.zeros_like(b)
+    pre = (ty.dofs >= ty.nnu) & (ty.dofs < ty.nni)
+    x[pre] = 1e-2 * rng.standard_normal(pre.sum())
+    bd, xd = np.zeros(A.ndof), np.zeros(A.ndof)
+    bd[ty.dofs], xd[ty.dofs] = b, x
+    u, p = slice(0, ty.nnu), slice(ty.nnu, ty.nni)
+    rhs = (T.T @ bd)[u] - Kc[u, p] @ xd[p]
+    xi = xd[: ty.nni].copy()
+    xi[u] = sl.spsolve(Kc[u, u].tocsc(), rhs)
+    solver = gf.MatrixPartitionedTyingsSolver(tol=1e-12)
+    got = host(solver.Solve(A, b, x))
+    assert solver.relres <= 10 * solver.tol and solver.iterations <= 60
+    ref = (T @ xi)[ty.dofs]
+    assert np.linalg.norm(got - ref) <= 1e6 * solver.tol * np.linalg.norm(ref)
+    assert np.array_equal(got, host(solver.Solve(A, b, x)))
