@@ -56,11 +56,11 @@ struct gf_pcg_s {
     DBuf<double> partial;  // [4][NBR]
     DBuf<double> scal;     // [8]: rz (2 slots), bb, rr, tol2, ...
     DBuf<int32_t> state;   // [0] done, [1] iterations, [2] maxiter
-    // structured periodic Quad4 operator (Regular n x n cell, periodic tyings, uniform geometry)
+    // structured periodic operator (Regular cell, periodic tyings, uniform geometry)
     bool structured = false;
-    int sn = 0, ntiles = 0, ntx = 0, per_xcd = 0;
+    int snx = 0, sny = 0, snz = 0, ntiles = 0, ntx = 0, per_xcd = 0;
     double sh_g[32] = {}, sh_v[4] = {};
-    DBuf<int32_t> sidx; // [n^d * nd] u-DOF of grid node component c, or -1
+    DBuf<int32_t> sidx; // [nodes of the cell * nd] u-DOF of grid node component c, or -1
     int nty = 0;
     DBuf<double> ke8;   // Hex8: [2][24][24] element matrices per unit K and per unit G
     DBuf<double> sr[2], sw[2], ss[2]; // Quad4 single-reduction iteration: r, w, s by iteration parity
@@ -114,19 +114,32 @@ __device__ inline void quad4_planar_qp_force(const double* g, double v, const do
     }
 }
 
-// ---- structured periodic operator: Quad4 Regular n x n cell with periodic tyings ---------------------
+// ---- structured periodic operator: Quad4 Regular nx x ny cell with periodic tyings -------------------
 // Every element has the same dN/dx and dV (Regular mesh), so they are kernel arguments.  The tied
 // operator K' x_u on a periodic field is the element-force assembly on the torus: node (i, j)
-// collects the elements (i-1, j-1), (i, j-1), (i-1, j), (i, j) taken modulo n (MatrixPartitionedTyings
-// condensation with C_du = periodic copy, MatrixPartitionedTyings.h:655-674).  sidx maps grid node
-// (i, j), component c to its u-DOF, or -1 for a prescribed DOF (the origin), whose value is 0.
+// collects the elements (i-1, j-1), (i, j-1), (i-1, j), (i, j) taken modulo nx, ny
+// (MatrixPartitionedTyings condensation with C_du = periodic copy, MatrixPartitionedTyings.h:655-674).
+// sidx maps grid node (i, j), component c to its u-DOF, or -1 for a prescribed DOF (the origin), whose
+// value is 0.  The last tile of a row or column owns what is left of it: the indices of the nodes and
+// elements past the cell's end that no owned node needs are clamped into range.
+// Any size takes these kernels (a 250 x 250 cell: 66 -> 22 ms per solve against the general operator's
+// four launches per iteration, each of 5 to 9 us).
+
+// line or element i of a direction of n, one period out of range at most where it is used
+__device__ inline int wrap_line(int i, int n)
+{
+    i += i < 0 ? n : 0;
+    i -= i >= n ? n : 0;
+    return min(i, n - 1);
+}
+
 struct ShapeQ4 {
     double g[4][8];
     double v[4];
 };
 
 template <int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int n, int ntx, int per_xcd, ShapeQ4 sh,
+__global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int nx, int ny, int ntx, int per_xcd, ShapeQ4 sh,
                                                                const int32_t* __restrict__ sidx,
                                                                const double* __restrict__ Ke,
                                                                const double* __restrict__ Ge,
@@ -145,12 +158,8 @@ __global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int n, int ntx, i
     // halo tile of the operand (periodic wrap, prescribed DOFs read as 0)
     for (int t = threadIdx.x; t < HX * HY; t += NT) {
         const int ly = t / HX, lx = t - (t / HX) * HX;
-        int gi = x0 - 1 + lx, gj = y0 - 1 + ly;
-        gi += gi < 0 ? n : 0;
-        gi -= gi >= n ? n : 0;
-        gj += gj < 0 ? n : 0;
-        gj -= gj >= n ? n : 0;
-        const int64_t k = (static_cast<int64_t>(gj) * n + gi) * 2;
+        const int gi = wrap_line(x0 - 1 + lx, nx), gj = wrap_line(y0 - 1 + ly, ny);
+        const int64_t k = (static_cast<int64_t>(gj) * nx + gi) * 2;
         const int32_t d0 = sidx[k], d1 = sidx[k + 1];
         s_x[t] = make_double2(d0 >= 0 ? x[d0] : 0.0, d1 >= 0 ? x[d1] : 0.0);
     }
@@ -158,10 +167,8 @@ __global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int n, int ntx, i
     // element forces of the (TX+1) x (TY+1) elements touching the tile
     for (int t = threadIdx.x; t < EX * EY; t += NT) {
         const int ly = t / EX, lx = t - (t / EX) * EX;
-        int ei = x0 - 1 + lx, ej = y0 - 1 + ly;
-        ei += ei < 0 ? n : 0;
-        ej += ej < 0 ? n : 0;
-        const int64_t e = static_cast<int64_t>(ej) * n + ei;
+        const int ei = wrap_line(x0 - 1 + lx, nx), ej = wrap_line(y0 - 1 + ly, ny);
+        const int64_t e = static_cast<int64_t>(ej) * nx + ei;
         const int n0 = ly * HX + lx;
         const int nid[4] = {n0, n0 + 1, n0 + HX + 1, n0 + HX};
         double u[4][2], f[4][2];
@@ -192,8 +199,9 @@ __global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int n, int ntx, i
     f1 += s_f[l0 + EX][3];
     f0 += s_f[l0 + EX + 1][0];
     f1 += s_f[l0 + EX + 1][1];
-    const int64_t k = (static_cast<int64_t>(y0 + oly) * n + x0 + olx) * 2;
-    const int32_t d0 = sidx[k], d1 = sidx[k + 1];
+    const bool own = x0 + olx < nx && y0 + oly < ny;
+    const int64_t k = own ? (static_cast<int64_t>(y0 + oly) * nx + x0 + olx) * 2 : 0;
+    const int32_t d0 = own ? sidx[k] : -1, d1 = own ? sidx[k + 1] : -1;
     const double2 po = s_x[(oly + 1) * HX + olx + 1]; // the operand at the owned node
     double acc = 0.0;
     if (d0 >= 0) {
@@ -220,7 +228,7 @@ __global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int n, int ntx, i
 // alpha (slots by parity), the iteration count and the done flag.
 template <int TX, int TY>
 __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
-    int n, int ntx, int ntiles, int per_xcd, ShapeQ4 sh, const int32_t* __restrict__ sidx,
+    int nx, int ny, int ntx, int ntiles, int per_xcd, ShapeQ4 sh, const int32_t* __restrict__ sidx,
     const double* __restrict__ Ke, const double* __restrict__ Ge, const double* __restrict__ invd,
     const double* __restrict__ rc, const double* __restrict__ wc, const double* __restrict__ sc,
     double* __restrict__ rn, double* __restrict__ wn, double* __restrict__ sn_, double* __restrict__ p,
@@ -250,12 +258,8 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
         hd[j][0] = hd[j][1] = -1;
         if (t < HX * HY) {
             const int ly = t / HX, lx = t - (t / HX) * HX;
-            int gi = x0 - 1 + lx, gj = y0 - 1 + ly;
-            gi += gi < 0 ? n : 0;
-            gi -= gi >= n ? n : 0;
-            gj += gj < 0 ? n : 0;
-            gj -= gj >= n ? n : 0;
-            const int64_t k = (static_cast<int64_t>(gj) * n + gi) * 2;
+            const int gi = wrap_line(x0 - 1 + lx, nx), gj = wrap_line(y0 - 1 + ly, ny);
+            const int64_t k = (static_cast<int64_t>(gj) * nx + gi) * 2;
             hd[j][0] = sidx[k];
             hd[j][1] = sidx[k + 1];
         }
@@ -270,8 +274,9 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
             hs[j][c] = it == 0 ? 0.0 : sc[d];
             hi[j][c] = invd[d];
         }
-    const int64_t ko = (static_cast<int64_t>(y0 + oly) * n + x0 + olx) * 2;
-    const int32_t od[2] = {sidx[ko], sidx[ko + 1]};
+    const bool own = x0 + olx < nx && y0 + oly < ny;
+    const int64_t ko = own ? (static_cast<int64_t>(y0 + oly) * nx + x0 + olx) * 2 : 0;
+    const int32_t od[2] = {own ? sidx[ko] : -1, own ? sidx[ko + 1] : -1};
     double op[2], ox[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -286,10 +291,8 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
         ek[j] = eg[j] = 0.0;
         if (t < EX * EY) {
             const int ly = t / EX, lx = t - (t / EX) * EX;
-            int ei = x0 - 1 + lx, ej = y0 - 1 + ly;
-            ei += ei < 0 ? n : 0;
-            ej += ej < 0 ? n : 0;
-            const int64_t e = static_cast<int64_t>(ej) * n + ei;
+            const int ei = wrap_line(x0 - 1 + lx, nx), ej = wrap_line(y0 - 1 + ly, ny);
+            const int64_t e = static_cast<int64_t>(ej) * nx + ei;
             ek[j] = Ke[e];
             eg[j] = Ge[e];
         }
@@ -421,12 +424,13 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
     }
 }
 
-// Hex8 Regular n^3 cell with periodic tyings: identical element geometry makes the element
+// Hex8 Regular nx x ny x nz cell with periodic tyings: identical element geometry makes the element
 // stiffness K_e = K_e,bulk KK + G_e KG with two fixed 24 x 24 matrices (isotropic linear elasticity,
 // C = K I(x)I + 2G (I_sym - I(x)I/3)).  Each thread owns one node and sums, over its 8 elements,
 // the node's 3 rows of K_e u_e; the x halo of the 8 x 8 x 4 node tile sits in LDS (per component).
 template <int TX, int TY, int TZ>
-__global__ void __launch_bounds__(TX * TY * TZ) k_apply_periodic_h8(int n, int ntx, int nty, const double* __restrict__ kkg,
+__global__ void __launch_bounds__(TX * TY * TZ) k_apply_periodic_h8(int nx, int ny, int nz, int ntx, int nty,
+                                                                    const double* __restrict__ kkg,
                                                                     const int32_t* __restrict__ sidx,
                                                                     const double* __restrict__ Ke,
                                                                     const double* __restrict__ Ge,
@@ -449,14 +453,8 @@ __global__ void __launch_bounds__(TX * TY * TZ) k_apply_periodic_h8(int n, int n
     for (int q = 0; q < NJ; ++q) {
         const int t = min(static_cast<int>(threadIdx.x) + q * NT, NH - 1);
         const int lz = t / (HX * HY), r = t - lz * HX * HY, ly = r / HX, lx = r - (r / HX) * HX;
-        int gi = x0 - 1 + lx, gj = y0 - 1 + ly, gk = z0 - 1 + lz;
-        gi += gi < 0 ? n : 0;
-        gi -= gi >= n ? n : 0;
-        gj += gj < 0 ? n : 0;
-        gj -= gj >= n ? n : 0;
-        gk += gk < 0 ? n : 0;
-        gk -= gk >= n ? n : 0;
-        const int64_t k = ((static_cast<int64_t>(gk) * n + gj) * n + gi) * 3;
+        const int gi = wrap_line(x0 - 1 + lx, nx), gj = wrap_line(y0 - 1 + ly, ny), gk = wrap_line(z0 - 1 + lz, nz);
+        const int64_t k = ((static_cast<int64_t>(gk) * ny + gj) * nx + gi) * 3;
 #pragma unroll
         for (int c = 0; c < 3; ++c) dd[q][c] = sidx[k + c];
     }
@@ -485,11 +483,9 @@ __global__ void __launch_bounds__(TX * TY * TZ) k_apply_periodic_h8(int n, int n
         const int ex = ((el + 1) >> 1) & 1, ey = (el >> 1) & 1, ez = el >> 2;
         const int ax = 1 - ex, ay = 1 - ey, az = 1 - ez;
         const int la = az * 4 + (ay ? (ax ? 2 : 3) : (ax ? 1 : 0));
-        int ei = x0 + olx - 1 + ex, ej = y0 + oly - 1 + ey, ek = z0 + olz - 1 + ez;
-        ei += ei < 0 ? n : 0;
-        ej += ej < 0 ? n : 0;
-        ek += ek < 0 ? n : 0;
-        const int64_t e = (static_cast<int64_t>(ek) * n + ej) * n + ei;
+        const int ei = wrap_line(x0 + olx - 1 + ex, nx), ej = wrap_line(y0 + oly - 1 + ey, ny),
+                  ek = wrap_line(z0 + olz - 1 + ez, nz);
+        const int64_t e = (static_cast<int64_t>(ek) * ny + ej) * nx + ei;
         // element nodes in the halo tile: lower corner (olx + ex, oly + ey, olz + ez)
         const int c0 = ((olz + ez) * HY + (oly + ey)) * HX + (olx + ex);
         double ue[24];
@@ -514,12 +510,13 @@ __global__ void __launch_bounds__(TX * TY * TZ) k_apply_periodic_h8(int n, int n
             acc[j] = fma(k, sk, fma(gm, sg, acc[j]));
         }
     }
-    const int64_t kn = ((static_cast<int64_t>(z0 + olz) * n + y0 + oly) * n + x0 + olx) * 3;
+    const bool own = x0 + olx < nx && y0 + oly < ny && z0 + olz < nz;
+    const int64_t kn = own ? ((static_cast<int64_t>(z0 + olz) * ny + y0 + oly) * nx + x0 + olx) * 3 : 0;
     const int ho = ((olz + 1) * HY + oly + 1) * HX + olx + 1; // the owned node in the halo tile
     double dot = 0.0;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        const int32_t d = sidx[kn + c];
+        const int32_t d = own ? sidx[kn + c] : -1;
         if (d >= 0) {
             y[d] = acc[c];
             dot += s_x[c][ho] * acc[c];
@@ -906,8 +903,9 @@ void apply(gf_pcg_s* P, const double* xu, const double* xp, double* yu, bool xu_
     if (P->structured && !xp) {
         const double* xs = xu_in_full ? P->xfull.p : xu;
         if ((!w || w == xs) && P->et == GF_HEX8) {
-            k_apply_periodic_h8<8, 8, 4><<<P->ntiles, 256, 0, s>>>(P->sn, P->ntx, P->nty, P->ke8.p, P->sidx.p, P->Ke.p,
-                                                                   P->Ge.p, xs, yu, w ? partial : nullptr, state);
+            k_apply_periodic_h8<8, 8, 4><<<P->ntiles, 256, 0, s>>>(P->snx, P->sny, P->snz, P->ntx, P->nty, P->ke8.p,
+                                                                   P->sidx.p, P->Ke.p, P->Ge.p, xs, yu,
+                                                                   w ? partial : nullptr, state);
             check_launch();
             return;
         }
@@ -917,8 +915,9 @@ void apply(gf_pcg_s* P, const double* xu, const double* xp, double* yu, bool xu_
                 for (int k = 0; k < 8; ++k) sh.g[q][k] = P->sh_g[q * 8 + k];
                 sh.v[q] = P->sh_v[q];
             }
-            k_apply_periodic_q4<32, 8><<<P->ntiles, 256, 0, s>>>(P->sn, P->ntx, P->per_xcd, sh, P->sidx.p, P->Ke.p,
-                                                                 P->Ge.p, xs, yu, w ? partial : nullptr, state);
+            k_apply_periodic_q4<32, 8><<<P->ntiles, 256, 0, s>>>(P->snx, P->sny, P->ntx, P->per_xcd, sh, P->sidx.p,
+                                                                 P->Ke.p, P->Ge.p, xs, yu, w ? partial : nullptr,
+                                                                 state);
             check_launch();
             return;
         }
@@ -1001,37 +1000,38 @@ bool uniform_per_element(const double* data, int64_t nelem, int n, double* first
     return true;
 }
 
-// Regular n x n Quad4 cell whose dependent DOFs are periodic copies (C_du rows = one unit entry of
-// the partner's u-DOF, or empty when the partner is prescribed) and whose elements share one
-// geometry: then K' x_u is applied by k_apply_periodic_q4.
+// Regular nx x ny Quad4 cell (at least 8 elements each way: a halo row wraps onto a line of its own)
+// whose dependent DOFs are periodic copies (C_du rows = one unit entry of the partner's u-DOF, or empty
+// when the partner is prescribed) and whose elements share one geometry: then K' x_u is applied by
+// k_apply_periodic_q4.
 void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_col_h, const double* cdu_val_h)
 {
     constexpr int TX = 32, TY = 8;
     auto v = P->v;
-    if (P->et != GF_QUAD4_PLANAR) return;
-    const int64_t n = static_cast<int64_t>(std::llround(std::sqrt(static_cast<double>(P->nelem))));
-    if (n * n != P->nelem || n % TX != 0 || n % TY != 0 || n >= (1 << 15)) return;
-    const int64_t N1 = n + 1;
-    if (v->nnode < N1 * N1 || v->ndim != 2) return;
-    for (int64_t j = 0; j < n; ++j)
-        for (int64_t i = 0; i < n; ++i) {
-            const int64_t e = j * n + i, a = j * N1 + i;
+    if (P->et != GF_QUAD4_PLANAR || v->ndim != 2 || P->nelem < 1) return;
+    const int64_t N1 = v->conn_h[3], nx = N1 - 1;
+    if (nx < 8 || P->nelem % nx != 0) return;
+    const int64_t ny = P->nelem / nx;
+    if (ny < 8 || nx >= (1 << 15) || ny >= (1 << 15) || v->nnode < N1 * (ny + 1)) return;
+    for (int64_t j = 0; j < ny; ++j)
+        for (int64_t i = 0; i < nx; ++i) {
+            const int64_t e = j * nx + i, a = j * N1 + i;
             const int64_t want[4] = {a, a + 1, a + N1 + 1, a + N1};
             for (int m = 0; m < 4; ++m)
                 if (v->conn_h[e * 4 + m] != want[m]) return;
         }
     auto dof = [&](int64_t node, int c) { return v->dofs_h[node * 2 + c]; };
     // independent grid nodes: u or p; dependent edge nodes: periodic copies of their partner
-    for (int64_t j = 0; j <= n; ++j)
-        for (int64_t i = 0; i <= n; ++i)
+    for (int64_t j = 0; j <= ny; ++j)
+        for (int64_t i = 0; i <= nx; ++i)
             for (int c = 0; c < 2; ++c) {
                 const int64_t d = dof(j * N1 + i, c);
-                if (i < n && j < n) {
+                if (i < nx && j < ny) {
                     if (d < 0 || d >= P->nni) return;
                     continue;
                 }
                 if (d < P->nni || d >= P->ndof) return;
-                const int64_t pd = dof((j % n) * N1 + (i % n), c), r = d - P->nni;
+                const int64_t pd = dof((j % ny) * N1 + (i % nx), c), r = d - P->nni;
                 const int64_t cnt = cdu_ptr_h[r + 1] - cdu_ptr_h[r];
                 if (pd < P->nnu) {
                     if (cnt != 1 || cdu_col_h[cdu_ptr_h[r]] != pd || cdu_val_h[cdu_ptr_h[r]] != 1.0) return;
@@ -1044,57 +1044,61 @@ void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_co
     std::vector<double> g(32), vol(4);
     if (!uniform_per_element(quad_dNx(P->q), P->nelem, 32, g.data())) return;
     if (!uniform_per_element(quad_vol(P->q), P->nelem, 4, vol.data())) return;
-    std::vector<int32_t> sidx(static_cast<size_t>(n * n * 2));
-    for (int64_t j = 0; j < n; ++j)
-        for (int64_t i = 0; i < n; ++i)
+    std::vector<int32_t> sidx(static_cast<size_t>(nx * ny * 2));
+    for (int64_t j = 0; j < ny; ++j)
+        for (int64_t i = 0; i < nx; ++i)
             for (int c = 0; c < 2; ++c) {
                 const int64_t d = dof(j * N1 + i, c);
-                sidx[(j * n + i) * 2 + c] = d < P->nnu ? static_cast<int32_t>(d) : -1;
+                sidx[(j * nx + i) * 2 + c] = d < P->nnu ? static_cast<int32_t>(d) : -1;
             }
     P->sidx.alloc(sidx.size());
     GF_HIP(hipMemcpy(P->sidx.p, sidx.data(), sidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     for (int k = 0; k < 32; ++k) P->sh_g[k] = g[k];
     for (int k = 0; k < 4; ++k) P->sh_v[k] = vol[k];
-    P->sn = static_cast<int>(n);
-    P->ntx = static_cast<int>(n / TX);
-    P->ntiles = static_cast<int>((n / TX) * (n / TY));
+    P->snx = static_cast<int>(nx);
+    P->sny = static_cast<int>(ny);
+    P->ntx = static_cast<int>((nx + TX - 1) / TX);
+    P->ntiles = P->ntx * static_cast<int>((ny + TY - 1) / TY);
     P->per_xcd = P->ntiles % 8 == 0 ? P->ntiles / 8 : 0;
     alloc_single_reduction(P);
     P->structured = true;
 }
 
-// Hex8 Regular n x n x n cell with periodic copies as dependent DOFs and identical element
-// geometry (to 1e-12): K' x_u is applied by k_apply_periodic_h8 with K_e = K KK + G KG.
+// Hex8 Regular nx x ny x nz cell (at least 4 elements each way) with periodic copies as dependent DOFs
+// and identical element geometry (to 1e-12): K' x_u is applied by k_apply_periodic_h8 with
+// K_e = K KK + G KG.
 void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_col_h, const double* cdu_val_h)
 {
     constexpr int TX = 8, TY = 8, TZ = 4;
     auto v = P->v;
-    if (P->et != GF_HEX8 || v->ndim != 3) return;
-    const int64_t n = static_cast<int64_t>(std::llround(std::cbrt(static_cast<double>(P->nelem))));
-    if (n * n * n != P->nelem || n % TX != 0 || n % TY != 0 || n % TZ != 0 || n >= 1024) return;
-    const int64_t N1 = n + 1;
-    if (v->nnode < N1 * N1 * N1) return;
-    auto node = [&](int64_t i, int64_t j, int64_t k) { return (k * N1 + j) * N1 + i; };
+    if (P->et != GF_HEX8 || v->ndim != 3 || P->nelem < 1) return;
+    const int64_t N1 = v->conn_h[3], nx = N1 - 1; // node 3 of the first element: one row up
+    if (nx < 4 || v->conn_h[4] % N1 != 0) return;
+    const int64_t M1 = v->conn_h[4] / N1, ny = M1 - 1; // node 4: one layer up
+    if (ny < 4 || P->nelem % (nx * ny) != 0) return;
+    const int64_t nz = P->nelem / (nx * ny);
+    if (nz < 4 || nx >= 1024 || ny >= 1024 || nz >= 1024 || v->nnode < N1 * M1 * (nz + 1)) return;
+    auto node = [&](int64_t i, int64_t j, int64_t k) { return (k * M1 + j) * N1 + i; };
     static const int OX[8] = {0, 1, 1, 0, 0, 1, 1, 0}, OY[8] = {0, 0, 1, 1, 0, 0, 1, 1}, OZ[8] = {0, 0, 0, 0, 1, 1, 1, 1};
-    for (int64_t k = 0; k < n; ++k)
-        for (int64_t j = 0; j < n; ++j)
-            for (int64_t i = 0; i < n; ++i) {
-                const int64_t e = (k * n + j) * n + i;
+    for (int64_t k = 0; k < nz; ++k)
+        for (int64_t j = 0; j < ny; ++j)
+            for (int64_t i = 0; i < nx; ++i) {
+                const int64_t e = (k * ny + j) * nx + i;
                 for (int m = 0; m < 8; ++m)
                     if (v->conn_h[e * 8 + m] != node(i + OX[m], j + OY[m], k + OZ[m])) return;
             }
     auto dof = [&](int64_t nd, int c) { return v->dofs_h[nd * 3 + c]; };
-    for (int64_t k = 0; k <= n; ++k)
-        for (int64_t j = 0; j <= n; ++j)
-            for (int64_t i = 0; i <= n; ++i)
+    for (int64_t k = 0; k <= nz; ++k)
+        for (int64_t j = 0; j <= ny; ++j)
+            for (int64_t i = 0; i <= nx; ++i)
                 for (int c = 0; c < 3; ++c) {
                     const int64_t d = dof(node(i, j, k), c);
-                    if (i < n && j < n && k < n) {
+                    if (i < nx && j < ny && k < nz) {
                         if (d < 0 || d >= P->nni) return;
                         continue;
                     }
                     if (d < P->nni || d >= P->ndof) return;
-                    const int64_t pd = dof(node(i % n, j % n, k % n), c), r = d - P->nni;
+                    const int64_t pd = dof(node(i % nx, j % ny, k % nz), c), r = d - P->nni;
                     const int64_t cnt = cdu_ptr_h[r + 1] - cdu_ptr_h[r];
                     if (pd < P->nnu) {
                         if (cnt != 1 || cdu_col_h[cdu_ptr_h[r]] != pd || cdu_val_h[cdu_ptr_h[r]] != 1.0) return;
@@ -1124,22 +1128,24 @@ void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* c
                     }
             }
     }
-    std::vector<int32_t> sidx(static_cast<size_t>(n * n * n * 3));
-    for (int64_t k = 0; k < n; ++k)
-        for (int64_t j = 0; j < n; ++j)
-            for (int64_t i = 0; i < n; ++i)
+    std::vector<int32_t> sidx(static_cast<size_t>(nx * ny * nz * 3));
+    for (int64_t k = 0; k < nz; ++k)
+        for (int64_t j = 0; j < ny; ++j)
+            for (int64_t i = 0; i < nx; ++i)
                 for (int c = 0; c < 3; ++c) {
                     const int64_t d = dof(node(i, j, k), c);
-                    sidx[((k * n + j) * n + i) * 3 + c] = d < P->nnu ? static_cast<int32_t>(d) : -1;
+                    sidx[((k * ny + j) * nx + i) * 3 + c] = d < P->nnu ? static_cast<int32_t>(d) : -1;
                 }
     P->sidx.alloc(sidx.size());
     GF_HIP(hipMemcpy(P->sidx.p, sidx.data(), sidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     P->ke8.alloc(kkg.size());
     GF_HIP(hipMemcpy(P->ke8.p, kkg.data(), kkg.size() * sizeof(double), hipMemcpyHostToDevice));
-    P->sn = static_cast<int>(n);
-    P->ntx = static_cast<int>(n / TX);
-    P->nty = static_cast<int>(n / TY);
-    P->ntiles = static_cast<int>((n / TX) * (n / TY) * (n / TZ));
+    P->snx = static_cast<int>(nx);
+    P->sny = static_cast<int>(ny);
+    P->snz = static_cast<int>(nz);
+    P->ntx = static_cast<int>((nx + TX - 1) / TX);
+    P->nty = static_cast<int>((ny + TY - 1) / TY);
+    P->ntiles = P->ntx * P->nty * static_cast<int>((nz + TZ - 1) / TZ);
     P->per_xcd = 0;
     P->structured = true;
 }
@@ -1354,7 +1360,7 @@ int gf_pcg_solve(gf_pcg P, const double* b_u, double* x_u, double tol, int64_t m
             for (int64_t k = 0; single && k < check_every && it < maxiter; ++k, ++it) {
                 const int i0 = static_cast<int>(it & 1), i1 = 1 - i0;
                 k_cgsr_periodic_q4<32, 8><<<P->ntiles, 256, 0, s>>>(
-                    P->sn, P->ntx, P->ntiles, P->per_xcd, sh, P->sidx.p, P->Ke.p, P->Ge.p, P->invdiag.p, P->sr[i0].p,
+                    P->snx, P->sny, P->ntx, P->ntiles, P->per_xcd, sh, P->sidx.p, P->Ke.p, P->Ge.p, P->invdiag.p, P->sr[i0].p,
                     P->sw[i0].p, P->ss[i0].p, P->sr[i1].p, P->sw[i1].p, P->ss[i1].p, P->z.p, P->x.p, P->partial.p,
                     P->spart.p + 3 * i0 * P->ntiles, P->spart.p + 3 * i1 * P->ntiles, P->scal.p, P->state.p, it);
             }

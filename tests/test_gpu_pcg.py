@@ -213,3 +213,48 @@ def test_bad_start_falls_back(gf, et, n, square):
     with pytest.raises(gf.GooseFEMError) as e:
         P.solve(bad, tol=1e-10)
     assert e.value.code == gf.GF_EINVAL
+
+
+@pytest.mark.parametrize("size", [(8, 8), (9, 33), (33, 9), (31, 8), (32, 15), (65, 17), (4, 4, 4), (5, 9, 6), (9, 8, 5),
+                                  (17, 4, 7), (8, 16, 4)])
+def test_structured_operator_of_any_size(gf, size):
+    """The structured operators on cells that are no multiple of their tiles (32 x 8 and 8 x 8 x 4 nodes):
+    the product against the sum of the oracle's element matrices over the wrapped grid (1e-13: FP64 sums
+    of some ten terms), and the solve's residual with that matrix."""
+    import scipy.sparse as sp
+
+    nd = len(size)
+    et = QUAD4_PLANAR if nd == 2 else HEX8
+    mesh = gf.Mesh.Quad4.Regular(*size) if nd == 2 else gf.Mesh.Hex8.Regular(*size)
+    coor, conn = mesh.coor, mesh.conn
+    ctrl = gf.Tyings.Control(coor, mesh.dofs)
+    iip = np.concatenate((ctrl.controlDofs.ravel(), ctrl.dofs[mesh.nodesOrigin]))
+    ty = gf.Tyings.Periodic(ctrl.coor, ctrl.dofs, ctrl.controlDofs, mesh.nodesPeriodic, iip)
+    x = oracle.Vector(conn, oracle.dofs(coor.shape[0], nd)).AsElement(coor)
+    oq = oracle.Quadrature(et, x)
+    quad = gf.Element.Hex8.Quadrature(x) if nd == 3 else gf.Element.Quad4.QuadraturePlanar(x)
+    rng = np.random.default_rng(sum(size))
+    G, K = np.exp(0.4 * rng.standard_normal(oq.nelem)), rng.uniform(5.0, 15.0, oq.nelem)
+    P = gf.TyingsPCG(gf.Vector(conn, ty.dofs), quad, K, G, ty)
+    assert P.structured
+    C = oracle.elastic_tangent(np.repeat(K[:, None], oq.nip, 1), np.repeat(G[:, None], oq.nip, 1))
+    Ke = oq.Int_gradN_dot_tensor4_dot_gradNT_dV(C)
+    # u-DOF of every node's periodic image; prescribed ones (the origin) get the spare number nnu
+    i = np.rint(coor).astype(int) % np.array(size)
+    image = np.zeros(coor.shape[0], dtype=int)
+    grid = {tuple(r): n for n, r in reversed(list(enumerate(np.rint(coor).astype(int))))}
+    for n, r in enumerate(i):
+        image[n] = grid[tuple(r)]
+    u = np.minimum(ty.dofs[image], ty.nnu)
+    d = u[conn].reshape(mesh.nelem, -1)
+    k = d.shape[1]
+    A = sp.csr_matrix((Ke.ravel(), (np.repeat(d, k, axis=1).ravel(), np.tile(d, (1, k)).ravel())),
+                      shape=(ty.nnu + 1,) * 2)[: ty.nnu, : ty.nnu]
+    xu = rng.standard_normal(ty.nnu)
+    y = host(P.apply(xu))
+    assert np.linalg.norm(y - A @ xu) <= 1e-13 * np.linalg.norm(A @ xu)
+    b = A @ xu
+    sol, it, res = P.solve(b, tol=1e-10)
+    assert res <= 1e-9 and np.linalg.norm(b - A @ host(sol)) <= 1e-9 * np.linalg.norm(b)
+    again, it2, _ = P.solve(b, tol=1e-10)
+    assert it2 == it and np.array_equal(host(again), host(sol))
