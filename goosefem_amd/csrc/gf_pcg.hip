@@ -43,6 +43,11 @@ struct Csr {
     DBuf<double> val;
 };
 
+// The element matrix of the structured Quad4 cell is k EK + g EG (isotropic law, one geometry)
+struct ElemQ4 {
+    double k[8][8], g[8][8];
+};
+
 } // namespace
 
 struct gf_pcg_s {
@@ -63,7 +68,10 @@ struct gf_pcg_s {
     DBuf<int32_t> sidx; // [nodes of the cell * nd] u-DOF of grid node component c, or -1
     int nty = 0;
     DBuf<double> ke8;   // Hex8: [2][24][24] element matrices per unit K and per unit G
-    DBuf<double> sr[2], sw[2], ss[2]; // Quad4 single-reduction iteration: r, w, s by iteration parity
+    ElemQ4 eq4 = {};  // Quad4: element matrices per unit K and per unit G
+    // Quad4 single-reduction iteration on the grid: r, w, s by iteration parity, p, x, 1 / diag
+    DBuf<double2> sgrid;
+    double2 *sr[2] = {}, *sw[2] = {}, *ss[2] = {}, *sp = nullptr, *sx = nullptr, *si = nullptr;
     DBuf<double> gp[2];               // general operator: the search direction by iteration parity
     DBuf<double> spart;               // its block partials [2][3][ntiles]
     DBuf<double> xprev; // the last converged solution (the previous-step start of the fallback)
@@ -122,8 +130,8 @@ __device__ inline void quad4_planar_qp_force(const double* g, double v, const do
 // sidx maps grid node (i, j), component c to its u-DOF, or -1 for a prescribed DOF (the origin), whose
 // value is 0.  The last tile of a row or column owns what is left of it: the indices of the nodes and
 // elements past the cell's end that no owned node needs are clamped into range.
-// Any size takes these kernels (a 250 x 250 cell: 66 -> 22 ms per solve against the general operator's
-// four launches per iteration, each of 5 to 9 us).
+// Any size takes these kernels (a 250 x 250 cell: 69 -> 28 ms per solve against the general operator's four
+// launches per iteration of 5 to 9 us each, 20 ms with the iteration below).
 
 // line or element i of a direction of n, one period out of range at most where it is used
 __device__ inline int wrap_line(int i, int n)
@@ -224,77 +232,62 @@ __global__ void __launch_bounds__(TX * TY) k_apply_periodic_q4(int nx, int ny, i
 // iteration instead of two, so one launch: the tile forms the new u on its halo ring from the
 // neighbours' r, w, s (double-buffered by iteration parity, since the launch writes the tile's own)
 // and the owned nodes' p and x are read and written by their tile only.  u is never stored.
+// The vectors are kept on the grid, both components of a node together (prescribed ones are zero, with
+// a zero in invd), so no load waits for an index; each node sums its rows of the four elements around
+// it from the u in LDS, in fused multiply-adds.
+// Bound: the latency of one launch (loads, reduction, halo, product, sums) on up to 1,024 tiles.
+// Measured per iteration: 7.0 us at 250 x 250 (9.7 us with the vectors in u-DOF order behind an index, element
+// forces point by point in LDS and the flag tested before any load), 11.7 us at 512 x 512 (19.1 us),
+// 6.8 to 7.0 us at 31 to 128 squared (9.2 to 9.4 us at 64 and 128).
 // Every block takes the same decisions from the same ordered partials; block 0 records gam and
 // alpha (slots by parity), the iteration count and the done flag.
 template <int TX, int TY>
 __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
-    int nx, int ny, int ntx, int ntiles, int per_xcd, ShapeQ4 sh, const int32_t* __restrict__ sidx,
-    const double* __restrict__ Ke, const double* __restrict__ Ge, const double* __restrict__ invd,
-    const double* __restrict__ rc, const double* __restrict__ wc, const double* __restrict__ sc,
-    double* __restrict__ rn, double* __restrict__ wn, double* __restrict__ sn_, double* __restrict__ p,
-    double* __restrict__ x, const double* __restrict__ init_partial, const double* __restrict__ pin,
-    double* __restrict__ pout, double* __restrict__ scal, int32_t* __restrict__ state, int64_t it)
+    int nx, int ny, int ntx, int ntiles, int per_xcd, ElemQ4 E, const double* __restrict__ Ke,
+    const double* __restrict__ Ge, const double2* __restrict__ invd, const double2* __restrict__ rc,
+    const double2* __restrict__ wc, const double2* __restrict__ sc, double2* __restrict__ rn,
+    double2* __restrict__ wn, double2* __restrict__ sn_, double2* __restrict__ p, double2* __restrict__ x,
+    const double* __restrict__ init_partial, const double* __restrict__ pin, double* __restrict__ pout,
+    double* __restrict__ scal, int32_t* __restrict__ state, int64_t it)
 {
-    if (state[0]) return; // uniform for the grid
-    constexpr int HX = TX + 2, HY = TY + 2, EX = TX + 1, EY = TY + 1, NT = TX * TY;
-    constexpr int NH = (HX * HY + NT - 1) / NT, NE = (EX * EY + NT - 1) / NT; // halo nodes, elements per thread
+    constexpr int HX = TX + 2, HY = TY + 2, NT = TX * TY;
+    constexpr int NH = (HX * HY + NT - 1) / NT; // halo nodes per thread
     static_assert(NT == BS, "the partial sums stride by BS");
-    __shared__ double2 s_x[HY * HX];                              // the new u on the halo tile
-    __shared__ double s_f[EY * EX][8];                            // element forces
-    __shared__ double2 s_u0[NT], s_sv[NT], s_rv[NT];              // owned nodes: old u, new s, new r
+    __shared__ double2 s_x[HY * HX];       // the new u on the halo tile
+    __shared__ double2 s_u0[NT], s_sv[NT], s_rv[NT]; // owned nodes: old u, new s, new r
     const int b = blockIdx.x;
     const int tile = per_xcd > 0 ? (b & 7) * per_xcd + (b >> 3) : b;
-    const int tx = tile % ntx, ty = tile / ntx;
+    const int ty = tile / ntx, tx = tile - ty * ntx;
     const int x0 = tx * TX, y0 = ty * TY;
     const int oly = threadIdx.x / TX, olx = threadIdx.x - (threadIdx.x / TX) * TX;
 
-    // every load that does not depend on this iteration's scalars is issued first, so that its
-    // latency overlaps the reduction of the previous launch's partials
-    int32_t hd[NH][2];
-    double hr[NH][2], hw[NH][2], hs[NH][2], hi[NH][2];
+    // every load is issued first, so that its latency overlaps the reduction of the previous launch's
+    // partials
+    const int done = state[0];
+    const double tol2 = scal[4], gam_prev = scal[5 + ((it + 1) & 1)], alpha_prev = scal[7 + ((it + 1) & 1)];
+    double2 hr[NH], hw[NH], hs[NH], hi[NH];
 #pragma unroll
     for (int j = 0; j < NH; ++j) {
-        const int t = threadIdx.x + j * NT;
-        hd[j][0] = hd[j][1] = -1;
-        if (t < HX * HY) {
-            const int ly = t / HX, lx = t - (t / HX) * HX;
-            const int gi = wrap_line(x0 - 1 + lx, nx), gj = wrap_line(y0 - 1 + ly, ny);
-            const int64_t k = (static_cast<int64_t>(gj) * nx + gi) * 2;
-            hd[j][0] = sidx[k];
-            hd[j][1] = sidx[k + 1];
-        }
+        const int t = min(static_cast<int>(threadIdx.x) + j * NT, HX * HY - 1);
+        const int ly = t / HX, lx = t - (t / HX) * HX;
+        const int k = wrap_line(y0 - 1 + ly, ny) * nx + wrap_line(x0 - 1 + lx, nx);
+        hr[j] = rc[k];
+        hw[j] = wc[k];
+        hs[j] = it == 0 ? make_double2(0.0, 0.0) : sc[k];
+        hi[j] = invd[k];
     }
-#pragma unroll
-    for (int j = 0; j < NH; ++j)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int32_t d = hd[j][c] >= 0 ? hd[j][c] : 0; // clamped: the values of d < 0 are unused
-            hr[j][c] = rc[d];
-            hw[j][c] = wc[d];
-            hs[j][c] = it == 0 ? 0.0 : sc[d];
-            hi[j][c] = invd[d];
-        }
     const bool own = x0 + olx < nx && y0 + oly < ny;
-    const int64_t ko = own ? (static_cast<int64_t>(y0 + oly) * nx + x0 + olx) * 2 : 0;
-    const int32_t od[2] = {own ? sidx[ko] : -1, own ? sidx[ko + 1] : -1};
-    double op[2], ox[2];
+    const int ko = own ? (y0 + oly) * nx + x0 + olx : 0;
+    const double2 op = it == 0 ? make_double2(0.0, 0.0) : p[ko], ox = x[ko];
+    double ek[4], eg[4]; // the elements (i-1, j-1), (i, j-1), (i-1, j), (i, j)
+    {
+        const int e0 = wrap_line(x0 + olx - 1, nx), e1 = wrap_line(x0 + olx, nx);
+        const int r0 = wrap_line(y0 + oly - 1, ny) * nx, r1 = wrap_line(y0 + oly, ny) * nx;
+        const int e[4] = {r0 + e0, r0 + e1, r1 + e0, r1 + e1};
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int32_t d = od[c] >= 0 ? od[c] : 0;
-        op[c] = it == 0 ? 0.0 : p[d];
-        ox[c] = x[d];
-    }
-    double ek[NE], eg[NE];
-#pragma unroll
-    for (int j = 0; j < NE; ++j) {
-        const int t = threadIdx.x + j * NT;
-        ek[j] = eg[j] = 0.0;
-        if (t < EX * EY) {
-            const int ly = t / EX, lx = t - (t / EX) * EX;
-            const int ei = wrap_line(x0 - 1 + lx, nx), ej = wrap_line(y0 - 1 + ly, ny);
-            const int64_t e = static_cast<int64_t>(ej) * nx + ei;
-            ek[j] = Ke[e];
-            eg[j] = Ge[e];
+        for (int j = 0; j < 4; ++j) {
+            ek[j] = Ke[e[j]];
+            eg[j] = Ge[e[j]];
         }
     }
 
@@ -315,7 +308,8 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
         }
     }
     block_sum3<BS>(gam, del, rr);
-    if (rr <= scal[4]) { // converged after `it` iterations
+    if (done) return; // uniform for the grid
+    if (rr <= tol2) { // converged after `it` iterations
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             scal[3] = rr;
             state[0] = 1;
@@ -325,8 +319,8 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
     double beta = 0.0, alpha = 0.0;
     if (it == 0) alpha = gam / del;
     else {
-        beta = gam / scal[5 + ((it + 1) & 1)];
-        alpha = gam / (del - beta * gam / scal[7 + ((it + 1) & 1)]);
+        beta = gam / gam_prev;
+        alpha = gam / (del - beta * gam / alpha_prev);
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal[5 + (it & 1)] = gam;
@@ -335,86 +329,58 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
         state[1] = static_cast<int32_t>(it + 1);
     }
 
-    // s = w + beta s, r = r - alpha s, u = r ./ diag on the halo tile (periodic wrap, prescribed
-    // DOFs read as 0); the owned nodes also keep the old u, the new s and the new r in LDS
+    // s = w + beta s, r = r - alpha s, u = r ./ diag on the halo tile (periodic wrap); the owned nodes
+    // also keep the old u, the new s and the new r in LDS
 #pragma unroll
     for (int j = 0; j < NH; ++j) {
         const int t = threadIdx.x + j * NT;
         if (t >= HX * HY) continue;
         const int ly = t / HX, lx = t - (t / HX) * HX;
-        double uv[2], u0[2], sv[2], rv[2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            uv[c] = u0[c] = sv[c] = rv[c] = 0.0;
-            if (hd[j][c] >= 0) {
-                sv[c] = it == 0 ? hw[j][c] : hw[j][c] + beta * hs[j][c];
-                rv[c] = hr[j][c] - alpha * sv[c];
-                uv[c] = rv[c] * hi[j][c];
-                u0[c] = hr[j][c] * hi[j][c];
-            }
-        }
-        s_x[t] = make_double2(uv[0], uv[1]);
+        const double2 sv = make_double2(hw[j].x + beta * hs[j].x, hw[j].y + beta * hs[j].y);
+        const double2 rv = make_double2(hr[j].x - alpha * sv.x, hr[j].y - alpha * sv.y);
+        s_x[t] = make_double2(rv.x * hi[j].x, rv.y * hi[j].y);
         if (lx >= 1 && lx <= TX && ly >= 1 && ly <= TY) {
             const int o = (ly - 1) * TX + lx - 1;
-            s_u0[o] = make_double2(u0[0], u0[1]);
-            s_sv[o] = make_double2(sv[0], sv[1]);
-            s_rv[o] = make_double2(rv[0], rv[1]);
+            s_u0[o] = make_double2(hr[j].x * hi[j].x, hr[j].y * hi[j].y);
+            s_sv[o] = sv;
+            s_rv[o] = rv;
         }
     }
     __syncthreads();
-    // w = K' u: element forces of the (TX+1) x (TY+1) elements touching the tile
+    // w = K' u at the owned node: its rows of the elements (i-1, j-1), where it is local node 2,
+    // (i, j-1) node 3, (i-1, j) node 1, (i, j) node 0
+    double2 u[9];
 #pragma unroll
-    for (int j = 0; j < NE; ++j) {
-        const int t = threadIdx.x + j * NT;
-        if (t >= EX * EY) continue;
-        const int ly = t / EX, lx = t - (t / EX) * EX;
-        const int n0 = ly * HX + lx;
-        const int nid[4] = {n0, n0 + 1, n0 + HX + 1, n0 + HX};
-        double u[4][2], f[4][2];
+    for (int q = 0; q < 9; ++q) u[q] = s_x[(oly + q / 3) * HX + olx + q % 3];
+    constexpr int LA[4] = {2, 3, 1, 0}, OX[4] = {0, 1, 1, 0}, OY[4] = {0, 0, 1, 1};
+    double f[2] = {0.0, 0.0};
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const double2 xx = s_x[nid[m]];
-            u[m][0] = xx.x;
-            u[m][1] = xx.y;
-            f[m][0] = f[m][1] = 0.0;
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            double fk = 0.0, fg = 0.0;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const double2 v = u[(j / 2 + OY[m]) * 3 + j % 2 + OX[m]];
+                fk = fma(E.k[2 * LA[j] + c][2 * m], v.x, fma(E.k[2 * LA[j] + c][2 * m + 1], v.y, fk));
+                fg = fma(E.g[2 * LA[j] + c][2 * m], v.x, fma(E.g[2 * LA[j] + c][2 * m + 1], v.y, fg));
+            }
+            f[c] = fma(ek[j], fk, fma(eg[j], fg, f[c]));
         }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) quad4_planar_qp_force(sh.g[q], sh.v[q], u, ek[j], eg[j], f);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            s_f[t][2 * m] = f[m][0];
-            s_f[t][2 * m + 1] = f[m][1];
-        }
-    }
-    __syncthreads();
-    // owned node: elements (i-1, j-1) as its node 2, (i, j-1) node 3, (i-1, j) node 1, (i, j) node 0
-    const int l0 = oly * EX + olx;
-    double f[2];
-    f[0] = s_f[l0][4];
-    f[1] = s_f[l0][5];
-    f[0] += s_f[l0 + 1][6];
-    f[1] += s_f[l0 + 1][7];
-    f[0] += s_f[l0 + EX][2];
-    f[1] += s_f[l0 + EX][3];
-    f[0] += s_f[l0 + EX + 1][0];
-    f[1] += s_f[l0 + EX + 1][1];
-    const double2 uo = s_x[(oly + 1) * HX + olx + 1], u0o = s_u0[threadIdx.x], svo = s_sv[threadIdx.x],
-                  rvo = s_rv[threadIdx.x];
-    const double un[2] = {uo.x, uo.y}, u0[2] = {u0o.x, u0o.y}, sv[2] = {svo.x, svo.y}, rv[2] = {rvo.x, rvo.y};
+    const double2 un = u[4], u0 = s_u0[threadIdx.x], sv = s_sv[threadIdx.x], rv = s_rv[threadIdx.x];
     double g = 0.0, dl = 0.0, r2 = 0.0;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int32_t d = od[c];
-        if (d < 0) continue;
-        const double pv = it == 0 ? u0[c] : u0[c] + beta * op[c];
-        x[d] = ox[c] + alpha * pv;
-        p[d] = pv;
-        sn_[d] = sv[c];
-        rn[d] = rv[c];
-        wn[d] = f[c];
-        g += rv[c] * un[c];
-        dl += f[c] * un[c];
-        r2 += rv[c] * rv[c];
+    if (own) {
+        const double2 iv = invd[ko];
+        const double2 w = make_double2(iv.x != 0.0 ? f[0] : 0.0, iv.y != 0.0 ? f[1] : 0.0);
+        const double2 pv = make_double2(u0.x + beta * op.x, u0.y + beta * op.y);
+        x[ko] = make_double2(ox.x + alpha * pv.x, ox.y + alpha * pv.y);
+        p[ko] = pv;
+        sn_[ko] = sv;
+        rn[ko] = rv;
+        wn[ko] = w;
+        g = rv.x * un.x + rv.y * un.y;
+        dl = w.x * un.x + w.y * un.y;
+        r2 = rv.x * rv.x + rv.y * rv.y;
     }
     block_sum3<NT>(g, dl, r2);
     if (threadIdx.x == 0) {
@@ -422,6 +388,33 @@ __global__ void __launch_bounds__(TX * TY) k_cgsr_periodic_q4(
         pout[ntiles + b] = dl;
         pout[2 * ntiles + b] = r2;
     }
+}
+
+// grid vectors of the iteration (two components per node, zero where prescribed) from the u-DOF ones
+__global__ void __launch_bounds__(BS) k_to_grid(int64_t n, const int32_t* __restrict__ sidx,
+                                                const double* __restrict__ r, const double* __restrict__ w,
+                                                const double* __restrict__ x, const double* __restrict__ invd,
+                                                double* __restrict__ rg, double* __restrict__ wg,
+                                                double* __restrict__ xg, double* __restrict__ ig)
+{
+    const int64_t t = blockIdx.x * static_cast<int64_t>(BS) + threadIdx.x;
+    if (t >= n) return;
+    const int32_t d = sidx[t];
+    const int32_t k = d >= 0 ? d : 0;
+    const double a = r[k], b = w[k], c = x[k], e = invd[k];
+    rg[t] = d >= 0 ? a : 0.0;
+    wg[t] = d >= 0 ? b : 0.0;
+    xg[t] = d >= 0 ? c : 0.0;
+    ig[t] = d >= 0 ? e : 0.0;
+}
+
+__global__ void __launch_bounds__(BS) k_from_grid(int64_t n, const int32_t* __restrict__ sidx,
+                                                  const double* __restrict__ xg, double* __restrict__ x)
+{
+    const int64_t t = blockIdx.x * static_cast<int64_t>(BS) + threadIdx.x;
+    if (t >= n) return;
+    const int32_t d = sidx[t];
+    if (d >= 0) x[d] = xg[t];
 }
 
 // Hex8 Regular nx x ny x nz cell with periodic tyings: identical element geometry makes the element
@@ -857,10 +850,12 @@ __global__ void k_residual_final(const double* __restrict__ partial, double* __r
 // the vectors and block partials of the single-reduction iteration (structured operators)
 void alloc_single_reduction(gf_pcg_s* P)
 {
-    for (int k = 0; k < 2; ++k) {
-        P->sr[k].alloc(P->nnu);
-        P->sw[k].alloc(P->nnu);
-        P->ss[k].alloc(P->nnu);
+    const size_t n = P->sidx.n / 2;
+    P->sgrid.alloc(9 * n);
+    double2* w = P->sgrid.p;
+    for (double2** b : {&P->sr[0], &P->sr[1], &P->sw[0], &P->sw[1], &P->ss[0], &P->ss[1], &P->sp, &P->sx, &P->si}) {
+        *b = w;
+        w += n;
     }
     P->spart.alloc(6 * static_cast<size_t>(P->ntiles));
 }
@@ -1060,6 +1055,20 @@ void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_co
     P->ntx = static_cast<int>((nx + TX - 1) / TX);
     P->ntiles = P->ntx * static_cast<int>((ny + TY - 1) / TY);
     P->per_xcd = P->ntiles % 8 == 0 ? P->ntiles / 8 : 0;
+    // K_e = k EK + g EG: EK(2m+j, 2n+l) = sum_q dV dNx(m,j) dNx(n,l), EG(2m+j, 2n+l) =
+    // sum_q dV [dNx(m,l) dNx(n,j) + delta_jl dNx(m).dNx(n) - 2/3 dNx(m,j) dNx(n,l)]
+    for (int q = 0; q < 4; ++q)
+        for (int m = 0; m < 4; ++m)
+            for (int o = 0; o < 4; ++o) {
+                const double *a = g.data() + q * 8 + 2 * m, *b = g.data() + q * 8 + 2 * o;
+                const double dot = a[0] * b[0] + a[1] * b[1];
+                for (int j = 0; j < 2; ++j)
+                    for (int l = 0; l < 2; ++l) {
+                        P->eq4.k[2 * m + j][2 * o + l] += vol[q] * a[j] * b[l];
+                        P->eq4.g[2 * m + j][2 * o + l] +=
+                            vol[q] * (a[l] * b[j] + (j == l ? dot : 0.0) - 2.0 / 3.0 * a[j] * b[l]);
+                    }
+            }
     alloc_single_reduction(P);
     P->structured = true;
 }
@@ -1328,11 +1337,7 @@ int gf_pcg_solve(gf_pcg P, const double* b_u, double* x_u, double tol, int64_t m
         int32_t cap = static_cast<int32_t>(maxiter);
         GF_HIP(hipMemcpyAsync(P->state.p + 2, &cap, sizeof(int32_t), hipMemcpyHostToDevice, s));
         int32_t st[2] = {0, 0};
-        ShapeQ4 sh;
-        for (int q = 0; q < 4; ++q) {
-            for (int k = 0; k < 8; ++k) sh.g[q][k] = P->sh_g[q * 8 + k];
-            sh.v[q] = P->sh_v[q];
-        }
+        auto d1 = [](double2* v) { return reinterpret_cast<double*>(v); };
         const bool done0 = rr <= tol * tol * (bb > 0.0 ? bb : 1.0);
         // Quad4: one launch per iteration (single-reduction CG).  Hex8 keeps three launches
         // (operator, update, direction): on its 3-D halo of 2.34 nodes per owned node, forming the
@@ -1351,8 +1356,11 @@ int gf_pcg_solve(gf_pcg P, const double* b_u, double* x_u, double tol, int64_t m
         if (single && !done0) {
             // r0 is in r, u0 = r0 ./ diag in the u-part of xfull: w0 = K' u0 with the partials of
             // (u0, w0) in the 'del' slot of the first launch's input
-            GF_HIP(hipMemcpyAsync(P->sr[0].p, P->r.p, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-            apply(P, nullptr, nullptr, P->sw[0].p, true, s, P->xfull.p, P->spart.p + P->ntiles, nullptr);
+            apply(P, nullptr, nullptr, P->qv.p, true, s, P->xfull.p, P->spart.p + P->ntiles, nullptr);
+            const int64_t ng = static_cast<int64_t>(P->sidx.n);
+            k_to_grid<<<nblocks(ng, BS), BS, 0, s>>>(ng, P->sidx.p, P->r.p, P->qv.p, P->x.p, P->invdiag.p, d1(P->sr[0]),
+                                                     d1(P->sw[0]), d1(P->sx), d1(P->si));
+            check_launch();
         }
         StatePipe pipe;
         int chunk = 0;
@@ -1360,8 +1368,8 @@ int gf_pcg_solve(gf_pcg P, const double* b_u, double* x_u, double tol, int64_t m
             for (int64_t k = 0; single && k < check_every && it < maxiter; ++k, ++it) {
                 const int i0 = static_cast<int>(it & 1), i1 = 1 - i0;
                 k_cgsr_periodic_q4<32, 8><<<P->ntiles, 256, 0, s>>>(
-                    P->snx, P->sny, P->ntx, P->ntiles, P->per_xcd, sh, P->sidx.p, P->Ke.p, P->Ge.p, P->invdiag.p, P->sr[i0].p,
-                    P->sw[i0].p, P->ss[i0].p, P->sr[i1].p, P->sw[i1].p, P->ss[i1].p, P->z.p, P->x.p, P->partial.p,
+                    P->snx, P->sny, P->ntx, P->ntiles, P->per_xcd, P->eq4, P->Ke.p, P->Ge.p, P->si, P->sr[i0], P->sw[i0],
+                    P->ss[i0], P->sr[i1], P->sw[i1], P->ss[i1], P->sp, P->sx, P->partial.p,
                     P->spart.p + 3 * i0 * P->ntiles, P->spart.p + 3 * i1 * P->ntiles, P->scal.p, P->state.p, it);
             }
             for (int64_t k = 0; hexs && k < check_every && it < maxiter; ++k, ++it) {
@@ -1390,6 +1398,8 @@ int gf_pcg_solve(gf_pcg P, const double* b_u, double* x_u, double tol, int64_t m
             if (chunk > 0 && pipe.wait(chunk - 1)[0]) break;
             ++chunk;
         }
+        if (single && !done0)
+            k_from_grid<<<nblocks(P->sidx.n, BS), BS, 0, s>>>(static_cast<int64_t>(P->sidx.n), P->sidx.p, d1(P->sx), P->x.p);
         // true residual ||b - K' x|| / ||b||
         GF_HIP(hipMemcpyAsync(x_u, P->x.p, n * sizeof(double), hipMemcpyDeviceToDevice, s));
         GF_HIP(hipMemcpyAsync(P->xfull.p, P->x.p, n * sizeof(double), hipMemcpyDeviceToDevice, s));
