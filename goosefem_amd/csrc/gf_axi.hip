@@ -3,13 +3,16 @@
 // B-matrix [nelem, nip, nne, 3, 3, 3] only five components per node are non-zero (:401-438):
 //   B(m,r,r,r) = B(m,r,z,z) = dN/dr,  B(m,t,t,r) = N / r_q,  B(m,z,r,r) = B(m,z,z,z) = dN/dz,
 // so the geometry is kept as G[e, q, m] = (dN/dr, N / r_q, dN/dz) (12 doubles per point instead of
-// 108) and dV = w J 2 pi r_q.  Every kernel keeps the reference's FP64 expression and summation
-// order (no contraction), so results equal the reference's bit for bit.  The stiffness runs the
+// 108) and dV = w J 2 pi r_q; the kernels that are bound by HBM form it again from the element's 64 bytes
+// of coordinates, with the function that made the stored one.  Every kernel keeps the reference's FP64
+// expression and summation order (no contraction), so results equal the reference's bit for bit.  The
+// stiffness runs the
 // 25 products of each node pair over the five non-zero slots a (outer) and b (inner), slot =
 // (i, j, value, nodal component): (r,r: dN/dr, u_r) (t,t: N/r, u_r) (z,z: dN/dz, u_z)
 // (r,z: dN/dr, u_z) (z,r: dN/dz, u_r), and K(m, c_a; n, c_b) += B_a(m) C(i_a, j_a, j_b, i_b) B_b(n) dV
 // (:298-398, in the listed order).
 #include "gf_internal.hpp"
+#include "gf_stage.hpp"
 
 using namespace gf;
 
@@ -27,23 +30,16 @@ struct AxiRule {
 struct gf_axi_s {
     int64_t nelem = 0;
     AxiRule rule;
-    DBuf<double> G, vol;
+    DBuf<double> x, G, vol;
 };
 
 namespace {
 
 constexpr int BS = 256;
 
-__global__ void k_axi_geometry(int64_t nelem, AxiRule R, const double* __restrict__ x, double* __restrict__ G,
-                               double* __restrict__ vol)
+// G (12) and dV of point q of the element with coordinates xv
+__device__ inline void axi_point_geometry(const AxiRule& R, int q, const double* __restrict__ xv, double* o, double& v)
 {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= nelem * R.nip) return;
-    const int64_t e = t / R.nip;
-    const int q = static_cast<int>(t - e * R.nip);
-    const double* xe = x + 8 * e;
-    double xv[8];
-    for (int k = 0; k < 8; ++k) xv[k] = xe[k];
     const double(*g)[2] = R.dNxi[q];
     const double* n = R.N[q];
     const double J00 = g[0][0] * xv[0] + g[1][0] * xv[2] + g[2][0] * xv[4] + g[3][0] * xv[6];
@@ -54,42 +50,72 @@ __global__ void k_axi_geometry(int64_t nelem, AxiRule R, const double* __restric
     const double det = J00 * J11 - J01 * J10;
     const double I00 = J11 / det, I01 = -1.0 * J01 / det, I10 = -1.0 * J10 / det, I11 = J00 / det;
     const double rq = n[0] * xv[1] + n[1] * xv[3] + n[2] * xv[5] + n[3] * xv[7];
-    double* o = G + 12 * t;
+#pragma unroll
     for (int m = 0; m < 4; ++m) {
         o[3 * m + 0] = I10 * g[m][0] + I11 * g[m][1];
         o[3 * m + 1] = 1.0 / rq * n[m];
         o[3 * m + 2] = I00 * g[m][0] + I01 * g[m][1];
     }
-    vol[t] = R.w[q] * det * 2.0 * M_PI * rq;
+    v = R.w[q] * det * 2.0 * M_PI * rq;
 }
 
-// gradN_vector (mode 0, :140-169), gradN_vector_T (1, :171-200), symGradN_vector (2, :202-233)
-__global__ void k_axi_grad(int64_t n, int nip, int mode, const double* __restrict__ G, const double* __restrict__ u_,
-                           double* __restrict__ out)
+__global__ void k_axi_geometry(int64_t nelem, AxiRule R, const double* __restrict__ x, double* __restrict__ G,
+                               double* __restrict__ vol)
 {
     const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= n) return;
-    const int64_t e = t / nip;
-    const double* b = G + 12 * t;
-    const double* u = u_ + 8 * e; // (u_z, u_r) per node
-    const double rr = b[0] * u[1] + b[3] * u[3] + b[6] * u[5] + b[9] * u[7];
-    const double tt = b[1] * u[1] + b[4] * u[3] + b[7] * u[5] + b[10] * u[7];
-    const double zz = b[2] * u[0] + b[5] * u[2] + b[8] * u[4] + b[11] * u[6];
-    double r[9] = {rr, 0.0, 0.0, 0.0, tt, 0.0, 0.0, 0.0, zz};
-    if (mode == 2) {
-        const double s = 0.5 * (b[0] * u[0] + b[3] * u[2] + b[6] * u[4] + b[9] * u[6] + b[2] * u[1] + b[5] * u[3] +
-                                b[8] * u[5] + b[11] * u[7]);
-        r[2] = s;
-        r[6] = s;
+    if (t >= nelem * R.nip) return;
+    const int64_t e = t / R.nip;
+    const int q = static_cast<int>(t - e * R.nip);
+    axi_point_geometry(R, q, x + 8 * e, G + 12 * t, vol[t]);
+}
+
+// gradN_vector (mode 0, :140-169), gradN_vector_T (1, :171-200), symGradN_vector (2, :202-233).
+// A workgroup owns BS / nip whole elements, one thread per point; coordinates, element vectors and tensors
+// go through LDS as contiguous 16-byte streams.  Bound by HBM, 416 bytes per element (736 with the stored
+// geometry): 300 k elements 47 -> 24.5 us.
+__global__ void __launch_bounds__(BS) k_axi_grad(int64_t nelem, AxiRule R, int mode, const double* __restrict__ x,
+                                                 const double* __restrict__ u_, double* __restrict__ out)
+{
+    extern __shared__ __align__(16) double smem[];
+    const int EB = BS / R.nip;
+    double *s_o = smem, *s_x = s_o + 9 * BS, *s_u = s_x + 8 * EB;
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * EB;
+    const int ne = static_cast<int>(min<int64_t>(EB, nelem - e0)), np = ne * R.nip;
+    stage_in<double, BS, 1>(s_x, x + 8 * e0, 8 * ne);
+    stage_in<double, BS, 1>(s_u, u_ + 8 * e0, 8 * ne);
+    __syncthreads();
+    if (threadIdx.x < np) {
+        const int el = threadIdx.x / R.nip, q = threadIdx.x - el * R.nip;
+        double b[12], v;
+        axi_point_geometry(R, q, s_x + 8 * el, b, v);
+        const double* u = s_u + 8 * el; // (u_z, u_r) per node
+        const double rr = b[0] * u[1] + b[3] * u[3] + b[6] * u[5] + b[9] * u[7];
+        const double tt = b[1] * u[1] + b[4] * u[3] + b[7] * u[5] + b[10] * u[7];
+        const double zz = b[2] * u[0] + b[5] * u[2] + b[8] * u[4] + b[11] * u[6];
+        double r2, r6;
+        if (mode == 2) {
+            r2 = r6 = 0.5 * (b[0] * u[0] + b[3] * u[2] + b[6] * u[4] + b[9] * u[6] + b[2] * u[1] + b[5] * u[3] +
+                             b[8] * u[5] + b[11] * u[7]);
+        }
+        else {
+            const double dzr = b[0] * u[0] + b[3] * u[2] + b[6] * u[4] + b[9] * u[6];
+            const double drz = b[2] * u[1] + b[5] * u[3] + b[8] * u[5] + b[11] * u[7];
+            r2 = mode == 0 ? dzr : drz;
+            r6 = mode == 0 ? drz : dzr;
+        }
+        double* o = s_o + 9 * threadIdx.x;
+        o[0] = rr;
+        o[1] = 0.0;
+        o[2] = r2;
+        o[3] = 0.0;
+        o[4] = tt;
+        o[5] = 0.0;
+        o[6] = r6;
+        o[7] = 0.0;
+        o[8] = zz;
     }
-    else {
-        const double dzr = b[0] * u[0] + b[3] * u[2] + b[6] * u[4] + b[9] * u[6];
-        const double drz = b[2] * u[1] + b[5] * u[3] + b[8] * u[5] + b[11] * u[7];
-        r[mode == 0 ? 2 : 6] = dzr;
-        r[mode == 0 ? 6 : 2] = drz;
-    }
-    double* o = out + 9 * t;
-    for (int k = 0; k < 9; ++k) o[k] = r[k];
+    __syncthreads();
+    stage_out<double, BS>(out + 9 * e0 * R.nip, s_o, 9 * np);
 }
 
 // one thread per (element, node m, node n): the 2 x 2 block K(m *, n *) of the element matrix
@@ -115,24 +141,47 @@ __global__ void k_axi_int_N(int64_t nelem, AxiRule R, const double* __restrict__
     Me[(2 * m + 1) * 8 + 2 * k + 1] = c;
 }
 
-// int_gradN_dot_tensor2_dV (:268-296): one thread per (element, node)
-__global__ void k_axi_int_t2(int64_t nelem, int nip, const double* __restrict__ G, const double* __restrict__ vol,
-                             const double* __restrict__ sig, double* __restrict__ f)
+// int_gradN_dot_tensor2_dV (:268-296): one thread per point forms the point's contributions to the four
+// nodes (in place of its tensor in LDS), then one thread per (element, node) adds them in point order.
+// Bound by HBM, 416 bytes per element (768 with the stored geometry): 300 k elements
+// 47.5 -> 26 us.
+__global__ void __launch_bounds__(BS) k_axi_int_t2(int64_t nelem, AxiRule R, const double* __restrict__ x,
+                                                   const double* __restrict__ sig, double* __restrict__ f)
 {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= nelem * 4) return;
-    const int64_t e = t / 4;
-    const int m = static_cast<int>(t % 4);
-    double f0 = 0.0, f1 = 0.0;
-    for (int q = 0; q < nip; ++q) {
-        const double* b = G + 12 * (e * nip + q) + 3 * m;
-        const double* s = sig + 9 * (e * nip + q);
-        const double v = vol[e * nip + q];
-        f0 += v * (b[2] * s[8] + b[0] * s[2]);
-        f1 += v * (b[0] * s[0] + b[1] * s[4] + b[2] * s[6]);
+    extern __shared__ __align__(16) double smem[];
+    const int EB = BS / R.nip;
+    double *s_s = smem, *s_x = s_s + 9 * BS; // s_x: coordinates, then the element vectors
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * EB;
+    const int ne = static_cast<int>(min<int64_t>(EB, nelem - e0)), np = ne * R.nip;
+    stage_in<double, BS, 5>(s_s, sig + 9 * e0 * R.nip, 9 * np);
+    stage_in<double, BS, 1>(s_x, x + 8 * e0, 8 * ne);
+    __syncthreads();
+    if (threadIdx.x < np) {
+        const int el = threadIdx.x / R.nip, q = threadIdx.x - el * R.nip;
+        double b[12], v, s[9];
+        axi_point_geometry(R, q, s_x + 8 * el, b, v);
+        double* c = s_s + 9 * threadIdx.x;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s[k] = c[k];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            c[2 * m] = v * (b[3 * m + 2] * s[8] + b[3 * m] * s[2]);
+            c[2 * m + 1] = v * (b[3 * m] * s[0] + b[3 * m + 1] * s[4] + b[3 * m + 2] * s[6]);
+        }
     }
-    f[8 * e + 2 * m] = f0;
-    f[8 * e + 2 * m + 1] = f1;
+    __syncthreads();
+    for (int t = threadIdx.x; t < 4 * ne; t += BS) {
+        const double* c = s_s + (t / 4) * R.nip * 9 + 2 * (t % 4);
+        double f0 = 0.0, f1 = 0.0;
+        for (int q = 0; q < R.nip; ++q) {
+            f0 += c[9 * q];
+            f1 += c[9 * q + 1];
+        }
+        s_x[2 * t] = f0;
+        s_x[2 * t + 1] = f1;
+    }
+    __syncthreads();
+    stage_out<double, BS>(f + 8 * e0, s_x, 8 * ne);
 }
 
 // int_gradN_dot_tensor4_dot_gradNT_dV (:298-398)
@@ -164,7 +213,9 @@ __global__ void k_axi_int_t4(int64_t nelem, int nip, const double* __restrict__ 
 void compute(gf_axi m, const double* x, hipStream_t s)
 {
     const int64_t n = m->nelem * m->rule.nip;
-    if (n) k_axi_geometry<<<nblocks(n, BS), BS, 0, s>>>(m->nelem, m->rule, x, m->G.p, m->vol.p);
+    if (!n) return;
+    GF_HIP(hipMemcpyAsync(m->x.p, x, m->x.n * sizeof(double), hipMemcpyDeviceToDevice, s));
+    k_axi_geometry<<<nblocks(n, BS), BS, 0, s>>>(m->nelem, m->rule, x, m->G.p, m->vol.p);
     check_launch();
 }
 
@@ -200,6 +251,7 @@ int gf_axi_create(gf_axi* out, int64_t nelem, int nip, const double* x, const do
                 R.dNxi[q][3][1] = +0.25 * (1.0 - a);
                 R.w[q] = w_h[q];
             }
+            m->x.alloc(8 * nelem);
             m->G.alloc(12 * nelem * nip);
             m->vol.alloc(nelem * nip);
             compute(m, x, S(stream));
@@ -240,8 +292,9 @@ int gf_axi_grad(gf_axi m, int mode, const double* elemvec, double* qtensor, void
     return guard([&] {
         GF_REQUIRE(m && elemvec && qtensor, "null argument");
         GF_REQUIRE(mode >= 0 && mode <= 2, "mode: 0 gradN_vector, 1 gradN_vector_T, 2 symGradN_vector");
-        const int64_t n = m->nelem * m->rule.nip;
-        if (n) k_axi_grad<<<nblocks(n, BS), BS, 0, S(stream)>>>(n, m->rule.nip, mode, m->G.p, elemvec, qtensor);
+        if (m->nelem)
+            k_axi_grad<<<nblocks(m->nelem, BS / m->rule.nip), BS, (9 * BS + 16 * (BS / m->rule.nip)) * sizeof(double),
+                         S(stream)>>>(m->nelem, m->rule, mode, m->x.p, elemvec, qtensor);
         check_launch();
     });
 }
@@ -261,8 +314,8 @@ int gf_axi_int_gradN_dot_tensor2_dV(gf_axi m, const double* qtensor, double* ele
     return guard([&] {
         GF_REQUIRE(m && qtensor && elemvec, "null argument");
         if (m->nelem)
-            k_axi_int_t2<<<nblocks(4 * m->nelem, BS), BS, 0, S(stream)>>>(m->nelem, m->rule.nip, m->G.p, m->vol.p,
-                                                                         qtensor, elemvec);
+            k_axi_int_t2<<<nblocks(m->nelem, BS / m->rule.nip), BS, (9 * BS + 8 * (BS / m->rule.nip)) * sizeof(double),
+                           S(stream)>>>(m->nelem, m->rule, m->x.p, qtensor, elemvec);
         check_launch();
     });
 }

@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "gf_internal.hpp"
+#include "gf_stage.hpp"
 
 using namespace gf;
 
@@ -94,6 +95,24 @@ inline void default_rule(int et, int rule, std::vector<double>& xi, std::vector<
 // ElementQuad4.h:493-532, ElementQuad4Planar.h:280-319 (x thick), Element.h:1178-1229 (Hex8, with
 // the chain rule over j)
 
+// dN/dx [4][2] and det J of one Quad4 point.  Shared by the set-up kernel and the kernels that recompute
+// the geometry, so all produce the same bits.
+__device__ inline void quad4_point_geometry(const double* __restrict__ xe, const double* __restrict__ g, double* o,
+                                            double& det)
+{
+    double J00 = g[0] * xe[0] + g[2] * xe[2] + g[4] * xe[4] + g[6] * xe[6];
+    double J01 = g[0] * xe[1] + g[2] * xe[3] + g[4] * xe[5] + g[6] * xe[7];
+    double J10 = g[1] * xe[0] + g[3] * xe[2] + g[5] * xe[4] + g[7] * xe[6];
+    double J11 = g[1] * xe[1] + g[3] * xe[3] + g[5] * xe[5] + g[7] * xe[7];
+    det = J00 * J11 - J01 * J10; // detail.h:17-37
+    double I00 = J11 / det, I01 = -1.0 * J01 / det, I10 = -1.0 * J10 / det, I11 = J00 / det;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        o[m * 2 + 0] = I00 * g[m * 2 + 0] + I01 * g[m * 2 + 1];
+        o[m * 2 + 1] = I10 * g[m * 2 + 0] + I11 * g[m * 2 + 1];
+    }
+}
+
 __global__ void k_compute_dN_quad4(int64_t n, int nip, int planar, double thick, const double* __restrict__ x,
                                    const double* __restrict__ dNxi, const double* __restrict__ w,
                                    double* __restrict__ dNx, double* __restrict__ vol)
@@ -102,20 +121,8 @@ __global__ void k_compute_dN_quad4(int64_t n, int nip, int planar, double thick,
     if (t >= n) return;
     int64_t e = t / nip;
     int q = static_cast<int>(t - e * nip);
-    const double* xe = x + e * 8;
-    const double* g = dNxi + q * 8;
-    double J00 = g[0] * xe[0] + g[2] * xe[2] + g[4] * xe[4] + g[6] * xe[6];
-    double J01 = g[0] * xe[1] + g[2] * xe[3] + g[4] * xe[5] + g[6] * xe[7];
-    double J10 = g[1] * xe[0] + g[3] * xe[2] + g[5] * xe[4] + g[7] * xe[6];
-    double J11 = g[1] * xe[1] + g[3] * xe[3] + g[5] * xe[5] + g[7] * xe[7];
-    double det = J00 * J11 - J01 * J10; // detail.h:17-37
-    double I00 = J11 / det, I01 = -1.0 * J01 / det, I10 = -1.0 * J10 / det, I11 = J00 / det;
-    double* o = dNx + t * 8;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        o[m * 2 + 0] = I00 * g[m * 2 + 0] + I01 * g[m * 2 + 1];
-        o[m * 2 + 1] = I10 * g[m * 2 + 0] + I11 * g[m * 2 + 1];
-    }
+    double det;
+    quad4_point_geometry(x + e * 8, dNxi + q * 8, dNx + t * 8, det);
     vol[t] = planar ? w[q] * det * thick : w[q] * det;
 }
 
@@ -172,59 +179,47 @@ __global__ void k_compute_dN_hex8(int64_t n, int nip, const double* __restrict__
     vol[t] = w[q] * det;
 }
 
+// The FP32 copies of a Hex8 quadrature's dN/dx and dV: formed in FP64 again from the coordinates (192 bytes
+// per element) and rounded once, which is the stored FP64 value rounded (1,600 bytes per element to read);
+// the rows leave through LDS as one contiguous stream.
+constexpr int GB32 = 256; // points per workgroup
+
+inline size_t geo32_lds_bytes(int nip)
+{
+    return static_cast<size_t>(GB32) * 24 * 4 + (GB32 / nip + 2) * 25 * 8 + static_cast<size_t>(nip) * 25 * 8;
+}
+
+__global__ void __launch_bounds__(GB32) k_geometry32_hex8(int64_t n, int nip, const double* __restrict__ x,
+                                                          const double* __restrict__ dNxi,
+                                                          const double* __restrict__ w, float* __restrict__ dNx,
+                                                          float* __restrict__ vol)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* s_o = reinterpret_cast<float*>(smem);                // [GB32][24]
+    double* s_x = reinterpret_cast<double*>(s_o + GB32 * 24);   // [GB32 / nip + 2][25]
+    double* s_d = s_x + (GB32 / nip + 2) * 25;                  // [nip][25]
+    const int64_t t0 = blockIdx.x * static_cast<int64_t>(GB32);
+    const int nq = static_cast<int>(min<int64_t>(GB32, n - t0));
+    const int64_t e0 = t0 / nip, e1 = (t0 + nq - 1) / nip;
+    stage_in_rows<double, GB32, 24>(s_x, x + e0 * 24, static_cast<int>(e1 - e0 + 1));
+    for (int i = threadIdx.x; i < nip * 24; i += GB32) s_d[i + i / 24] = dNxi[i];
+    __syncthreads();
+    if (threadIdx.x < nq) {
+        const int p = static_cast<int>(t0 - e0 * nip) + threadIdx.x, el = p / nip, q = p - el * nip;
+        double gd[24], det;
+        hex8_point_geometry(s_x + el * 25, s_d + q * 25, gd, det);
+#pragma unroll
+        for (int k = 0; k < 24; ++k) s_o[threadIdx.x * 24 + k] = static_cast<float>(gd[k]);
+        vol[t0 + threadIdx.x] = static_cast<float>(w[q] * det);
+    }
+    __syncthreads();
+    stage_out<float, GB32>(dNx + t0 * 24, s_o, nq * 24);
+}
+
 __global__ void k_to_f32(int64_t n, const double* __restrict__ a, float* __restrict__ b)
 {
     int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (t < n) b[t] = static_cast<float>(a[t]);
-}
-
-// ---- LDS staging of contiguous slices ---------------------------------------------------------------
-// The quadrature kernels read and write per-point / per-element records (dN/dx rows, element
-// vectors, tensors) of 8 to 72 bytes.  A workgroup moves its contiguous slice of each array between
-// HBM and LDS with full-wave contiguous 16-byte accesses (when the array is 16-byte aligned; element
-// by element otherwise) and the threads compute on LDS, so no global access is strided per lane.
-template <class T, int NT, int KB>
-__device__ inline void stage_in(T* __restrict__ lds, const T* __restrict__ g, int count)
-{
-    // KB: 16-byte loads in flight per thread before their LDS writes (the call site's typical count)
-    constexpr int VW = 16 / static_cast<int>(sizeof(T));
-    typedef T V __attribute__((ext_vector_type(VW)));
-    int done = 0;
-    if ((reinterpret_cast<uintptr_t>(g) & 15) == 0) {
-        const int nv = count / VW;
-        for (int base = 0; base < nv; base += KB * NT) {
-            V r[KB];
-            // unconditional loads (an index past the end re-reads the last chunk), so that all KB
-            // are issued before the first wait
-#pragma unroll
-            for (int k = 0; k < KB; ++k) {
-                const int i = base + k * NT + threadIdx.x;
-                r[k] = reinterpret_cast<const V*>(g)[i < nv ? i : nv - 1];
-            }
-#pragma unroll
-            for (int k = 0; k < KB; ++k) {
-                const int i = base + k * NT + threadIdx.x;
-                if (i < nv) reinterpret_cast<V*>(lds)[i] = r[k];
-            }
-        }
-        done = nv * VW;
-    }
-    for (int i = done + threadIdx.x; i < count; i += NT) lds[i] = g[i];
-}
-
-template <class T, int NT>
-__device__ inline void stage_out(T* __restrict__ g, const T* __restrict__ lds, int count)
-{
-    constexpr int VW = 16 / static_cast<int>(sizeof(T));
-    typedef T V __attribute__((ext_vector_type(VW)));
-    int done = 0;
-    if ((reinterpret_cast<uintptr_t>(g) & 15) == 0) {
-        const int nv = count / VW;
-        for (int i = threadIdx.x; i < nv; i += NT)
-            __builtin_nontemporal_store(reinterpret_cast<const V*>(lds)[i], reinterpret_cast<V*>(g) + i);
-        done = nv * VW;
-    }
-    for (int i = done + threadIdx.x; i < count; i += NT) g[i] = lds[i];
 }
 
 // ---- gradients: mode 0 GradN_vector, 1 GradN_vector_T, 2 SymGradN_vector -------------------------
@@ -232,34 +227,40 @@ __device__ inline void stage_out(T* __restrict__ g, const T* __restrict__ lds, i
 // GradN_vector (mode 0), GradN_vector_T (1), SymGradN_vector (2): 2-D node vectors (Quad4 tdim 2 /
 // planar tdim 3, ElementQuad4.h:348-434, ElementQuad4Planar.h:129-221) and Hex8 (the generic loops of
 // Element.h:924-1022), in the reference's expression order.  A workgroup of QB threads owns QB
-// consecutive points (e, q); LDS holds their dN/dx rows [QB][nne nd], the element vectors of the
-// elements they span, and the output tensors [QB][TD TD].
-template <int ND>
-inline size_t grad_lds_bytes(int qb, int nip, int td, size_t sz)
-{
-    const int nn = ND == 2 ? 8 : 24;
-    return (static_cast<size_t>(qb) * nn + static_cast<size_t>(qb) * td * td + (qb / nip + 2) * static_cast<size_t>(nn)) * sz;
-}
-
+// consecutive points (e, q) and moves its slices through LDS.
+//
+// Quad4: bound by HBM.  dN/dx of a point is formed from the 64 bytes of element coordinates with
+// quad4_point_geometry, the function that produced the stored ones (FP32: the FP64 dN/dx rounded once, as
+// the stored FP32 copy is), so the results are the stored geometry's bit for bit, for 416 instead of 608
+// bytes per element (planar, FP64; FP32 240 instead of 304).  2.0 M planar elements: 217 -> 137 us FP64 (6.1 TB/s), 102 -> 93 us
+// FP32.
 template <class T, int TD, int mode>
-__global__ void __launch_bounds__(256) k_grad_2d_lds(int64_t n, int nip, const T* __restrict__ dNx,
-                                                     const T* __restrict__ elemvec, T* __restrict__ qtensor)
+__global__ void __launch_bounds__(256) k_grad_2d_x(int64_t n, int nip, const double* __restrict__ x,
+                                                   const double* __restrict__ dNxi, const T* __restrict__ elemvec,
+                                                   T* __restrict__ qtensor)
 {
     constexpr int QB = 256;
     extern __shared__ __align__(16) unsigned char smem[];
-    T* s_o = reinterpret_cast<T*>(smem); // [QB][TD*TD]
-    T* s_g = s_o + QB * TD * TD;           // [QB][8]
-    T* s_u = s_g + QB * 8;           // [elements][8]
+    const int nemax = QB / nip + 2;
+    double* s_x = reinterpret_cast<double*>(smem);  // [nemax][8]
+    T* s_u = reinterpret_cast<T*>(s_x + nemax * 8); // [nemax][8]
+    T* s_o = s_u + nemax * 8;                        // [QB][TD TD]
     const int64_t t0 = static_cast<int64_t>(blockIdx.x) * QB;
     const int nq = static_cast<int>(min<int64_t>(QB, n - t0));
     const int64_t e0 = t0 / nip, e1 = (t0 + nq - 1) / nip;
-    stage_in<T, QB, 8 / (16 / sizeof(T))>(s_g, dNx + t0 * 8, nq * 8);
-    stage_in<T, QB, 1>(s_u, elemvec + e0 * 8, static_cast<int>(e1 - e0 + 1) * 8);
+    const int ne = static_cast<int>(e1 - e0 + 1);
+    stage_in<double, QB, 1>(s_x, x + e0 * 8, ne * 8);
+    stage_in<T, QB, 1>(s_u, elemvec + e0 * 8, ne * 8);
     __syncthreads();
     if (threadIdx.x < nq) {
-        const int64_t e = (t0 + threadIdx.x) / nip;
-        const T* u = s_u + (e - e0) * 8;
-        const T* g = s_g + threadIdx.x * 8;
+        // point t0 + threadIdx.x: t0 = e0 nip + (t0 % nip), so the division is a 32-bit one
+        const int p = static_cast<int>(t0 - e0 * nip) + threadIdx.x, el = p / nip, q = p - el * nip;
+        double gd[8], det;
+        quad4_point_geometry(s_x + el * 8, dNxi + q * 8, gd, det);
+        T g[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) g[k] = static_cast<T>(gd[k]);
+        const T* u = s_u + el * 8;
         T a00 = g[0] * u[0] + g[2] * u[2] + g[4] * u[4] + g[6] * u[6];
         T a01 = g[0] * u[1] + g[2] * u[3] + g[4] * u[5] + g[6] * u[7];
         T a10 = g[1] * u[0] + g[3] * u[2] + g[5] * u[4] + g[7] * u[6];
@@ -292,6 +293,19 @@ __global__ void __launch_bounds__(256) k_grad_2d_lds(int64_t n, int nip, const T
     }
     __syncthreads();
     stage_out<T, QB>(qtensor + t0 * TD * TD, s_o, nq * TD * TD);
+}
+
+inline size_t grad2x_lds_bytes(int nip, int td, size_t sz)
+{
+    const size_t ne = 256 / nip + 2;
+    return ne * 8 * 8 + ne * 8 * sz + 256 * static_cast<size_t>(td * td) * sz;
+}
+
+// Hex8 with the stored geometry: rules of so few points that the coordinates of a workgroup's elements
+// outgrow LDS.  LDS holds the points' dN/dx rows [QB][24], element vectors and output tensors.
+inline size_t grad3_lds_bytes(int qb, int nip, size_t sz)
+{
+    return (static_cast<size_t>(qb) * 24 + static_cast<size_t>(qb) * 9 + (qb / nip + 2) * 24) * sz;
 }
 
 template <class T, int mode>
@@ -372,14 +386,13 @@ __global__ void __launch_bounds__(QB3) k_grad_3d_x(int64_t n, int nip, const dou
     for (int i = threadIdx.x; i < nip * 24; i += QB3) s_d[i] = dNxi[i];
     __syncthreads();
     if (threadIdx.x < nq) {
-        const int64_t t = t0 + threadIdx.x, e = t / nip;
-        const int q = static_cast<int>(t - e * nip);
+        const int p = static_cast<int>(t0 - e0 * nip) + threadIdx.x, el = p / nip, q = p - el * nip;
         double gd[24], det;
-        hex8_point_geometry(s_x + (e - e0) * 24, s_d + q * 24, gd, det);
+        hex8_point_geometry(s_x + el * 24, s_d + q * 24, gd, det);
         T g[24];
 #pragma unroll
         for (int k = 0; k < 24; ++k) g[k] = static_cast<T>(gd[k]);
-        const T* u = s_u + (e - e0) * 24;
+        const T* u = s_u + el * 24;
         T r[9];
 #pragma unroll
         for (int k = 0; k < 9; ++k) r[k] = T(0);
@@ -486,53 +499,156 @@ __global__ void k_int_tensor2(int64_t n, int nip, int nne, const T* __restrict__
     for (int j = 0; j < ND; ++j) elemvec[t * ND + j] = f[j];
 }
 
-// Staged form of k_int_tensor2: a workgroup of EB NNE threads owns EB consecutive elements; LDS
-// holds their dN/dx [EB nip NNE ND], dV [EB nip], tensors [EB nip TD TD] and the output element
-// vectors [EB NNE ND].  Thread (e, m) sums over the points in the order of k_int_tensor2.
-template <class T, int NNE, int ND, int TD, int EB>
-__global__ void __launch_bounds__(EB* NNE) k_int_tensor2_lds(int64_t nelem, int nip, const T* __restrict__ dNx,
-                                                             const T* __restrict__ vol, const T* __restrict__ qtensor,
-                                                             T* __restrict__ elemvec)
+// The same integral with the geometry recomputed from the element coordinates, by the set-up's own
+// functions (bit-identical; FP32: dN/dx and dV rounded once, as the stored FP32 copies are).  A workgroup
+// owns PB / nip whole elements; one thread per point forms the point's contributions
+// (dN/dx(m, :) . sigma(:, j)) dV of every node from registers, then one thread per (element, node) adds
+// its points' contributions in order, from LDS: the order of k_int_tensor2, and the point's data is read
+// once instead of once per node.
+// Bound: HBM (Quad4; Hex8 FP64 close to FP64 issue).  Bytes per element, stored -> recomputed geometry:
+// Quad4 planar FP64 640 -> 416, FP32 320 -> 240; Hex8 FP64 2,368 -> 960, FP32 1,184 -> 576.
+// 2.0 M planar Quad4: 239 -> 142 us FP64 (5.9 TB/s), 128 -> 96 us FP32; 395 k Hex8: 178 -> 153 us FP64, 91 ->
+// 85 us FP32 (the stored FP32 geometry, below).
+constexpr int PB2 = 256; // Quad4 points per workgroup
+
+template <class T, int TD>
+__global__ void __launch_bounds__(PB2) k_int_tensor2_q4(int64_t nelem, int nip, int planar, double thick,
+                                                        const double* __restrict__ x, const double* __restrict__ dNxi,
+                                                        const double* __restrict__ w, const T* __restrict__ qtensor,
+                                                        T* __restrict__ elemvec)
 {
-    constexpr int NT = EB * NNE;
+    constexpr int ROW = TD * TD > 8 ? TD * TD : 8; // a point's contributions overwrite its tensor
+    constexpr int TB = TD * TD == ROW ? 0 : PB2 * ROW; // (TD = 2: the tensors lie behind them)
     extern __shared__ __align__(16) unsigned char smem[];
+    const int EB = PB2 / nip; // elements of the workgroup
+    T* s_c = reinterpret_cast<T*>(smem);                        // [PB2][ROW]
+    T* s_s = s_c + TB;                                          // [PB2][TD TD]
+    double* s_x = reinterpret_cast<double*>(s_s + PB2 * TD * TD); // [EB][8], then the element vectors
     const int64_t e0 = static_cast<int64_t>(blockIdx.x) * EB;
-    const int ne = static_cast<int>(min<int64_t>(EB, nelem - e0));
-    T* s_g = reinterpret_cast<T*>(smem); // EB nip NNE ND
-    T* s_s = s_g + EB * nip * NNE * ND;   // EB nip TD TD
-    T* s_o = s_s + EB * nip * TD * TD;    // EB NNE ND
-    T* s_v = s_o + EB * NNE * ND;         // EB nip
-    stage_in<T, NT, NNE * ND / (16 / sizeof(T))>(s_g, dNx + e0 * nip * NNE * ND, ne * nip * NNE * ND);
-    stage_in<T, NT, (TD * TD + (16 / sizeof(T)) - 1) / (16 / sizeof(T))>(s_s, qtensor + e0 * nip * TD * TD, ne * nip * TD * TD);
-    stage_in<T, NT, 1>(s_v, vol + e0 * nip, ne * nip);
+    const int ne = static_cast<int>(min<int64_t>(EB, nelem - e0)), np = ne * nip;
+    stage_in<T, PB2, (TD * TD * sizeof(T) + 15) / 16>(s_s, qtensor + e0 * nip * TD * TD, np * TD * TD);
+    stage_in<double, PB2, 1>(s_x, x + e0 * 8, ne * 8);
     __syncthreads();
-    const int el = threadIdx.x / NNE, m = threadIdx.x - el * NNE;
-    if (el < ne) {
-        T f[ND];
+    if (threadIdx.x < np) {
+        const int el = threadIdx.x / nip, q = threadIdx.x - el * nip;
+        double gd[8], det;
+        quad4_point_geometry(s_x + el * 8, dNxi + q * 8, gd, det);
+        const T v = static_cast<T>(planar ? w[q] * det * thick : w[q] * det);
+        T s[TD * TD], c[8];
 #pragma unroll
-        for (int j = 0; j < ND; ++j) f[j] = T(0);
-        for (int q = 0; q < nip; ++q) {
-            const T* g = s_g + ((el * nip + q) * NNE + m) * ND;
-            const T* sq = s_s + (el * nip + q) * TD * TD;
-            T v = s_v[el * nip + q];
+        for (int k = 0; k < TD * TD; ++k) s[k] = s_s[threadIdx.x * TD * TD + k];
 #pragma unroll
-            for (int j = 0; j < ND; ++j) {
-                T a = g[0] * sq[0 * TD + j] + g[1] * sq[1 * TD + j];
-                if (ND == 3) a = a + g[2] * sq[2 * TD + j];
-                f[j] += a * v;
+        for (int m = 0; m < 4; ++m) {
+            const T g0 = static_cast<T>(gd[2 * m]), g1 = static_cast<T>(gd[2 * m + 1]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const T a = g0 * s[j] + g1 * s[TD + j];
+                c[2 * m + j] = a * v;
             }
         }
 #pragma unroll
-        for (int j = 0; j < ND; ++j) s_o[(el * NNE + m) * ND + j] = f[j];
+        for (int k = 0; k < 8; ++k) s_c[threadIdx.x * ROW + k] = c[k];
     }
     __syncthreads();
-    stage_out<T, NT>(elemvec + e0 * NNE * ND, s_o, ne * NNE * ND);
+    T* s_o = reinterpret_cast<T*>(s_x);
+    for (int t = threadIdx.x; t < ne * 4; t += PB2) {
+        const T* c = s_c + (t / 4) * nip * ROW + (t % 4) * 2;
+        T f0 = T(0), f1 = T(0);
+        for (int q = 0; q < nip; ++q) {
+            f0 += c[q * ROW];
+            f1 += c[q * ROW + 1];
+        }
+        s_o[2 * t] = f0;
+        s_o[2 * t + 1] = f1;
+    }
+    __syncthreads();
+    stage_out<T, PB2>(elemvec + e0 * 8, s_o, ne * 8);
 }
 
-template <class T, int NNE, int ND, int TD, int EB>
-inline size_t int2_lds_bytes(int nip)
+inline size_t int2_q4_lds_bytes(int nip, int td, size_t sz)
 {
-    return static_cast<size_t>(EB) * (nip * NNE * ND + nip * TD * TD + NNE * ND + nip) * sizeof(T);
+    return static_cast<size_t>(PB2) * (td == 3 ? 9 : 12) * sz + static_cast<size_t>(PB2 / nip) * 8 * 8;
+}
+
+constexpr int PB3 = 128; // Hex8 points per workgroup
+
+// FP32 reads the stored FP32 geometry (each thread its point's 96 bytes; gx, gv), FP64 the coordinates
+// (gx) and weights (gv).
+template <class T>
+__global__ void __launch_bounds__(PB3) k_int_tensor2_h8(int64_t nelem, int nip, const T* __restrict__ gx,
+                                                        const double* __restrict__ dNxi, const T* __restrict__ gv,
+                                                        const T* __restrict__ qtensor, T* __restrict__ elemvec)
+{
+    constexpr bool STORED = std::is_same_v<T, float>;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int EB = PB3 / nip;
+    T* s_c = reinterpret_cast<T*>(smem);                  // [PB3][13]: four nodes' contributions at a time
+    T* s_s = s_c + PB3 * 13;                              // [PB3][9], then the element vectors [EB][24]
+    double* s_x = reinterpret_cast<double*>(s_s + PB3 * 24 / (nip < 2 ? 1 : 2)); // [EB][25] (FP64)
+    double* s_d = s_x + EB * 25;                          // [nip][25] (FP64)
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * EB;
+    const int ne = static_cast<int>(min<int64_t>(EB, nelem - e0)), np = ne * nip;
+    stage_in<T, PB3, (9 * sizeof(T) + 15) / 16>(s_s, qtensor + e0 * nip * 9, np * 9);
+    const int el = threadIdx.x / nip, q = threadIdx.x - el * nip;
+    T g[24], s[9], v = T(0);
+    if constexpr (STORED) {
+        typedef float V __attribute__((ext_vector_type(4)));
+        const int64_t t = e0 * nip + min(static_cast<int>(threadIdx.x), np - 1);
+        const V* row = reinterpret_cast<const V*>(gx + t * 24);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const V r = row[k];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) g[4 * k + i] = r[i];
+        }
+        v = gv[t];
+    }
+    else {
+        stage_in_rows<double, PB3, 24>(s_x, gx + e0 * 24, ne);
+        for (int i = threadIdx.x; i < nip * 24; i += PB3) s_d[i + i / 24] = dNxi[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < np) {
+        if constexpr (!STORED) {
+            double det;
+            hex8_point_geometry(s_x + el * 25, s_d + q * 25, g, det);
+            v = gv[q] * det;
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s[k] = s_s[threadIdx.x * 9 + k];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads(); // the tensors (h = 0), then the first nodes' contributions (h = 1) are read
+        if (threadIdx.x < np) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const T* gm = g + (4 * h + m) * 3;
+                    T a = gm[0] * s[j] + gm[1] * s[3 + j];
+                    a = a + gm[2] * s[6 + j];
+                    s_c[threadIdx.x * 13 + m * 3 + j] = a * v;
+                }
+        }
+        __syncthreads();
+        for (int t = threadIdx.x; t < ne * 12; t += PB3) {
+            const int e = t / 12, k = t - e * 12;
+            const T* c = s_c + e * nip * 13 + k;
+            T f = T(0);
+            for (int i = 0; i < nip; ++i) f += c[i * 13];
+            s_s[e * 24 + 12 * h + k] = f;
+        }
+    }
+    __syncthreads();
+    stage_out<T, PB3>(elemvec + e0 * 24, s_s, ne * 24);
+}
+
+// (at least 9 values per point and 24 per element behind the contributions)
+inline size_t int2_h8_lds_bytes(int nip, size_t sz)
+{
+    return static_cast<size_t>(PB3) * 13 * sz + static_cast<size_t>(PB3) * 24 / (nip < 2 ? 1 : 2) * sz +
+           (sz == 4 ? 0 : static_cast<size_t>(PB3 / nip) * 25 * 8 + static_cast<size_t>(nip) * 25 * 8);
 }
 
 // Int_gradN_dot_tensor4_dot_gradNT_dV FP64 (Element.h:1131-1176): thread per (e, m, n) block
@@ -658,23 +774,38 @@ __global__ void __launch_bounds__(4 * T4_EB)
 
 // ---- material ----------------------------------------------------------------------------------
 
+// Linear elastic stress per point.  Bound by HBM (72 + 16 bytes read, 72 written per 3 x 3 point in FP64):
+// the tensors go through LDS in whole 16-byte streams, in place; a thread reading and writing its own
+// 72-byte record took 315 us for 8.0 M points in FP64, 229 us this way (5.3 TB/s).  In FP32 the two are level
+// by themselves (103 and 113 us), but the streaming stores leave the caches to the next kernel: the whole
+// force evaluation is 1.5 to 2 % faster.
 template <class T, int TD>
-__global__ void k_elastic_stress(int64_t n, const T* __restrict__ eps, const T* __restrict__ K,
-                                 const T* __restrict__ G, T* __restrict__ sig)
+__global__ void __launch_bounds__(BS) k_elastic_stress(int64_t n, const T* __restrict__ eps, const T* __restrict__ K,
+                                                       const T* __restrict__ G, T* __restrict__ sig)
 {
-    int64_t p = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (p >= n) return;
-    const T* e = eps + p * TD * TD;
-    T* s = sig + p * TD * TD;
-    T tr = (TD == 3) ? e[0] + e[4] + e[8] : e[0] + e[3];
-    T k = K[p], g = G[p];
+    __shared__ __align__(16) T s_t[BS * TD * TD];
+    const int64_t p0 = blockIdx.x * static_cast<int64_t>(BS);
+    const int np = static_cast<int>(min<int64_t>(BS, n - p0));
+    const int64_t p = p0 + min(static_cast<int>(threadIdx.x), np - 1);
+    const T k = K[p], g = G[p];
+    stage_in<T, BS, (TD * TD * sizeof(T) + 15) / 16>(s_t, eps + p0 * TD * TD, np * TD * TD);
+    __syncthreads();
+    if (threadIdx.x < np) {
+        T* s = s_t + threadIdx.x * TD * TD;
+        T e[TD * TD];
 #pragma unroll
-    for (int i = 0; i < TD; ++i)
+        for (int i = 0; i < TD * TD; ++i) e[i] = s[i];
+        T tr = (TD == 3) ? e[0] + e[4] + e[8] : e[0] + e[3];
 #pragma unroll
-        for (int j = 0; j < TD; ++j) {
-            if (i == j) s[i * TD + j] = k * tr + T(2) * g * (e[i * TD + j] - tr / T(3));
-            else s[i * TD + j] = T(2) * g * e[i * TD + j];
-        }
+        for (int i = 0; i < TD; ++i)
+#pragma unroll
+            for (int j = 0; j < TD; ++j) {
+                if (i == j) s[i * TD + j] = k * tr + T(2) * g * (e[i * TD + j] - tr / T(3));
+                else s[i * TD + j] = T(2) * g * e[i * TD + j];
+            }
+    }
+    __syncthreads();
+    stage_out<T, BS>(sig + p0 * TD * TD, s_t, np * TD * TD);
 }
 
 // Tangent C_ijab = K d_ij d_ab + 2 G (0.5 (d_ia d_jb + d_ib d_ja) - d_ij d_ab / 3) per point.  Every
@@ -772,8 +903,13 @@ void ensure32(gf_quad_s* q, hipStream_t s)
     int64_t n1 = q->nelem * q->nip * q->nne * q->ndim, n2 = q->nelem * q->nip;
     if (q->dNx32.n != static_cast<size_t>(n1)) q->dNx32.alloc(n1);
     if (q->vol32.n != static_cast<size_t>(n2)) q->vol32.alloc(n2);
-    if (n1) k_to_f32<<<nblocks(n1, BS), BS, 0, s>>>(n1, q->dNx.p, q->dNx32.p);
-    if (n2) k_to_f32<<<nblocks(n2, BS), BS, 0, s>>>(n2, q->vol.p, q->vol32.p);
+    if (n2 && q->et == GF_HEX8 && geo32_lds_bytes(q->nip) <= 65536)
+        k_geometry32_hex8<<<nblocks(n2, GB32), GB32, geo32_lds_bytes(q->nip), s>>>(n2, q->nip, q->x.p, q->dNxi_d.p,
+                                                                                  q->w_d.p, q->dNx32.p, q->vol32.p);
+    else if (n2) {
+        k_to_f32<<<nblocks(n1, BS), BS, 0, s>>>(n1, q->dNx.p, q->dNx32.p);
+        k_to_f32<<<nblocks(n2, BS), BS, 0, s>>>(n2, q->vol.p, q->vol32.p);
+    }
     check_launch();
     q->have32 = true;
 }
@@ -786,37 +922,47 @@ int grad_dispatch(gf_quad q, const void* elemvec, void* qtensor, int dtype, int 
         int64_t n = q->nelem * q->nip;
         if (n == 0) return;
         hipStream_t s = S(stream);
-        auto launch = [&](auto tag, auto mtag, const auto* u, auto* o, const auto* g) {
+        auto geometry = [&](auto tag) { // the stored dN/dx in the arithmetic's type
+            if constexpr (std::is_same_v<decltype(tag), float>) {
+                ensure32(q, s);
+                return static_cast<const float*>(q->dNx32.p);
+            }
+            else
+                return static_cast<const double*>(q->dNx.p);
+        };
+        auto launch = [&](auto tag, auto mtag, const auto* u, auto* o) {
             using T = decltype(tag);
             constexpr int M = decltype(mtag)::value;
             const size_t sz = sizeof(T);
-            // Hex8 FP64: the geometry recomputed from the coordinates (1536 -> 192 bytes of dN/dx per
-            // element); FP32 reads the stored FP32 copy (768 bytes per element), cheaper than the
-            // FP64 recomputation; rules with few points per element: the stored geometry
-            if (q->et == GF_HEX8 && sizeof(T) == 8 && grad3x_lds_bytes(q->nip, sz) <= 65536)
-                k_grad_3d_x<T, M><<<nblocks(n, QB3), QB3, grad3x_lds_bytes(q->nip, sz), s>>>(n, q->nip, q->x.p,
-                                                                                             q->dNxi_d.p, u, o);
-            else if (q->et == GF_HEX8)
-                k_grad_3d_lds<T, M><<<nblocks(n, 128), 128, grad_lds_bytes<3>(128, q->nip, 3, sz), s>>>(n, q->nip, g,
-                                                                                                        u, o);
+            // the geometry is recomputed from the coordinates, except for Hex8 in FP32, where the FP64
+            // recomputation (some 430 FP64 operations per point) takes as long as 768 bytes per element
+            // of stored FP32 geometry do (395 k elements: 85 against 80 us), and a Hex8 rule of one
+            // point, whose workgroups span too many elements for LDS
+            if (q->et == GF_HEX8) {
+                if constexpr (std::is_same_v<T, double>) {
+                    if (grad3x_lds_bytes(q->nip, sz) <= 65536) {
+                        k_grad_3d_x<T, M><<<nblocks(n, QB3), QB3, grad3x_lds_bytes(q->nip, sz), s>>>(
+                            n, q->nip, q->x.p, q->dNxi_d.p, u, o);
+                        return;
+                    }
+                }
+                k_grad_3d_lds<T, M><<<nblocks(n, 128), 128, grad3_lds_bytes(128, q->nip, sz), s>>>(
+                    n, q->nip, geometry(tag), u, o);
+            }
             else if (q->et == GF_QUAD4_PLANAR)
-                k_grad_2d_lds<T, 3, M><<<nblocks(n, 256), 256, grad_lds_bytes<2>(256, q->nip, 3, sz), s>>>(n, q->nip,
-                                                                                                           g, u, o);
+                k_grad_2d_x<T, 3, M><<<nblocks(n, 256), 256, grad2x_lds_bytes(q->nip, 3, sz), s>>>(n, q->nip, q->x.p,
+                                                                                                   q->dNxi_d.p, u, o);
             else
-                k_grad_2d_lds<T, 2, M><<<nblocks(n, 256), 256, grad_lds_bytes<2>(256, q->nip, 2, sz), s>>>(n, q->nip,
-                                                                                                           g, u, o);
+                k_grad_2d_x<T, 2, M><<<nblocks(n, 256), 256, grad2x_lds_bytes(q->nip, 2, sz), s>>>(n, q->nip, q->x.p,
+                                                                                                   q->dNxi_d.p, u, o);
         };
-        auto by_mode = [&](auto tag, const auto* u, auto* o, const auto* g) {
-            if (mode == 0) launch(tag, std::integral_constant<int, 0>(), u, o, g);
-            else if (mode == 1) launch(tag, std::integral_constant<int, 1>(), u, o, g);
-            else launch(tag, std::integral_constant<int, 2>(), u, o, g);
+        auto by_mode = [&](auto tag, const auto* u, auto* o) {
+            if (mode == 0) launch(tag, std::integral_constant<int, 0>(), u, o);
+            else if (mode == 1) launch(tag, std::integral_constant<int, 1>(), u, o);
+            else launch(tag, std::integral_constant<int, 2>(), u, o);
         };
-        if (dtype == GF_F64)
-            by_mode(double(0), static_cast<const double*>(elemvec), static_cast<double*>(qtensor), q->dNx.p);
-        else {
-            ensure32(q, s);
-            by_mode(float(0), static_cast<const float*>(elemvec), static_cast<float*>(qtensor), q->dNx32.p);
-        }
+        if (dtype == GF_F64) by_mode(double(0), static_cast<const double*>(elemvec), static_cast<double*>(qtensor));
+        else by_mode(float(0), static_cast<const float*>(elemvec), static_cast<float*>(qtensor));
         check_launch();
     });
 }
@@ -981,35 +1127,55 @@ int gf_quad_int_gradN_dot_tensor2_dV(gf_quad q, const void* qtensor, void* elemv
         const int64_t E = q->nelem;
         if (E == 0) return;
         hipStream_t s = S(stream);
-        auto launch = [&](auto tag, const auto* in, auto* o, const auto* g, const auto* v) {
+        auto launch = [&](auto tag, const auto* in, auto* o) {
             using T = decltype(tag);
-            // rules with many points (LDS need above 64 KiB): the unstaged kernel, thread per (e, m)
-            const size_t need = q->et == GF_HEX8 ? int2_lds_bytes<T, 8, 3, 3, 16>(q->nip)
-                                                 : int2_lds_bytes<T, 4, 2, 3, 64>(q->nip);
-            if (need > 65536) {
+            const size_t sz = sizeof(T);
+            const int nip = q->nip;
+            // rules of more points than a workgroup has threads, or whose points' LDS outgrows 64 KiB: the
+            // unstaged kernel with the stored geometry, thread per (e, m)
+            const bool staged = q->et == GF_HEX8 ? nip <= PB3 && int2_h8_lds_bytes(nip, sz) <= 65536
+                                                 : nip <= PB2 && int2_q4_lds_bytes(nip, 3, sz) <= 65536;
+            if (!staged) {
+                const T *g, *v;
+                if constexpr (std::is_same_v<T, float>) {
+                    ensure32(q, s);
+                    g = q->dNx32.p;
+                    v = q->vol32.p;
+                }
+                else {
+                    g = q->dNx.p;
+                    v = q->vol.p;
+                }
                 const int64_t n = E * q->nne;
-                if (q->et == GF_HEX8) k_int_tensor2<T, 3, 3><<<nblocks(n, BS), BS, 0, s>>>(n, q->nip, q->nne, g, v, in, o);
+                if (q->et == GF_HEX8) k_int_tensor2<T, 3, 3><<<nblocks(n, BS), BS, 0, s>>>(n, nip, q->nne, g, v, in, o);
                 else if (q->et == GF_QUAD4_PLANAR)
-                    k_int_tensor2<T, 2, 3><<<nblocks(n, BS), BS, 0, s>>>(n, q->nip, q->nne, g, v, in, o);
-                else k_int_tensor2<T, 2, 2><<<nblocks(n, BS), BS, 0, s>>>(n, q->nip, q->nne, g, v, in, o);
+                    k_int_tensor2<T, 2, 3><<<nblocks(n, BS), BS, 0, s>>>(n, nip, q->nne, g, v, in, o);
+                else k_int_tensor2<T, 2, 2><<<nblocks(n, BS), BS, 0, s>>>(n, nip, q->nne, g, v, in, o);
                 return;
             }
-            if (q->et == GF_HEX8)
-                k_int_tensor2_lds<T, 8, 3, 3, 16><<<nblocks(E, 16), 128, int2_lds_bytes<T, 8, 3, 3, 16>(q->nip), s>>>(
-                    E, q->nip, g, v, in, o);
+            if (q->et == GF_HEX8) {
+                const T *gx, *gv;
+                if constexpr (std::is_same_v<T, float>) {
+                    ensure32(q, s);
+                    gx = q->dNx32.p;
+                    gv = q->vol32.p;
+                }
+                else {
+                    gx = q->x.p;
+                    gv = q->w_d.p;
+                }
+                k_int_tensor2_h8<T><<<nblocks(E, PB3 / nip), PB3, int2_h8_lds_bytes(nip, sz), s>>>(
+                    E, nip, gx, q->dNxi_d.p, gv, in, o);
+            }
             else if (q->et == GF_QUAD4_PLANAR)
-                k_int_tensor2_lds<T, 4, 2, 3, 64><<<nblocks(E, 64), 256, int2_lds_bytes<T, 4, 2, 3, 64>(q->nip), s>>>(
-                    E, q->nip, g, v, in, o);
+                k_int_tensor2_q4<T, 3><<<nblocks(E, PB2 / nip), PB2, int2_q4_lds_bytes(nip, 3, sz), s>>>(
+                    E, nip, 1, q->thick, q->x.p, q->dNxi_d.p, q->w_d.p, in, o);
             else
-                k_int_tensor2_lds<T, 4, 2, 2, 64><<<nblocks(E, 64), 256, int2_lds_bytes<T, 4, 2, 2, 64>(q->nip), s>>>(
-                    E, q->nip, g, v, in, o);
+                k_int_tensor2_q4<T, 2><<<nblocks(E, PB2 / nip), PB2, int2_q4_lds_bytes(nip, 2, sz), s>>>(
+                    E, nip, 0, q->thick, q->x.p, q->dNxi_d.p, q->w_d.p, in, o);
         };
-        if (dtype == GF_F64)
-            launch(double(0), static_cast<const double*>(qtensor), static_cast<double*>(elemvec), q->dNx.p, q->vol.p);
-        else {
-            ensure32(q, s);
-            launch(float(0), static_cast<const float*>(qtensor), static_cast<float*>(elemvec), q->dNx32.p, q->vol32.p);
-        }
+        if (dtype == GF_F64) launch(double(0), static_cast<const double*>(qtensor), static_cast<double*>(elemvec));
+        else launch(float(0), static_cast<const float*>(qtensor), static_cast<float*>(elemvec));
         check_launch();
     });
 }
