@@ -98,6 +98,44 @@ struct ShapeTable {
 constexpr int BS = 256;
 
 // ---- per-element force, FP64 in the reference's expression order ------------------------------
+// The contributions c[m][i] of one Gauss point to the element's nodal forces; g = dN/dxi [4][2] and w the
+// weight of the point
+__device__ inline void element_point_f64(const double (*g)[2], double w, const double x[4][2], const double u[4][2],
+                                         double k, double gmod, double c[4][2])
+{
+    double J00 = g[0][0] * x[0][0] + g[1][0] * x[1][0] + g[2][0] * x[2][0] + g[3][0] * x[3][0];
+    double J01 = g[0][0] * x[0][1] + g[1][0] * x[1][1] + g[2][0] * x[2][1] + g[3][0] * x[3][1];
+    double J10 = g[0][1] * x[0][0] + g[1][1] * x[1][0] + g[2][1] * x[2][0] + g[3][1] * x[3][0];
+    double J11 = g[0][1] * x[0][1] + g[1][1] * x[1][1] + g[2][1] * x[2][1] + g[3][1] * x[3][1];
+    double det = J00 * J11 - J01 * J10;
+    double I00 = J11 / det, I01 = -1.0 * J01 / det, I10 = -1.0 * J10 / det, I11 = J00 / det;
+    double d[4][2];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        d[m][0] = I00 * g[m][0] + I01 * g[m][1];
+        d[m][1] = I10 * g[m][0] + I11 * g[m][1];
+    }
+    double vol = w * det * 1.0;
+    // SymGradN_vector, ElementQuad4Planar.h:191-221
+    double e00 = d[0][0] * u[0][0] + d[1][0] * u[1][0] + d[2][0] * u[2][0] + d[3][0] * u[3][0];
+    double e11 = d[0][1] * u[0][1] + d[1][1] * u[1][1] + d[2][1] * u[2][1] + d[3][1] * u[3][1];
+    double e01 = 0.5 * (d[0][0] * u[0][1] + d[1][0] * u[1][1] + d[2][0] * u[2][1] + d[3][0] * u[3][1] +
+                        d[0][1] * u[0][0] + d[1][1] * u[1][0] + d[2][1] * u[2][0] + d[3][1] * u[3][0]);
+    double e22 = 0.0;
+    // linear elastic law (tdim 3, plane strain)
+    double tr = e00 + e11 + e22;
+    double s00 = k * tr + 2.0 * gmod * (e00 - tr / 3.0);
+    double s11 = k * tr + 2.0 * gmod * (e11 - tr / 3.0);
+    double s01 = 2.0 * gmod * e01;
+    double s10 = 2.0 * gmod * e01;
+    // Int_gradN_dot_tensor2_dV, ElementQuad4Planar.h:253-278
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        c[m][0] = (d[m][0] * s00 + d[m][1] * s10) * vol;
+        c[m][1] = (d[m][0] * s01 + d[m][1] * s11) * vol;
+    }
+}
+
 __device__ inline void element_force_f64(const ShapeTable& T, const double x[4][2], const double u[4][2],
                                          double k, double gmod, double f[4][2])
 {
@@ -105,37 +143,12 @@ __device__ inline void element_force_f64(const ShapeTable& T, const double x[4][
     for (int m = 0; m < 4; ++m) f[m][0] = f[m][1] = 0.0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const double(*g)[2] = T.g[q];
-        double J00 = g[0][0] * x[0][0] + g[1][0] * x[1][0] + g[2][0] * x[2][0] + g[3][0] * x[3][0];
-        double J01 = g[0][0] * x[0][1] + g[1][0] * x[1][1] + g[2][0] * x[2][1] + g[3][0] * x[3][1];
-        double J10 = g[0][1] * x[0][0] + g[1][1] * x[1][0] + g[2][1] * x[2][0] + g[3][1] * x[3][0];
-        double J11 = g[0][1] * x[0][1] + g[1][1] * x[1][1] + g[2][1] * x[2][1] + g[3][1] * x[3][1];
-        double det = J00 * J11 - J01 * J10;
-        double I00 = J11 / det, I01 = -1.0 * J01 / det, I10 = -1.0 * J10 / det, I11 = J00 / det;
-        double d[4][2];
+        double c[4][2];
+        element_point_f64(T.g[q], T.w[q], x, u, k, gmod, c);
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-            d[m][0] = I00 * g[m][0] + I01 * g[m][1];
-            d[m][1] = I10 * g[m][0] + I11 * g[m][1];
-        }
-        double vol = T.w[q] * det * 1.0;
-        // SymGradN_vector, ElementQuad4Planar.h:191-221
-        double e00 = d[0][0] * u[0][0] + d[1][0] * u[1][0] + d[2][0] * u[2][0] + d[3][0] * u[3][0];
-        double e11 = d[0][1] * u[0][1] + d[1][1] * u[1][1] + d[2][1] * u[2][1] + d[3][1] * u[3][1];
-        double e01 = 0.5 * (d[0][0] * u[0][1] + d[1][0] * u[1][1] + d[2][0] * u[2][1] + d[3][0] * u[3][1] +
-                            d[0][1] * u[0][0] + d[1][1] * u[1][0] + d[2][1] * u[2][0] + d[3][1] * u[3][0]);
-        double e22 = 0.0;
-        // linear elastic law (tdim 3, plane strain)
-        double tr = e00 + e11 + e22;
-        double s00 = k * tr + 2.0 * gmod * (e00 - tr / 3.0);
-        double s11 = k * tr + 2.0 * gmod * (e11 - tr / 3.0);
-        double s01 = 2.0 * gmod * e01;
-        double s10 = 2.0 * gmod * e01;
-        // Int_gradN_dot_tensor2_dV, ElementQuad4Planar.h:253-278
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            f[m][0] += (d[m][0] * s00 + d[m][1] * s10) * vol;
-            f[m][1] += (d[m][0] * s01 + d[m][1] * s11) * vol;
+            f[m][0] += c[m][0];
+            f[m][1] += c[m][1];
         }
     }
 }
@@ -458,6 +471,121 @@ __global__ void __launch_bounds__(TX * TY) k_vv_structured(
         reinterpret_cast<double2*>(a1)[on] = an;
         if (fint_out) reinterpret_cast<double2*>(fint_out)[on] = make_double2(f0, f1);
     }
+}
+
+// The reference-order FP64 step on small grids: four lanes per element, one Gauss point each (an element's
+// four points are a serial chain of some 750 FP64 operations in the kernel above, and a small grid has too
+// few wavefronts to hide it), whose contributions each node adds in point order, then in element order: the
+// same sums, so the same bits.  A workgroup owns SX x SY nodes, and its 16 x 4 elements are one pass of its
+// 256 threads; thread t < 17 x 5 also carries node t of the halo tile through the update.
+// Bound: the latency of one launch.  Per step: 5.4 us from 40 x 40 to 128 x 128 elements (8.2 to 12.3 us with
+// one thread per element), 6.3 us at 200 x 200 (8.5), 9.2 us at 300 x 300 (10.1); at 400 x 400 the 1.4 times
+// redundant elements cost more than the latency (13.3 us against 12.1), so larger grids keep the kernel above.
+constexpr int SX = 15, SY = 3;
+constexpr int SPLIT_TILES = 2500; // 325 x 325 elements
+
+__global__ void __launch_bounds__(256) k_vv_split(
+    int nx, int ny, int ntx, int ntiles, int per_xcd, ShapeTable T, const double* __restrict__ coor, double sx, double sy,
+    const float* __restrict__ Ke, float Kconst, const float* __restrict__ Ge, const double* __restrict__ inv_mass,
+    const uint8_t* __restrict__ im_code, const double* __restrict__ im_tab, const double* __restrict__ fext, double dt,
+    double c, double hdt, const double2* __restrict__ u0, const double2* __restrict__ v0, const double2* __restrict__ a0,
+    double2* __restrict__ u1, double2* __restrict__ v1, double2* __restrict__ a1, double2* __restrict__ fint_out)
+{
+    constexpr int HX = SX + 2, HY = SY + 2, EX = SX + 1, EY = SY + 1, ROW = 9; // ROW: LDS pitch of a point
+    static_assert(EX * EY * 4 == 256 && HX * HY <= 256, "one pass of the workgroup");
+    __shared__ double2 s_u[HX * HY], s_x[HX * HY];
+    __shared__ double s_c[256 * ROW];
+    __shared__ double s_g[4][4][2];
+    const int b = blockIdx.x;
+    const int tile = (b & 7) * per_xcd + (b >> 3); // XCD-aware, as above
+    if (tile >= ntiles) return; // uniform for the whole block
+    const int ty = tile / ntx, tx = tile - ty * ntx;
+    const int x0 = tx * SX, y0 = ty * SY;
+    const int NX = nx + 1, NY = ny + 1;
+    const int t = threadIdx.x;
+    const int lx = t % HX, ly = t / HX;
+    const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
+    const bool node = t < HX * HY && gx >= 0 && gx < NX && gy >= 0 && gy < NY;
+    const bool owner = node && lx >= 1 && lx <= SX && ly >= 1 && ly <= SY;
+    const int64_t n = node ? static_cast<int64_t>(gy) * NX + gx : 0;
+    // the element of this thread's Gauss point
+    const int el = t / 4, q = t % 4, elx = el % EX, ely = el / EX;
+    const int ex = x0 - 1 + elx, ey = y0 - 1 + ely;
+    const bool elem = ex >= 0 && ex < nx && ey >= 0 && ey < ny;
+    const int64_t e = elem ? static_cast<int64_t>(ey) * nx + ex : 0;
+    const double k = static_cast<double>(Ke ? Ke[e] : Kconst), gmod = static_cast<double>(Ge[e]);
+    if (t < 32) (&s_g[0][0][0])[t] = (&T.g[0][0][0])[t];
+    double2 v = make_double2(0.0, 0.0), a = v, un = v, im = v, fe = v;
+    if (node) {
+        const double2 u = u0[n];
+        v = v0[n];
+        a = a0[n];
+        s_x[t] = coor ? reinterpret_cast<const double2*>(coor)[n]
+                      : make_double2(static_cast<double>(gx) * sx, static_cast<double>(gy) * sy);
+        un.x = u.x + dt * v.x + c * a.x;
+        un.y = u.y + dt * v.y + c * a.y;
+        s_u[t] = un;
+    }
+    if (owner) {
+        if (im_code) {
+            const uchar2 code = reinterpret_cast<const uchar2*>(im_code)[n];
+            im = make_double2(im_tab[code.x], im_tab[code.y]);
+        }
+        else
+            im = reinterpret_cast<const double2*>(inv_mass)[n];
+        if (fext) fe = reinterpret_cast<const double2*>(fext)[n];
+    }
+    __syncthreads();
+    if (elem) {
+        const int n0 = ely * HX + elx, nid[4] = {n0, n0 + 1, n0 + HX + 1, n0 + HX};
+        double x[4][2], u[4][2], g[4][2], p[4][2];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const double2 xx = s_x[nid[m]], uu = s_u[nid[m]];
+            x[m][0] = xx.x;
+            x[m][1] = xx.y;
+            u[m][0] = uu.x;
+            u[m][1] = uu.y;
+            g[m][0] = s_g[q][m][0];
+            g[m][1] = s_g[q][m][1];
+        }
+        element_point_f64(g, T.w[0], x, u, k, gmod, p); // the Gauss weights are equal
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            s_c[t * ROW + 2 * m] = p[m][0];
+            s_c[t * ROW + 2 * m + 1] = p[m][1];
+        }
+    }
+    __syncthreads();
+    if (!owner) return;
+    // elements in ascending number: (gx-1, gy-1) node 2, (gx, gy-1) node 3, (gx-1, gy) node 1, (gx, gy) node 0
+    const bool hasL = gx > 0, hasR = gx < nx, hasB = gy > 0, hasT = gy < ny;
+    const bool has[4] = {hasB && hasL, hasB && hasR, hasT && hasL, hasT && hasR};
+    constexpr int LN[4] = {2, 3, 1, 0};
+    double f0 = 0.0, f1 = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const double* p = s_c + ((ly - 1 + j / 2) * EX + lx - 1 + j % 2) * 4 * ROW + 2 * LN[j];
+        double g0 = 0.0, g1 = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            g0 += p[i * ROW];
+            g1 += p[i * ROW + 1];
+        }
+        if (has[j]) {
+            f0 += g0;
+            f1 += g1;
+        }
+    }
+    double2 an, vn;
+    an.x = im.x * (fe.x - f0);
+    an.y = im.y * (fe.y - f1);
+    vn.x = v.x + hdt * (a.x + an.x);
+    vn.y = v.y + hdt * (a.y + an.y);
+    u1[n] = un;
+    v1[n] = vn;
+    a1[n] = an;
+    if (fint_out) fint_out[n] = make_double2(f0, f1);
 }
 
 // ---- general path --------------------------------------------------------------------------------
@@ -795,18 +923,23 @@ struct TileCfg {
 };
 
 // Node tile per workgroup (measured on MI355X at 2048^2): the closed-form rectangle bodies 64 x 8,
-// the FP32 algebraic body 32 x 16, the FP64 bodies 32 x 8.  GF_EXPLICIT_TILE=<tx>x<ty> overrides.
-TileCfg tile_config(int body)
+// the FP32 algebraic body 32 x 16, the FP64 bodies 32 x 8 (small grids in reference-order FP64: k_vv_split).  GF_EXPLICIT_TILE=<tx>x<ty> overrides.
+TileCfg tile_override()
 {
     static const TileCfg over = [] {
         TileCfg c{0, 0};
         if (const char* e = std::getenv("GF_EXPLICIT_TILE")) {
             int a = 0, b = 0;
-            if (std::sscanf(e, "%dx%d", &a, &b) == 2) c = TileCfg{a, b};
+            if (std::sscanf(e, "%dx%d", &a, &b) == 2 && a > 0) c = TileCfg{a, b};
         }
         return c;
     }();
-    if (over.tx > 0) return over;
+    return over;
+}
+
+TileCfg tile_config(int body)
+{
+    if (tile_override().tx > 0) return tile_override();
     switch (body) {
         case B_F32_RECT:
         case B_F64_RECT: return TileCfg{64, 8};
@@ -850,12 +983,17 @@ void launch_structured(int body, unsigned grid, hipStream_t s, int nx, int ny, i
 // Node blocks of the fused general step (k_explicit_blocks).  Used when every DOF belongs to
 // exactly one (node, component) -- a bijection onto [0, ndof) -- so that a DOF's contributions are
 // those of one node; tied meshes keep the element kernel + per-DOF gather.  The blocks come from a
-// recursive coordinate bisection of the nodes: a set is split across its longer extent with a
-// multiple of BS nodes on the lower side, until it holds at most BS, so every block is a compact
-// patch of BS nodes (one block may hold fewer).  Each block's nodes are then put in ascending
+// recursive coordinate bisection of the nodes: a set is split across its longer extent in proportion to
+// the numbers of blocks on either side, so every block is a compact patch of about PATCH nodes.  208
+// nodes touch about 250 elements, so that the element phase is one pass of the 256 threads; patches of
+// 256 nodes touch 290 and leave three of four waves waiting for a second pass (0.49 M elements: 345
+// instead of 369 us per 20 steps in FP32, 557 instead of 572 in reference-order FP64; 11 k elements 117
+// instead of 135 and 163 instead of 185).  Each block's nodes are then put in ascending
 // number so that neighbouring threads touch neighbouring DOFs.  rank[e]: position of original
 // element e in the locality order; cp, kp, gp: connectivity [4] and moduli in that order.  Blocks
 // whose local nodes and element forces would not fit in 64 KiB of LDS keep the two-kernel path.
+constexpr int64_t PATCH = 208;
+
 void build_node_blocks(gf_explicit_s* x, gf_vector v, const double* coor_d, const std::vector<int32_t>& rank,
                        const std::vector<int32_t>& cp, const std::vector<float>& kp, const std::vector<float>& gp)
 {
@@ -874,12 +1012,19 @@ void build_node_blocks(gf_explicit_s* x, gf_vector v, const double* coor_d, cons
     std::vector<int32_t> node(nn);
     for (int64_t n = 0; n < nn; ++n) node[n] = static_cast<int32_t>(n);
     // recursive coordinate bisection, iteratively over a stack of node ranges
-    std::vector<std::pair<int64_t, int64_t>> todo{{0, nn}};
+    struct Part {
+        int64_t b, e, np; // a node range and the number of blocks it is cut into
+    };
+    std::vector<Part> todo{{0, nn, (nn + PATCH - 1) / PATCH}};
+    std::vector<std::pair<int64_t, int64_t>> leaf;
     while (!todo.empty()) {
-        const auto [b, e] = todo.back();
+        const auto [b, e, np] = todo.back();
         todo.pop_back();
         const int64_t n = e - b;
-        if (n <= BS) continue;
+        if (np <= 1) {
+            leaf.push_back({b, e});
+            continue;
+        }
         double l[2] = {xy[2 * node[b]], xy[2 * node[b] + 1]}, h[2] = {l[0], l[1]};
         for (int64_t k = b; k < e; ++k)
             for (int i = 0; i < 2; ++i) {
@@ -887,13 +1032,13 @@ void build_node_blocks(gf_explicit_s* x, gf_vector v, const double* coor_d, cons
                 h[i] = std::max(h[i], xy[2 * node[k] + i]);
             }
         const int dim = (h[0] - l[0] >= h[1] - l[1]) ? 0 : 1;
-        const int64_t lower = std::max<int64_t>(BS, ((n + BS) / (2 * BS)) * BS); // a multiple of BS, < n
+        const int64_t npl = np / 2, lower = n * npl / np;
         std::nth_element(node.begin() + b, node.begin() + b + lower, node.begin() + e, [&](int32_t p, int32_t q) {
             const double xp = xy[2 * p + dim], xq = xy[2 * q + dim];
             return xp < xq || (xp == xq && p < q);
         });
-        todo.push_back({b, b + lower});
-        todo.push_back({b + lower, e});
+        todo.push_back({b + lower, e, np - npl});
+        todo.push_back({b, b + lower, npl});
     }
     // (e, m) of every node, e ascending then m: the reference's scatter order for each component
     std::vector<int64_t> nptr(nn + 1, 0);
@@ -975,8 +1120,8 @@ void build_node_blocks(gf_explicit_s* x, gf_vector v, const double* coor_d, cons
         for (int32_t n : halo) lidx[n] = -1;
         return true;
     };
-    for (int64_t k0 = 0; k0 < nn; k0 += BS)
-        if (!emit(k0, std::min(nn, k0 + BS))) return;
+    for (const auto& [k0, k1] : leaf)
+        if (!emit(k0, k1)) return;
     x->bkptr.upload(bkptr);
     x->blptr.upload(blptr);
     x->bnloc.upload(bnloc);
@@ -1206,10 +1351,19 @@ int gf_explicit_step(gf_explicit x, int64_t nsteps, int precision, int store_fin
             const int ntx = (nx + 1 + TXr - 1) / TXr, nty = (ny + 1 + TYr - 1) / TYr;
             const int ntiles = ntx * nty, per_xcd = (ntiles + 7) / 8;
             const unsigned grid = static_cast<unsigned>(per_xcd * 8);
+            const int stx = (nx + SX) / SX, stiles = stx * ((ny + SY) / SY), sper = (stiles + 7) / 8;
+            const bool split = body == B_REF64 && stiles <= SPLIT_TILES && !tile_override().tx;
             for (int64_t k = 0; k < nsteps; ++k) {
                 const int i0 = x->cur, i1 = 1 - x->cur;
                 double* fo = (store_fint && k == nsteps - 1) ? x->fint.p : nullptr;
-                if (TXr == 32 && TYr == 8)
+                auto d2 = [](double* p) { return reinterpret_cast<double2*>(p); };
+                if (split)
+                    k_vv_split<<<8 * sper, 256, 0, s>>>(
+                        nx, ny, stx, stiles, sper, T, x->reg_x ? nullptr : x->coor.p, x->sx, x->sy,
+                        x->k_uniform ? nullptr : x->Ke.p, x->k_value, x->Ge.p, x->inv_mass.p,
+                        x->im_code.n ? x->im_code.p : nullptr, x->im_tab.p, fext, dt, c, hdt, d2(x->u[i0].p),
+                        d2(x->vv[i0].p), d2(x->a[i0].p), d2(x->u[i1].p), d2(x->vv[i1].p), d2(x->a[i1].p), d2(fo));
+                else if (TXr == 32 && TYr == 8)
                     launch_structured<32, 8>(body, grid, s, nx, ny, ntx, nty, per_xcd, T, x, fext, dt, c, hdt, i0, i1, fo);
                 else if (TXr == 64 && TYr == 8)
                     launch_structured<64, 8>(body, grid, s, nx, ny, ntx, nty, per_xcd, T, x, fext, dt, c, hdt, i0, i1, fo);
