@@ -13,8 +13,10 @@
 // each MFMA lane evaluates the T entries it feeds, the 15 MFMAs accumulate the 32 x 32 tile, and the
 // 24 x 24 result is stored straight from the accumulators as contiguous FP64 rows.
 //
-// GF_F64: the same per-entry accumulation order as the reference loop (q, i, l for each (j, k)),
-// with one wavefront per element reading C and dNx from LDS (each thread owns one (m, n) block).
+// GF_F64: the same per-entry accumulation order as the reference loop (q, i, l for each (j, k)) on the
+// vector units, four elements per wavefront (k_stiffness_f64).
+#include <type_traits>
+
 #include "gf_internal.hpp"
 
 using namespace gf;
@@ -257,38 +259,81 @@ __global__ void __launch_bounds__(64 * WAVES) k_stiffness_bf16x3(int64_t nelem, 
     }
 }
 
-// FP64 in reference order, one wavefront per element, C and dNx from LDS.  STREAM: the element
-// matrix goes through the wave's C area in LDS and leaves as one contiguous 16-byte stream
-// (elemmat 16-byte aligned) instead of nine strided scalar stores per lane.
-template <bool STREAM>
+// FP64 in reference order: acc(j, k) += ((dNx(m,i) C(i,j,k,l)) dNx(n,l)) dV over q, i, l.  8 GRP lanes
+// per element, 8 / GRP elements per wave: a lane owns node m and 8 / GRP column nodes, so one product
+// dNx(m,i) C(i,j,k,l) and one LDS read of C serve 8 / GRP of its blocks, and the same read serves the
+// wave's elements.  The tangent and gradients of a point go to registers one point ahead and from there
+// to LDS.  Bound by FP64 issue: the order allows no FMA and no regrouping, so an entry costs three
+// operations a term plus its share of the first product (3.25 with GRP 2, 3.5 with GRP 4, 4 with GRP 8).
+// At 82,861 elements: 395 us (GRP 2; the vector units issue in 83% of its cycles), 414 (GRP 4), 473
+// (GRP 8); 507 us for a whole element staged per wave with every lane forming all four operations.
+constexpr int SG = 82;      // offset of a point's gradients behind its 81 tangent entries
+constexpr int SP = SG + 24; // LDS pitch of an element (its 16-byte reads hit disjoint banks)
+
+template <int LPE> // lanes per element
+struct PointStage {
+    static constexpr int R = (81 + 24 + LPE - 1) / LPE;
+    double r[R];
+    double v;
+    // point q of element e for lane l of LPE: 81 tangent entries, then the 24 gradients
+    __device__ void load(const double* __restrict__ C, const double* __restrict__ dNx, const double* __restrict__ vol,
+                         int64_t e, int q, int l)
+    {
+        const double* c = C + e * NC + q * 81;
+        const double* g = dNx + e * NG + q * 24;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int t = l + LPE * k;
+            r[k] = t < 81 ? c[t] : g[min(t - 81, 23)];
+        }
+        v = vol[e * NQ + q];
+    }
+    __device__ void store(double* dst, int l) const
+    {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int t = l + LPE * k;
+            if (t < 105) dst[t + (t >= 81)] = r[k];
+        }
+    }
+};
+
+// STREAM: each element matrix leaves through LDS as one contiguous 16-byte stream (elemmat 16-byte
+// aligned) instead of scalar stores.
+template <int GRP, bool STREAM>
 __global__ void __launch_bounds__(64 * WAVES) k_stiffness_f64(int64_t nelem, const double* __restrict__ C,
                                                                const double* __restrict__ dNx,
                                                                const double* __restrict__ vol,
                                                                double* __restrict__ elemmat)
 {
-    static_assert(NC >= 576, "the element matrix must fit the C area");
-    __shared__ __align__(16) double sC[WAVES][NC];
-    __shared__ double sg[WAVES][NG];
-    __shared__ double sv[WAVES][NQ];
+    constexpr int LPE = 8 * GRP, EPW = 64 / LPE, NB = 8 / GRP;
+    static_assert(EPW * SP <= 576, "the staged points must fit the element matrix");
+    __shared__ __align__(16) double lds[WAVES][576];
     const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int m = lane / 8, n = lane % 8;
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * WAVES;
-    for (int64_t e = static_cast<int64_t>(blockIdx.x) * WAVES + w; e < nelem; e += stride) {
-        for (int t = lane; t < NC; t += 64) sC[w][t] = C[e * NC + t];
-        for (int t = lane; t < NG; t += 64) sg[w][t] = dNx[e * NG + t];
-        if (lane < NQ) sv[w][lane] = vol[e * NQ + lane];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        double acc[3][3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) acc[j][k] = 0.0;
+    const int s = lane / LPE, l = lane % LPE, m = l / GRP, n0 = NB * (l % GRP);
+    double* sh = lds[w];
+    double* se = sh + s * SP;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * WAVES * EPW;
+    int64_t e0 = (static_cast<int64_t>(blockIdx.x) * WAVES + w) * EPW;
+    if (e0 >= nelem) return; // uniform per wave; the kernel has no workgroup barrier
+    PointStage<LPE> st;
+    st.load(C, dNx, vol, min(e0 + s, nelem - 1), 0, l);
+    for (; e0 < nelem; e0 += stride) {
+        const int64_t ec = min(e0 + s, nelem - 1), en = min(e0 + stride + s, nelem - 1);
+        double acc[NB][3][3] = {};
+#pragma unroll 1
         for (int q = 0; q < NQ; ++q) {
-            const double* g = sg[w] + q * 24;
-            const double* Cq = sC[w] + q * 81;
-            const double v = sv[w][q];
+            st.store(se, l);
+            const double v = st.v;
+            wave_sync();
+            st.load(C, dNx, vol, q + 1 < NQ ? ec : en, q + 1 < NQ ? q + 1 : 0, l);
+            double gm[3], gn[NB][3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) gm[i] = se[SG + 3 * m + i];
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) gn[n][i] = se[SG + 3 * (n0 + n) + i];
 #pragma unroll
             for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -296,34 +341,44 @@ __global__ void __launch_bounds__(64 * WAVES) k_stiffness_f64(int64_t nelem, con
 #pragma unroll
                     for (int k = 0; k < 3; ++k)
 #pragma unroll
-                        for (int l = 0; l < 3; ++l)
-                            acc[j][k] += g[m * 3 + i] * Cq[((i * 3 + j) * 3 + k) * 3 + l] * g[n * 3 + l] * v;
+                        for (int d = 0; d < 3; ++d) {
+                            const double gc = gm[i] * se[((i * 3 + j) * 3 + k) * 3 + d];
+#pragma unroll
+                            for (int n = 0; n < NB; ++n) acc[n][j][k] += gc * gn[n][d] * v;
+                        }
+            wave_sync(); // every lane is done reading the point
         }
-        double* Ke = elemmat + e * 576;
         if constexpr (STREAM) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); // every lane is done reading C
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 1
+            for (int t = 0; t < EPW; ++t) {
+                if (e0 + t >= nelem) break; // uniform per wave
+                if (s == t) {
+#pragma unroll
+                    for (int j = 0; j < 3; ++j)
+#pragma unroll
+                        for (int n = 0; n < NB; ++n)
+#pragma unroll
+                            for (int k = 0; k < 3; ++k) sh[(m * 3 + j) * 24 + (n0 + n) * 3 + k] = acc[n][j][k];
+                }
+                wave_sync();
+                typedef double d2 __attribute__((ext_vector_type(2)));
+                d2* Ke = reinterpret_cast<d2*>(elemmat + (e0 + t) * 576);
+#pragma unroll
+                for (int r = 0; r < 5; ++r)
+                    if (r < 4 || lane < 32)
+                        __builtin_nontemporal_store(reinterpret_cast<const d2*>(sh)[lane + 64 * r], Ke + lane + 64 * r);
+                wave_sync();
+            }
+        }
+        else if (e0 + s < nelem) {
+            double* Ke = elemmat + (e0 + s) * 576;
 #pragma unroll
             for (int j = 0; j < 3; ++j)
 #pragma unroll
-                for (int k = 0; k < 3; ++k) sC[w][(m * 3 + j) * 24 + n * 3 + k] = acc[j][k];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            typedef double d2 __attribute__((ext_vector_type(2)));
-            for (int t = lane; t < 288; t += 64)
-                __builtin_nontemporal_store(reinterpret_cast<const d2*>(sC[w])[t], reinterpret_cast<d2*>(Ke) + t);
-        }
-        else {
+                for (int n = 0; n < NB; ++n)
 #pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int k = 0; k < 3; ++k) Ke[(m * 3 + j) * 24 + n * 3 + k] = acc[j][k];
+                    for (int k = 0; k < 3; ++k) Ke[(m * 3 + j) * 24 + (n0 + n) * 3 + k] = acc[n][j][k];
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 }
 
@@ -400,9 +455,16 @@ __global__ void __launch_bounds__(256) k_elemmat_dot_rows(int64_t nrows, const T
     }
 }
 
-unsigned grid_for(int64_t nelem)
+// Lanes per element of k_stiffness_f64: few lanes share most work, but a mesh has to fill the chip with
+// them.  Two groups (four elements a wave) from where they are about one full set of resident waves;
+// eight (one element a wave) up to where four groups would leave half of the SIMDs without one.  Times in
+// us with GRP 2 / 4 / 8: 512 elements 26.1 / 17.0 / 13.3; 2,548: 27.0 / 25.4 / 23.1; 6,120: 43.5 / 36.6 /
+// 40.3; 22,680: 113 / 114 / 130; 82,861: 397 / 414 / 473.
+constexpr int64_t F64_GRP2 = 16384, F64_GRP4 = 4096;
+
+unsigned grid_for(int64_t nelem, int per_wave = 1)
 {
-    int64_t g = (nelem + WAVES - 1) / WAVES;
+    int64_t g = (nelem + WAVES * per_wave - 1) / (WAVES * per_wave);
     return static_cast<unsigned>(std::min<int64_t>(g, 256 * 64));
 }
 
@@ -441,10 +503,14 @@ int stiffness_f64_hex8(gf_quad q, const double* C, double* elemmat, hipStream_t 
         GF_REQUIRE(quad_etype(q) == GF_HEX8 && quad_nip(q) == NQ, "Hex8 with 8 points");
         const int64_t ne = quad_nelem(q);
         if (ne == 0) return;
-        if (aligned16(elemmat))
-            k_stiffness_f64<true><<<grid_for(ne), 64 * WAVES, 0, s>>>(ne, C, quad_dNx(q), quad_vol(q), elemmat);
-        else
-            k_stiffness_f64<false><<<grid_for(ne), 64 * WAVES, 0, s>>>(ne, C, quad_dNx(q), quad_vol(q), elemmat);
+        auto run = [&](auto grp) {
+            constexpr int G = decltype(grp)::value;
+            auto kern = aligned16(elemmat) ? k_stiffness_f64<G, true> : k_stiffness_f64<G, false>;
+            kern<<<grid_for(ne, 8 / G), 64 * WAVES, 0, s>>>(ne, C, quad_dNx(q), quad_vol(q), elemmat);
+        };
+        if (ne >= F64_GRP2) run(std::integral_constant<int, 2>());
+        else if (ne >= F64_GRP4) run(std::integral_constant<int, 4>());
+        else run(std::integral_constant<int, 8>());
         check_launch();
     });
 }
