@@ -212,6 +212,7 @@ struct gf_vector_s {
     //   node-centric: elemvec entries (e*nne + m) with conn(e,m) == n (ascending)
     gf::DBuf<int32_t> node_eptr, node_eidx;
     bool one_node_per_dof = false; // dofs is a permutation of 0 .. nnode ndim - 1
+    bool identity = false;         // dofs(n, i) = n ndim + i
     // host copies (int64) for set-up code that builds derived structures
     std::vector<int64_t> conn_h, dofs_h;
 };

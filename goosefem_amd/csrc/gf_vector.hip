@@ -228,6 +228,9 @@ int gf_vector_create(gf_vector* out, const int64_t* conn_h, int64_t nelem, int n
             build_csr(v->dofs_h, v->ndof, ptr, idx);
             v->one_node_per_dof = v->ndof == nnode * ndim;
             for (int64_t d = 0; d < v->ndof && v->one_node_per_dof; ++d) v->one_node_per_dof = ptr[d + 1] - ptr[d] == 1;
+            v->identity = v->one_node_per_dof;
+            for (size_t k = 0; k < v->dofs_h.size() && v->identity; ++k)
+                v->identity = v->dofs_h[k] == static_cast<int64_t>(k);
             v->dof_nptr.upload(ptr);
             v->dof_nidx.upload(idx);
             // node <- (e, m)

@@ -453,7 +453,8 @@ int gf_matrix_dot_nodevec(gf_matrix A, const double* x, double* b, void* stream)
  * forbid hipMalloc).  The dofval staging of x and A x lives in a static device array of the
  * library, 2 x 2^20 doubles (16 MiB) per device: matrices above 2^20 rows fail with GF_EINVAL.
  * Calls that overlap on one GPU share that array and race; the stream must belong to the current
- * device.  Results are bit-identical to gf_matrix_dot_nodevec, which allocates and synchronises. */
+ * device.  Results are bit-identical to gf_matrix_dot_nodevec, which needs no staging and does not
+ * synchronise unless b overlaps x (then it allocates and synchronises). */
 int gf_matrix_dot_nodevec_noalloc(gf_matrix A, const double* x, double* b, void* stream);
 /* Todense()  (Matrix.h:338-355, :790-802): out [nrows, nrows] */
 int gf_matrix_todense(gf_matrix A, double* out, void* stream);
