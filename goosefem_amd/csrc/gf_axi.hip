@@ -6,8 +6,7 @@
 // 108) and dV = w J 2 pi r_q; the kernels that are bound by HBM form it again from the element's 64 bytes
 // of coordinates, with the function that made the stored one.  Every kernel keeps the reference's FP64
 // expression and summation order (no contraction), so results equal the reference's bit for bit.  The
-// stiffness runs the
-// 25 products of each node pair over the five non-zero slots a (outer) and b (inner), slot =
+// stiffness runs the 25 products of each node pair over the five non-zero slots a (outer) and b (inner), slot =
 // (i, j, value, nodal component): (r,r: dN/dr, u_r) (t,t: N/r, u_r) (z,z: dN/dz, u_z)
 // (r,z: dN/dr, u_z) (z,r: dN/dz, u_r), and K(m, c_a; n, c_b) += B_a(m) C(i_a, j_a, j_b, i_b) B_b(n) dV
 // (:298-398, in the listed order).
@@ -118,8 +117,6 @@ __global__ void __launch_bounds__(BS) k_axi_grad(int64_t nelem, AxiRule R, int m
     stage_out<double, BS>(out + 9 * e0 * R.nip, s_o, 9 * np);
 }
 
-// one thread per (element, node m, node n): the 2 x 2 block K(m *, n *) of the element matrix
-
 // int_N_scalar_NT_dV (:235-266)
 __global__ void k_axi_int_N(int64_t nelem, AxiRule R, const double* __restrict__ vol, const double* __restrict__ qs,
                             double* __restrict__ M)
@@ -184,30 +181,93 @@ __global__ void __launch_bounds__(BS) k_axi_int_t2(int64_t nelem, AxiRule R, con
     stage_out<double, BS>(f + 8 * e0, s_x, 8 * ne);
 }
 
-// int_gradN_dot_tensor4_dot_gradNT_dV (:298-398)
-__global__ void k_axi_int_t4(int64_t nelem, int nip, const double* __restrict__ G, const double* __restrict__ vol,
-                             const double* __restrict__ C, double* __restrict__ K)
+// int_gradN_dot_tensor4_dot_gradNT_dV (:298-398), one thread per (element, node m): per point the products
+// B_a(m) C are formed once and used for all four column nodes, in the listed order.  A workgroup owns 64
+// elements.  Four points at a time each thread forms the geometry of one of them; the 25 entries of a
+// point's tangents go to registers one point ahead and through LDS, and so do the rows of K_e, which leave
+// as one 16-byte stream (scalar stores if elemmat is not 16-byte aligned).  Bound by HBM: the tangents (all
+// of a 648-byte record's lines hold a used entry) and K_e.  225 k elements: 128 us, 285 us with one
+// thread per node pair reading its own tangent and storing its own 2 x 2 block.
+constexpr int T4_EB = 64, T4_KROW = 18, T4_NC = (25 * T4_EB + BS - 1) / BS;
+
+__global__ void __launch_bounds__(BS, 4) k_axi_int_t4(int64_t nelem, AxiRule R, const double* __restrict__ x,
+                                                   const double* __restrict__ C, double* __restrict__ K)
 {
-    const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (t >= nelem * 16) return;
-    const int64_t e = t / 16;
-    const int m = static_cast<int>(t % 16) / 4, n = static_cast<int>(t % 4);
+    static_assert(BS == 4 * T4_EB, "one thread per (element, node)");
     constexpr int si[5] = {0, 1, 2, 0, 2}, sj[5] = {0, 1, 2, 2, 0}, sv[5] = {0, 1, 2, 0, 2}, sc[5] = {1, 1, 0, 0, 1};
-    double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    for (int q = 0; q < nip; ++q) {
-        const double* bm = G + 12 * (e * nip + q) + 3 * m;
-        const double* bn = G + 12 * (e * nip + q) + 3 * n;
-        const double* c = C + 81 * (e * nip + q);
-        const double v = vol[e * nip + q];
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) double smem[T4_EB * (4 * 13 + 25)];
+    static_assert(T4_EB * (4 * 13 + 25) >= BS * T4_KROW, "the rows of K must fit");
+    double *s_g = smem, *s_c = smem + T4_EB * 4 * 13; // [element][point of four][G, dV], [element][25]
+    const int t = threadIdx.x, el = t / 4, m = t % 4, nip = R.nip;
+    const int64_t e0 = blockIdx.x * static_cast<int64_t>(T4_EB);
+    const int ne = static_cast<int>(min<int64_t>(T4_EB, nelem - e0));
+    // entry (a, b) of a tangent is its (i_a, j_a, j_b, i_b) component: both pairs at even positions of nine
+    const double* Cb = C + e0 * nip * 81;
+    int src[T4_NC];
 #pragma unroll
-        for (int a = 0; a < 5; ++a)
-#pragma unroll
-            for (int b = 0; b < 5; ++b)
-                acc[sc[a]][sc[b]] += bm[sv[a]] * c[((si[a] * 3 + sj[a]) * 3 + sj[b]) * 3 + si[b]] * bn[sv[b]] * v;
+    for (int k = 0; k < T4_NC; ++k) {
+        const int w = min(t + k * BS, 25 * ne - 1), r = w % 25, a = r / 5, b = r % 5;
+        const int ia = a < 3 ? 4 * a : a == 3 ? 2 : 6, jb = b < 3 ? 4 * b : b == 3 ? 6 : 2;
+        src[k] = (w / 25) * nip * 81 + 9 * ia + jb;
     }
-    double* Ke = K + 64 * e;
-    for (int i = 0; i < 2; ++i)
-        for (int j = 0; j < 2; ++j) Ke[(2 * m + i) * 8 + 2 * n + j] = acc[i][j];
+    double pre[T4_NC];
+#pragma unroll
+    for (int k = 0; k < T4_NC; ++k) pre[k] = Cb[src[k]];
+    double acc[4][2][2] = {};
+    for (int q0 = 0; q0 < nip; q0 += 4) {
+        if (q0 + m < nip) {
+            double o[12], v;
+            axi_point_geometry(R, q0 + m, x + 8 * (e0 + min(el, ne - 1)), o, v);
+            double* g = s_g + 13 * t;
+#pragma unroll
+            for (int k = 0; k < 12; ++k) g[k] = o[k];
+            g[12] = v;
+        }
+#pragma unroll 1
+        for (int q = q0; q < min(q0 + 4, nip); ++q) {
+#pragma unroll
+            for (int k = 0; k < T4_NC; ++k)
+                if (t + k * BS < 25 * T4_EB) s_c[t + k * BS] = pre[k];
+            __syncthreads();
+            if (q + 1 < nip) {
+#pragma unroll
+                for (int k = 0; k < T4_NC; ++k) pre[k] = Cb[src[k] + 81 * (q + 1)];
+            }
+            const double *g = s_g + 13 * (4 * el + q - q0), *c = s_c + 25 * el;
+            const double v = g[12];
+            double bn[12], bm[3];
+#pragma unroll
+            for (int k = 0; k < 12; ++k) bn[k] = g[k];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) bm[k] = g[3 * m + k];
+#pragma unroll
+            for (int a = 0; a < 5; ++a)
+#pragma unroll
+                for (int b = 0; b < 5; ++b) {
+                    const double bc = bm[sv[a]] * c[5 * a + b];
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) acc[n][sc[a]][sc[b]] += bc * bn[3 * n + sv[b]] * v;
+                }
+            __syncthreads(); // the point's tangents (and, after four, the geometry) are consumed
+        }
+    }
+    {
+        d2* row = reinterpret_cast<d2*>(smem + T4_KROW * t); // rows 2 m, 2 m + 1: 16 contiguous doubles
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) row[4 * i + n] = d2{acc[n][i][0], acc[n][i][1]};
+    }
+    __syncthreads();
+    double* Kb = K + 64 * e0;
+    if ((reinterpret_cast<uintptr_t>(K) & 15) == 0) {
+        for (int w = t; w < 32 * ne; w += BS)
+            __builtin_nontemporal_store(reinterpret_cast<const d2*>(smem + T4_KROW * (w / 8))[w % 8],
+                                        reinterpret_cast<d2*>(Kb) + w);
+    }
+    else
+        for (int w = t; w < 64 * ne; w += BS) Kb[w] = smem[T4_KROW * (w / 16) + w % 16];
 }
 
 void compute(gf_axi m, const double* x, hipStream_t s)
@@ -325,8 +385,7 @@ int gf_axi_int_gradN_dot_tensor4_dot_gradNT_dV(gf_axi m, const double* qtensor, 
     return guard([&] {
         GF_REQUIRE(m && qtensor && elemmat, "null argument");
         if (m->nelem)
-            k_axi_int_t4<<<nblocks(16 * m->nelem, BS), BS, 0, S(stream)>>>(m->nelem, m->rule.nip, m->G.p, m->vol.p,
-                                                                          qtensor, elemmat);
+            k_axi_int_t4<<<nblocks(m->nelem, T4_EB), BS, 0, S(stream)>>>(m->nelem, m->rule, m->x.p, qtensor, elemmat);
         check_launch();
     });
 }

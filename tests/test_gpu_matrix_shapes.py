@@ -92,3 +92,27 @@ def test_dot_on_a_nodevec(gf, mesh, numbering):
         buf[a:a + nnode * nd] = xd.ravel()
         A.Dot(buf[a:a + nnode * nd].view(nnode, nd), buf[b:b + nnode * nd].view(nnode, nd))
         assert np.array_equal(host(buf[b:b + nnode * nd].view(nnode, nd)), ref)
+
+
+@pytest.mark.parametrize("nelem,nip", [(1, 4), (63, 1), (64, 3), (65, 4), (130, 5), (7, 9), (3, 16)])
+def test_axisymmetric_stiffness(gf, nelem, nip):
+    """Workgroups of 64 elements, points four at a time; a general tensor, so that every slot pairing counts."""
+    import torch
+
+    rng = np.random.default_rng(nelem + nip)
+    c, conn = oracle.quad4_regular(nelem, 1)
+    zr = np.stack((c[:, 0], 0.5 + c[:, 1]), axis=1) + 0.1 * rng.uniform(-1, 1, c.shape)
+    x = oracle.Vector(conn, oracle.dofs(c.shape[0], 2)).AsElement(zr)
+    xi, w = rng.uniform(-0.9, 0.9, (nip, 2)), rng.uniform(0.5, 1.5, nip)
+    oq = oracle.QuadratureAxisymmetric(x, xi, w)
+    gq = gf.Element.Quad4.QuadratureAxisymmetric(x, xi, w)
+    C = rng.standard_normal((nelem, nip, 3, 3, 3, 3))
+    ref = oq.Int_gradN_dot_tensor4_dot_gradNT_dV(C)
+    assert np.array_equal(host(gq.Int_gradN_dot_tensor4_dot_gradNT_dV(C)), ref)
+    # arrays that are not 16-byte aligned
+    cb = torch.zeros(C.size + 1, dtype=torch.float64, device="cuda")
+    cb[1:] = torch.from_numpy(C.ravel()).cuda()
+    out = torch.zeros(ref.size + 1, dtype=torch.float64, device="cuda")
+    gq.Int_gradN_dot_tensor4_dot_gradNT_dV(cb[1:].view(C.shape), out=out[1:].view(ref.shape))
+    assert out[0].item() == 0.0
+    assert np.array_equal(host(out[1:].view(ref.shape)), ref)
