@@ -146,11 +146,20 @@ def _fn(name):
     return f
 
 
+_fns = {}  # name -> (ABI function, number of arguments)
+
+
 def _call(name, *args):
-    f = _fn(name)
-    if len(args) != len(f.argtypes):
-        raise TypeError(f"{name} takes {len(f.argtypes)} arguments ({len(args)} given)")
-    _check(f(*args))
+    fn = _fns.get(name)
+    if fn is None:
+        f = _fn(name)
+        fn = _fns[name] = (f, len(f.argtypes))
+    f, n = fn
+    if len(args) != n:
+        raise TypeError(f"{name} takes {n} arguments ({len(args)} given)")
+    rc = f(*args)
+    if rc != GF_OK:
+        _check(rc)
 
 
 def _hp(a: np.ndarray):
@@ -159,6 +168,11 @@ def _hp(a: np.ndarray):
 
 # -------------------------------------------------------------------------------------------------
 # device memory helpers (torch)
+#
+# They run several times in every operator, whose kernel takes a few microseconds on a small mesh: a
+# force evaluation (six kernels) of 1,230 elements took 72 us bound by them and takes 50.  Hence the device as an
+# index, the stream's handle without a Stream object, and operands that need no conversion passed through
+# after four checks.
 # -------------------------------------------------------------------------------------------------
 
 
@@ -177,6 +191,9 @@ def to_device(a, dtype=None):
     torch = _torch()
     if isinstance(a, torch.Tensor):
         t = a
+        if (t.is_cuda and t.dtype is (dtype or torch.float64) and t.is_contiguous()
+                and t.get_device() == torch.cuda.current_device()):
+            return t  # what .to().contiguous() below would return
     else:
         t = torch.from_numpy(np.ascontiguousarray(a))
     if dtype is None:
@@ -201,12 +218,17 @@ def _dp(t):
 
 
 def _stream():
-    return _vp(_torch().cuda.current_stream().cuda_stream)
+    """The handle of torch's current stream on the current device."""
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:  # not every torch build has it
+        return _vp(torch.cuda.current_stream().cuda_stream)
+    return _vp(raw(torch.cuda.current_device()))
 
 
 def _empty(shape, dtype=None):
     torch = _torch()
-    return torch.empty(shape, dtype=dtype or torch.float64, device=device())
+    return torch.empty(shape, dtype=dtype or torch.float64, device=torch.cuda.current_device())
 
 
 def _out(out, shape, dtype=None):
@@ -1339,10 +1361,13 @@ def elastic_stress(eps, K, G):
     eps = eps.contiguous() if isinstance(eps, torch.Tensor) and eps.is_cuda else to_device(eps)
     td = eps.shape[-1]
     nq = eps.numel() // (td * td)
-    Kq = to_device(torch.as_tensor(K).expand(eps.shape[:-2]) if not isinstance(K, torch.Tensor)
-                   else K.expand(eps.shape[:-2]), dtype=eps.dtype)
-    Gq = to_device(torch.as_tensor(G).expand(eps.shape[:-2]) if not isinstance(G, torch.Tensor)
-                   else G.expand(eps.shape[:-2]), dtype=eps.dtype)
+    points = eps.shape[:-2]
+
+    def modulus(a):
+        a = a if isinstance(a, torch.Tensor) else torch.as_tensor(a)
+        return to_device(a if a.shape == points else a.expand(points), dtype=eps.dtype)
+
+    Kq, Gq = modulus(K), modulus(G)
     out = torch.empty_like(eps)
     _call("gf_material_elastic_stress", _i64(nq), _i32(td), _dp(eps), _dp(Kq), _dp(Gq), _dp(out),
           _i32(_dtype_code(eps)), _stream())
