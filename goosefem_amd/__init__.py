@@ -2064,13 +2064,9 @@ class ExplicitQuad4(_Handle):
         _torch().cuda.current_stream().synchronize()
 
     def state(self):
-        n = self._vec.ndof
-        outs = []
-        for ptr in self._state_ptrs():
-            o = _empty((n,))
-            _hip_memcpy_d2d(o, ptr, 8 * n)
-            outs.append(o)
-        return tuple(outs)
+        outs = tuple(_empty((self._vec.ndof,)) for _ in range(3))
+        _call("gf_explicit_copy_state", self._h, *(_dp(o) for o in outs), _stream())
+        return outs
 
     def step(self, nsteps=1, precision=F64, store_fint=False, stream=None):
         s = _stream() if stream is None else stream

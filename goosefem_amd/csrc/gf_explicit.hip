@@ -153,7 +153,7 @@ __global__ void k_quotient_range(int64_t nelem, ShapeTable T, const int32_t* __r
 
 // The contributions c[m][i] of one Gauss point to the element's nodal forces; g = dN/dxi [4][2] and w the
 // weight of the point.  RCP: the quotients of the inverse by one reciprocal (k_quotient_range), the same
-// bits with 100 fewer of 790 FP64 instructions per element (general mesh of 656 k elements, FP64 issue bound
+// bits with 100 fewer of 790 FP64 instructions per element (general mesh of 514 k elements, FP64 issue bound
 // in this body: 28.1 -> 26.2 us per step; 400 x 400 grid 12.0 -> 11.2).
 template <bool RCP>
 __device__ inline void element_point_f64(const double (*g)[2], double w, const double x[4][2], const double u[4][2],
@@ -1053,6 +1053,26 @@ void launch_structured(int body, unsigned grid, hipStream_t s, int nx, int ny, i
     }
 }
 
+// The state to the caller's arrays in one launch, 16 bytes a thread.  Three device-to-device copies took
+// 10 us more at 8,450 DOFs, where a step takes 4.
+template <bool VEC>
+__global__ void __launch_bounds__(BS) k_copy_state(int64_t n, const double* __restrict__ u, const double* __restrict__ v,
+                                                   const double* __restrict__ a, double* __restrict__ uo,
+                                                   double* __restrict__ vo, double* __restrict__ ao)
+{
+    const double* src = blockIdx.y == 0 ? u : blockIdx.y == 1 ? v : a;
+    double* dst = blockIdx.y == 0 ? uo : blockIdx.y == 1 ? vo : ao;
+    const int64_t t = blockIdx.x * static_cast<int64_t>(BS) + threadIdx.x;
+    if constexpr (VEC) {
+        if (2 * t + 1 < n) {
+            __builtin_nontemporal_store(reinterpret_cast<const dvec2*>(src)[t], reinterpret_cast<dvec2*>(dst) + t);
+            return;
+        }
+        if (2 * t < n) dst[2 * t] = src[2 * t];
+    }
+    else if (t < n) dst[t] = src[t];
+}
+
 // Node blocks of the fused general step (k_explicit_blocks).  Used when every DOF belongs to
 // exactly one (node, component) -- a bijection onto [0, ndof) -- so that a DOF's contributions are
 // those of one node; tied meshes keep the element kernel + per-DOF gather.  The blocks come from a
@@ -1372,6 +1392,19 @@ int gf_explicit_state(gf_explicit x, double** u, double** v, double** a)
         if (u) *u = x->u[x->cur].p;
         if (v) *v = x->vv[x->cur].p;
         if (a) *a = x->a[x->cur].p;
+    });
+}
+
+int gf_explicit_copy_state(gf_explicit x, double* u, double* v, double* a, void* stream)
+{
+    return guard([&] {
+        GF_REQUIRE(x && u && v && a, "null argument");
+        const int64_t n = x->ndof;
+        if (!n) return;
+        const bool vec = aligned16(u) && aligned16(v) && aligned16(a);
+        (vec ? k_copy_state<true> : k_copy_state<false>)<<<dim3(nblocks(vec ? (n + 1) / 2 : n, BS), 3), BS, 0, S(stream)>>>(
+            n, x->u[x->cur].p, x->vv[x->cur].p, x->a[x->cur].p, u, v, a);
+        check_launch();
     });
 }
 

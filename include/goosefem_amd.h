@@ -522,6 +522,8 @@ int gf_explicit_create(gf_explicit* out, gf_vector v, const double* coor, const 
 int gf_explicit_destroy(gf_explicit x);
 /* state arrays (device, [ndof] each); writable between steps */
 int gf_explicit_state(gf_explicit x, double** u, double** v, double** a);
+/* the same state copied into the caller's arrays [ndof] */
+int gf_explicit_copy_state(gf_explicit x, double* u, double* v, double* a, void* stream);
 /* run nsteps steps; precision GF_F64 (bit-exact with the serial reference order), GF_F32 (FP32
  * strain/stress/force, FP64 assembly and update) or GF_F64_FAST (FP64 element work with FMA).
  * store_fint != 0 keeps the internal force of the last step (one extra [ndof] write). */

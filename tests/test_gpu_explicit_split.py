@@ -33,3 +33,22 @@ def test_split_step_bit_exact(gf, nx, ny, distort, kvar, any_mass, force):  # no
         gu, gv, ga = (host(t) for t in X.state())
         assert np.array_equal(gu, u) and np.array_equal(gv, v) and np.array_equal(ga, a)
         assert np.array_equal(host(X.fint()), fint)
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (14, 16), (127, 2)])  # 8, 510 and 768 DOFs: around a workgroup's 512
+def test_state_copies(gf, nx, ny, offset):  # noqa: F811
+    import torch
+
+    coor, conn, dofs, q, inv, Ke, Ge, u, v, a = _explicit_setup(nx, ny, fixed=False)
+    X = gf.ExplicitQuad4(gf.Vector(conn, dofs), coor, Ke, Ge, inv, 0.01)
+    rng = np.random.default_rng(nx)
+    ref = [rng.standard_normal(dofs.size) for _ in range(3)]
+    X.set_state(*ref)
+    assert all(np.array_equal(host(t), r) for t, r in zip(X.state(), ref))
+    n = dofs.size
+    buf = torch.full((3, n + 3), np.nan, dtype=torch.float64, device="cuda")
+    gf._call("gf_explicit_copy_state", X._h, *(gf._vp(buf[i, offset:].data_ptr()) for i in range(3)), gf._stream())
+    got = host(buf)
+    assert all(np.array_equal(got[i, offset:offset + n], ref[i]) for i in range(3))
+    assert np.isnan(got[:, :offset]).all() and np.isnan(got[:, offset + n:]).all()
