@@ -8,10 +8,9 @@
 // v_mfma_f32_32x32x16_bf16 (tile padded to 32 x 32, contraction to 80).  Both operands are split
 // x = hi + lo with hi = bf16(x), lo = bf16(x - hi); the product accumulates hi*hi + hi*lo + lo*hi
 // in FP32 (the dropped lo*lo term and the bf16 rounding of lo are ~2^-16 relative).
-// One wavefront owns one element at a time: C_q (8 x 81), dNx and dV are staged in LDS with
-// coalesced 16-byte loads (the next element's loads are issued before the current one is computed);
-// each MFMA lane evaluates the T entries it feeds, the 15 MFMAs accumulate the 32 x 32 tile, and the
-// 24 x 24 result is stored straight from the accumulators as contiguous FP64 rows.
+// One wavefront owns one element: C_q (8 x 81) and dNx, dV go through LDS, dNx split into its parts on the
+// way; each MFMA lane evaluates the T entries it feeds, the 15 MFMAs accumulate the 32 x 32 tile, and the
+// 24 x 24 result leaves through LDS as one contiguous stream.
 //
 // GF_F64: the same per-entry accumulation order as the reference loop (q, i, l for each (j, k)) on the
 // vector units, four elements per wavefront (k_stiffness_f64).
@@ -45,8 +44,8 @@ constexpr int KKP = 80;            // contraction length 72, padded to 5 x 16
 
 struct alignas(16) WaveLDS {
     float C[NC];
-    float g[NG];
-    float vol[NQ];
+    float gv[NG];    // dN/dx dV
+    uint32_t hl[NG]; // dN/dx in two bf16 parts, the high one in the low half
 };
 
 // hi/lo split of eight values, converted in pairs (one packed conversion per pair and part)
@@ -65,12 +64,9 @@ __device__ inline void split8(const float (&x)[8], bf16x8& hi, bf16x8& lo)
     }
 }
 
-// one element's C, dNx, dV in registers (16-byte loads), so that the next element's loads are in
-// flight while the current one is computed.  C is FP64 (the reference's qtensor4) or FP32.
-// Loads are unconditional (lanes past the end of an array re-read its last entry, which
-// store_stage ignores), so that no branch hides them from the compiler's wait counting.
-constexpr int NG2 = NG / 2, RG = (NG2 + 63) / 64;
-
+// one element's C on its way to LDS; C is FP64 (the reference's qtensor4) or FP32.  Loads are unconditional
+// (lanes past the end re-read the last entry, which store ignores), so that no branch hides them from the
+// compiler's wait counting.
 template <class TC>
 struct StageC;
 
@@ -117,82 +113,64 @@ struct StageC<float> {
     }
 };
 
-template <class TC>
-struct Stage {
-    StageC<TC> c;
-    double2 g[RG];
-    double v;
-};
-
-template <class TC>
-__device__ inline void load_stage(Stage<TC>& st, const TC* __restrict__ C, const double* __restrict__ dNx,
-                                  const double* __restrict__ vol, int64_t e, int lane)
+// The 32 x 32 FP32 tile whose top-left 24 x 24 block is K_e of the element with the staged C, gv and hl.
+//
+// MFMA: lane l supplies A row (l % 32) and B column (l % 32) at contraction slots 8 (l / 32) + s of each
+// 16-wide chunk.  The contraction index kk = (q, j2, i) is laid out so that each half-wave h owns
+// quadrature points 4h..4h+3: slot s of chunk ch is t = 8 ch + s, q = 4h + t / 9, (j2, i) = t % 9 (t < 36; the
+// last 4 slots are zero).  Every index below is then a compile-time constant plus a per-lane base.  Row
+// (m, j) of A and column (n, k) of T share the decomposition 3 m + j = 3 n + k, so both operands use
+// dNx(q, m, :):  A = delta(j, j2) dNx(q, m, i),  T = sum_l C_q(i, j2, j, l) dV_q dNx(q, m, l).  Rows and
+// columns 24..31 are padding, no part of the block: they repeat node 7.
+//
+// The vector units issue nearly all of the time here, so A comes split from LDS (once per entry instead of
+// once per use): a pair of slots is two entries' halves side by side under the lane's mask of j.
+__device__ __forceinline__ floatx16 element_tile(const float* C, const float* gv, const uint32_t* hl, int lane)
 {
-    st.c.load(C, e, lane);
-    const double2* ge = reinterpret_cast<const double2*>(dNx + e * NG);
-#pragma unroll
-    for (int k = 0; k < RG; ++k) st.g[k] = ge[min(lane + 64 * k, NG2 - 1)];
-    st.v = vol[e * NQ + min(lane, NQ - 1)];
-}
-
-template <class TC>
-__device__ inline void store_stage(const Stage<TC>& st, WaveLDS& L, int lane)
-{
-    st.c.store(L.C, lane);
-#pragma unroll
-    for (int k = 0; k < RG; ++k) {
-        const int t = lane + 64 * k;
-        if (t < NG2) {
-            L.g[2 * t] = static_cast<float>(st.g[k].x);
-            L.g[2 * t + 1] = static_cast<float>(st.g[k].y);
-        }
-    }
-    if (lane < NQ) L.vol[lane] = static_cast<float>(st.v);
-}
-
-// The 32 x 32 FP32 tile whose top-left 24 x 24 block is K_e of the element staged in L.
-__device__ __forceinline__ floatx16 element_tile(const WaveLDS& L, int lane)
-{
-    // MFMA: lane l supplies A row (l % 32) and B column (l % 32) at contraction slots
-    // 8 (l / 32) + s of each 16-wide chunk.  The contraction index kk = (q, j2, i) is laid out so
-    // that each half-wave h owns quadrature points 4h..4h+3: slot s of chunk ch is
-    // t = 8 ch + s, q = 4h + t / 9, (j2, i) = t % 9 (t < 36; the last 4 slots are zero).  Every
-    // index below is then a compile-time constant plus a per-lane base.  Row (m, j) of A and
-    // column (n, k) of T share the decomposition 3 m + j = 3 n + k, so both operands use
-    // dNx(q, m, :):  A = delta(j, j2) dNx(q, m, i),  T = sum_l C_q(i, j2, j, l) dV_q dNx(q, m, l).
     const int row = lane % 32, h = lane / 32;
     const int j = row % 3, m = row < 24 ? row / 3 : 7;
-    const bool live = row < 24; // rows 24..31 of the 32 x 32 tile are padding
-    const float* Cb = L.C + h * 4 * 81 + j * 3;
-    const float* gb = L.g + (h * 4 * NN + m) * 3;
-    const float* vb = L.vol + h * 4;
+    const float* Cb = C + h * 4 * 81 + j * 3;
+    const float* gb = gv + (h * 4 * NN + m) * 3;
+    const uint32_t* ab = hl + (h * 4 * NN + m) * 3;
+    // the slots of a pair that are the lane's: both of group j2 = J, or the last of J with the first of J + 1
+    const uint32_t both[3] = {j == 0 ? ~0u : 0u, j == 1 ? ~0u : 0u, j == 2 ? ~0u : 0u};
+    const uint32_t over[3] = {j == 0 ? 0xFFFFu : j == 1 ? 0xFFFF0000u : 0u, j == 1 ? 0xFFFFu : j == 2 ? 0xFFFF0000u : 0u,
+                              j == 2 ? 0xFFFFu : j == 0 ? 0xFFFF0000u : 0u};
+    uint32_t a[12]; // the half-wave's 4 points x 3 components
+#pragma unroll
+    for (int t = 0; t < 12; ++t) a[t] = ab[(t / 3) * 24 + t % 3];
     floatx16 acc = {};
-    float gq[3] = {0.0f, 0.0f, 0.0f}, gv[3] = {0.0f, 0.0f, 0.0f};
+    float g[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int ch = 0; ch < KKP / 16; ++ch) {
-        float av[8], bv[8];
+        float bv[8];
+        uint32_t ah[4], al[4];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             const int t = ch * 8 + s;
-            av[s] = 0.0f;
             bv[s] = 0.0f;
             if (t < 36) {
                 const int ql = t / 9, r = t % 9, j2 = r / 3, i = r % 3;
                 if (r == 0) {
-                    const float v = vb[ql];
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        gq[c] = live ? gb[ql * 24 + c] : 0.0f;
-                        gv[c] = gq[c] * v;
-                    }
+                    for (int c = 0; c < 3; ++c) g[c] = gb[ql * 24 + c];
                 }
                 const float* Cq = Cb + ql * 81 + (i * 3 + j2) * 9;
-                bv[s] = fmaf(Cq[0], gv[0], fmaf(Cq[1], gv[1], Cq[2] * gv[2]));
-                av[s] = j == j2 ? gq[i] : 0.0f;
+                bv[s] = fmaf(Cq[0], g[0], fmaf(Cq[1], g[1], Cq[2] * g[2]));
+                if (s % 2 == 0) {
+                    // slots t and t + 1 (35 is odd, so a pair never crosses the end)
+                    const int r1 = (t + 1) % 9;
+                    const uint32_t lo = a[ql * 3 + i], hi = a[((t + 1) / 9) * 3 + r1 % 3];
+                    const uint32_t mask = j2 == r1 / 3 ? both[j2] : over[j2];
+                    ah[s / 2] = __builtin_amdgcn_perm(hi, lo, 0x05040100) & mask;
+                    al[s / 2] = __builtin_amdgcn_perm(hi, lo, 0x07060302) & mask;
+                }
             }
+            else if (s % 2 == 0) ah[s / 2] = al[s / 2] = 0u;
         }
         bf16x8 ahi, alo, bhi, blo;
-        split8(av, ahi, alo);
+        __builtin_memcpy(&ahi, ah, sizeof(ahi));
+        __builtin_memcpy(&alo, al, sizeof(alo));
         split8(bv, bhi, blo);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, bhi, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, blo, acc, 0, 0, 0);
@@ -208,55 +186,70 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Store K_e: the tile's 24 x 24 block goes through LDS (into the staged C, which is no longer read)
-// so that each lane writes 9 doubles with full-wave contiguous stores and no lane is masked off.
+// Store K_e: the tile's 24 x 24 block goes through LDS (into the staged C, which is no longer read) and
+// leaves as one contiguous stream, 16 bytes a lane (VEC: elemmat 16-byte aligned).
 // Accumulator layout: value r of lane l is K[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
-template <class TK>
-__device__ __forceinline__ void store_tile(WaveLDS& L, const floatx16& acc, TK* __restrict__ Ke, int lane)
+template <class TK, bool VEC>
+__device__ __forceinline__ void store_tile(float* Ks, const floatx16& acc, TK* __restrict__ Ke, int lane)
 {
     const int row = lane % 32, h = lane / 32;
-    float* Ks = L.C;
     wave_sync();
     if (row < 24) {
 #pragma unroll
         for (int r = 0; r < 12; ++r) Ks[(8 * (r / 4) + 4 * h + (r % 4)) * 24 + row] = acc[r];
     }
     wave_sync();
+    if constexpr (VEC) {
+        constexpr int VW = 16 / static_cast<int>(sizeof(TK)), NV = 576 / VW;
+        typedef TK vec __attribute__((ext_vector_type(VW)));
 #pragma unroll
-    for (int k = 0; k < 9; ++k) Ke[lane + 64 * k] = static_cast<TK>(Ks[lane + 64 * k]);
+        for (int k = 0; k < (NV + 63) / 64; ++k) {
+            const int t = lane + 64 * k;
+            if (t < NV) {
+                vec v;
+#pragma unroll
+                for (int c = 0; c < VW; ++c) v[c] = static_cast<TK>(Ks[VW * t + c]);
+                __builtin_nontemporal_store(v, reinterpret_cast<vec*>(Ke) + t);
+            }
+        }
+    }
+    else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) Ke[lane + 64 * k] = static_cast<TK>(Ks[lane + 64 * k]);
+    }
 }
 
-// One wavefront per element, grid-stride.  The loop is rotated (store K_e of element e, then
-// wait for element e + stride's loads, which were issued before those stores) so that waiting for
-// the next element's data never waits for the previous element's stores.
-template <class TC, class TK>
+// One wavefront per element, all of whose loads are issued first; many small waves hide them (a wave that
+// goes through several elements with the next one's loads in flight measured slower).  Bound by HBM: 6,496
+// bytes per element with FP32 arrays (C 2,592, dN/dx and dV 1,600, K_e 2,304).  276,480 elements: 321-333 us,
+// 5.4-5.6 TB/s (331-339 us with A split at each use and scalar stores); 140,000: 160 us (173-179); 6,120: 9.4 us
+// (11.7).  Forming the geometry from the coordinates saves 1,408 of the bytes and costs more: 323 us with
+// one point per lane for eight elements at a time, 350 for four, 386 spread over the wave of each element;
+// vector issue and waves in flight are then what is short.
+template <class TC, class TK, bool VEC>
 __global__ void __launch_bounds__(64 * WAVES) k_stiffness_bf16x3(int64_t nelem, const TC* __restrict__ C,
-                                                                  const double* __restrict__ dNx,
-                                                                  const double* __restrict__ vol,
-                                                                  TK* __restrict__ elemmat)
+                                                                 const double* __restrict__ dNx,
+                                                                 const double* __restrict__ vol, TK* __restrict__ elemmat)
 {
     __shared__ WaveLDS lds[WAVES];
     const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
     WaveLDS& L = lds[w];
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * WAVES;
-    int64_t e = static_cast<int64_t>(blockIdx.x) * WAVES + w;
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * WAVES + w;
     if (e >= nelem) return; // uniform per wave; the kernel has no workgroup barrier
-    Stage<TC> st;
-    load_stage(st, C, dNx, vol, e, lane);
-    store_stage(st, L, lane);
-    wave_sync();
-    load_stage(st, C, dNx, vol, min(e + stride, nelem - 1), lane);
-    floatx16 acc = element_tile(L, lane);
-    for (;;) {
-        store_tile(L, acc, elemmat + e * 576, lane);
-        e += stride;
-        if (e >= nelem) break;
-        wave_sync();
-        store_stage(st, L, lane);
-        wave_sync();
-        load_stage(st, C, dNx, vol, min(e + stride, nelem - 1), lane);
-        acc = element_tile(L, lane);
+    StageC<TC> st;
+    st.load(C, e, lane);
+#pragma unroll
+    for (int k = 0; k < NG / 64; ++k) {
+        const int t = lane + 64 * k;
+        const float f = static_cast<float>(dNx[e * NG + t]), v = static_cast<float>(vol[e * NQ + t / 24]);
+        const __bf16 hi = static_cast<__bf16>(f), lo = static_cast<__bf16>(f - static_cast<float>(hi));
+        L.gv[t] = f * v;
+        L.hl[t] = __builtin_bit_cast(uint16_t, hi) | static_cast<uint32_t>(__builtin_bit_cast(uint16_t, lo)) << 16;
     }
+    st.store(L.C, lane);
+    wave_sync();
+    const floatx16 acc = element_tile(L.C, L.gv, L.hl, lane);
+    store_tile<TK, VEC>(L.C, acc, elemmat + e * 576, lane);
 }
 
 // FP64 in reference order: acc(j, k) += ((dNx(m,i) C(i,j,k,l)) dNx(n,l)) dV over q, i, l.  8 GRP lanes
@@ -472,29 +465,29 @@ unsigned grid_for(int64_t nelem, int per_wave = 1)
 
 namespace gf {
 
+template <class TC, class TK>
+void launch_bf16x3(gf_quad q, const TC* C, TK* elemmat, hipStream_t s)
+{
+    GF_REQUIRE(quad_etype(q) == GF_HEX8 && quad_nip(q) == NQ, "GF_BF16X3 needs Hex8 with 8 points");
+    GF_REQUIRE(aligned16(C), "GF_BF16X3 needs a 16-byte aligned qtensor4 array");
+    const int64_t ne = quad_nelem(q);
+    if (ne == 0) return;
+    auto kern = aligned16(elemmat) ? k_stiffness_bf16x3<TC, TK, true> : k_stiffness_bf16x3<TC, TK, false>;
+    kern<<<nblocks(ne, WAVES), 64 * WAVES, 0, s>>>(ne, C, quad_dNx(q), quad_vol(q), elemmat);
+    check_launch();
+}
+
 int stiffness_bf16x3(gf_quad q, const double* C, double* elemmat, hipStream_t s)
 {
     return guard([&] {
-        GF_REQUIRE(quad_etype(q) == GF_HEX8 && quad_nip(q) == NQ, "GF_BF16X3 needs Hex8 with 8 points");
-        GF_REQUIRE(aligned16(C) && aligned16(elemmat),
-                   "GF_BF16X3 needs 16-byte aligned qtensor4 and elemmat arrays");
-        const int64_t ne = quad_nelem(q);
-        if (ne == 0) return;
-        k_stiffness_bf16x3<double, double><<<grid_for(ne), 64 * WAVES, 0, s>>>(ne, C, quad_dNx(q), quad_vol(q), elemmat);
-        check_launch();
+        GF_REQUIRE(aligned16(elemmat), "GF_BF16X3 needs 16-byte aligned qtensor4 and elemmat arrays");
+        launch_bf16x3(q, C, elemmat, s);
     });
 }
 
 int stiffness_bf16x3_f32(gf_quad q, const float* C, float* elemmat, hipStream_t s)
 {
-    return guard([&] {
-        GF_REQUIRE(quad_etype(q) == GF_HEX8 && quad_nip(q) == NQ, "GF_BF16X3 needs Hex8 with 8 points");
-        GF_REQUIRE(aligned16(C), "GF_BF16X3 needs a 16-byte aligned qtensor4 array");
-        const int64_t ne = quad_nelem(q);
-        if (ne == 0) return;
-        k_stiffness_bf16x3<float, float><<<grid_for(ne), 64 * WAVES, 0, s>>>(ne, C, quad_dNx(q), quad_vol(q), elemmat);
-        check_launch();
-    });
+    return guard([&] { launch_bf16x3(q, C, elemmat, s); });
 }
 
 int stiffness_f64_hex8(gf_quad q, const double* C, double* elemmat, hipStream_t s)

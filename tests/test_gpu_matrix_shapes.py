@@ -116,3 +116,34 @@ def test_axisymmetric_stiffness(gf, nelem, nip):
     gq.Int_gradN_dot_tensor4_dot_gradNT_dV(cb[1:].view(C.shape), out=out[1:].view(ref.shape))
     assert out[0].item() == 0.0
     assert np.array_equal(host(out[1:].view(ref.shape)), ref)
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 1, 1), (2, 2, 1), (5, 1, 1), (17, 19, 23)])
+def test_matrix_core_stiffness_of_any_number_of_elements(gf, n):
+    """Four elements per workgroup, the last one partly filled.  An operand keeps its first two bf16 parts: the second is at most 2^-9 of it and what
+    is left 2^-18, so a product of two loses 3 * 2^-18 (both remainders and the low parts' product); the 72
+    sums and the rounding of the operands in FP32 add 77 * 2^-24, all relative to the sum of the terms'
+    magnitudes."""
+    import torch
+
+    c, conn = oracle.hex8_regular(*n)
+    rng = np.random.default_rng(sum(n))
+    c = c + 0.1 * rng.uniform(-1, 1, c.shape)
+    x = oracle.Vector(conn, oracle.dofs(c.shape[0], 3)).AsElement(c)
+    q = oracle.Quadrature(HEX8, x)
+    C = rng.standard_normal((q.nelem, 8, 3, 3, 3, 3)).astype(np.float32)
+    gq = gf.Element.Hex8.Quadrature(x)
+    ref = q.Int_gradN_dot_tensor4_dot_gradNT_dV(C.astype(np.float64))
+    Cd = torch.from_numpy(C).cuda()
+    k32 = host(gq.Int_gradN_dot_tensor4_dot_gradNT_dV(Cd, gf.BF16X3))
+    g, ab = np.abs(q.dNx), np.zeros_like(ref)
+    for k in range(8):
+        t = np.einsum("eijkl,enl,e->eijnk", np.abs(C[:, k], dtype=np.float64), g[:, k], q.dV()[:, k])
+        ab += np.einsum("emi,eijnk->emjnk", g[:, k], t).reshape(ref.shape)
+    assert (np.abs(k32 - ref) <= (3 * 2.0**-18 + 77 * 2.0**-24) * ab).all()
+    k64 = host(gq.Int_gradN_dot_tensor4_dot_gradNT_dV(Cd.double(), gf.BF16X3))
+    assert np.array_equal(k64.astype(np.float32), k32)
+    buf = torch.full((k32.size + 2,), np.nan, dtype=torch.float32, device="cuda")
+    out = buf[1:-1].view(k32.shape)  # not 16-byte aligned
+    gq.Int_gradN_dot_tensor4_dot_gradNT_dV(Cd, gf.BF16X3, out=out)
+    assert np.array_equal(host(out), k32) and np.isnan(host(buf[[0, -1]])).all()
