@@ -1077,15 +1077,20 @@ __global__ void __launch_bounds__(BS) k_copy_state(int64_t n, const double* __re
 // exactly one (node, component) -- a bijection onto [0, ndof) -- so that a DOF's contributions are
 // those of one node; tied meshes keep the element kernel + per-DOF gather.  The blocks come from a
 // recursive coordinate bisection of the nodes: a set is split across its longer extent in proportion to
-// the numbers of blocks on either side, so every block is a compact patch of about PATCH nodes.  208
-// nodes touch about 250 elements, so that the element phase is one pass of the 256 threads; patches of
+// the numbers of blocks on either side, so every block is a compact patch of about 208 nodes.  These
+// touch about 250 elements, so that the element phase is one pass of the 256 threads; patches of
 // 256 nodes touch 290 and leave three of four waves waiting for a second pass (0.49 M elements: 345
 // instead of 369 us per 20 steps in FP32, 557 instead of 572 in reference-order FP64; 11 k elements 117
-// instead of 135 and 163 instead of 185).  Each block's nodes are then put in ascending
+// instead of 135 and 163 instead of 185).  A mesh whose step streams more than the 256 MB last-level cache
+// (about 140 bytes a node: u, v, a of both parities, coordinates, connectivity, moduli) takes patches of 256
+// nodes: each patch reads and writes whole rows of lines only where its rows are as wide, and the lines that
+// patches share then come from HBM.  us per step, FP32 / reference-order FP64 / FP64 with FMA, with 208 and
+// 256 nodes: 1.5 M elements 39.2 / 59.0 / 45.1 and 40.1 / 68.9 / 51.0; 2.1 M 78.4 / 119 / 103 and
+// 78.0 / 124 / 100; 3.9 M 144 / 218 / 189 and 142 / 196 / 158.  Each block's nodes are then put in ascending
 // number so that neighbouring threads touch neighbouring DOFs.  rank[e]: position of original
 // element e in the locality order; cp, kp, gp: connectivity [4] and moduli in that order.  Blocks
 // whose local nodes and element forces would not fit in 64 KiB of LDS keep the two-kernel path.
-constexpr int64_t PATCH = 208;
+constexpr int64_t PATCH = 208, PATCH_HBM = 256, HBM_NODES = (int64_t(256) << 20) / 140;
 
 void build_node_blocks(gf_explicit_s* x, gf_vector v, const double* coor_d, const std::vector<int32_t>& rank,
                        const std::vector<int32_t>& cp, const std::vector<float>& kp, const std::vector<float>& gp)
@@ -1108,7 +1113,8 @@ void build_node_blocks(gf_explicit_s* x, gf_vector v, const double* coor_d, cons
     struct Part {
         int64_t b, e, np; // a node range and the number of blocks it is cut into
     };
-    std::vector<Part> todo{{0, nn, (nn + PATCH - 1) / PATCH}};
+    const int64_t patch = nn <= HBM_NODES ? PATCH : PATCH_HBM;
+    std::vector<Part> todo{{0, nn, (nn + patch - 1) / patch}};
     std::vector<std::pair<int64_t, int64_t>> leaf;
     while (!todo.empty()) {
         const auto [b, e, np] = todo.back();

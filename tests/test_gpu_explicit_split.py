@@ -52,3 +52,13 @@ def test_state_copies(gf, nx, ny, offset):  # noqa: F811
     got = host(buf)
     assert all(np.array_equal(got[i, offset:offset + n], ref[i]) for i in range(3))
     assert np.isnan(got[:, :offset]).all() and np.isnan(got[:, offset + n:]).all()
+
+
+@pytest.mark.parametrize("n", [1383, 1385])  # 1,915,456 and 1,920,996 nodes: the last with patches of 208, the first of 256
+def test_general_mesh_on_either_side_of_the_cache(gf, n):  # noqa: F811
+    coor, conn, dofs, q, inv, Ke, Ge, u, v, a = _explicit_setup(n, n, shuffle=True)
+    X = gf.ExplicitQuad4(gf.Vector(conn, dofs), coor, Ke, Ge, inv, 0.01)
+    X.set_state(u, v, a)
+    oracle.vv_steps(1, QUAD4_PLANAR, conn, dofs, q.dNx, q.dV(), Ke, Ge, inv, 0.01, u, v, a)
+    X.step(1, gf.F64)
+    assert all(np.array_equal(host(g), r) for g, r in zip(X.state(), (u, v, a)))
