@@ -597,7 +597,8 @@ def bench_newton(args):
 def bench_statics(args):
     """One load increment of the statics example on the device: a Quad4 plane-strain n^2 plate, J2
     linear hardening, bottom edge fixed, top edge sheared; Newton iterations of the fused element
-    pass, MatrixPartitioned assembly (CSR + the four blocks) and the partitioned Jacobi-PCG solve."""
+    pass, MatrixPartitioned assembly (CSR + the four blocks) and the partitioned solve (CG preconditioned
+    by multigrid on the grid)."""
     import torch
 
     import goosefem_amd as gf
@@ -655,9 +656,10 @@ def bench_statics(args):
     nnu = vector.nnu
     cg_its = sum(its)
     t_it = t_solve / max(cg_its, 1)
-    # per CG iteration: A_uu p (12 B/nnz + p, q), the update (p, q, diag, x, r read; x, r, z
-    # written) and the direction (z, p read; p written): 12 nnz + 15 * 8 nnu bytes
-    b_it = 12 * nnz_uu + 120 * nnu
+    # per CG iteration: three passes over the fine grid's nine 2 x 2 stencil blocks (down, up, product) and two
+    # over the coarse grids' (a third of the nodes in all), 288 bytes a node each, and 12 vector passes; the
+    # solve's share of the whole (t_solve) also holds the residual, its norms and the host's part
+    b_it = mesh.nnode * (3 * 288 + 2 * 288 / 3 + 12 * 16)
     ach = b_it / t_it / 1e9
     res = {
         "metric": "Statics load increment (J2 plate, Newton + partitioned PCG) wall time",
@@ -670,7 +672,7 @@ def bench_statics(args):
                    "plastic_fraction": float((mat.epsp > 0).double().mean())},
         "dtype": "f64",
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
-                     "kernel": "partitioned Jacobi-PCG iteration (k_cg_apply_dir + k_cg_update)",
+                     "kernel": "multigrid-preconditioned CG iteration (k_mg_*)",
                      "traffic": None, "algorithmic_bytes_per_launch": b_it, "avg_launch_us": t_it * 1e6},
         "breakdown_s": {"fused_element_pass": t_el, "matrix_assemble": t_asm, "solve": t_solve,
                         "pattern_build": t_pattern},
@@ -1047,10 +1049,10 @@ def api_kernels(kind, n):
                           ("Int_gradN_dot_tensor2_dV", t_int, bytes_int)):
             gbs = scale * b * E / t / 1e9
             row[key] = {"us": t * 1e6, "achieved_GBs": gbs, "frac": gbs / HBM_PEAK_GBS}
-            if kind == "hex8" and nm == "f64" and key != "Int_gradN_dot_tensor2_dV":
-                # the FP64 Hex8 gradients recompute dN/dx from the element coordinates: they move
-                # coordinates 192 + u_e 192 + qtensor 576 B per element, not the stored 1536 B of dN/dx
-                moved = nne * nd * 8 * 2 + nip * 9 * 8
+            if kind == "quad4" or nm == "f64":
+                # the Quad4 kernels and the FP64 Hex8 ones form dN/dx from the FP64 element coordinates: they
+                # move those (64 or 192 B per element), the element vector and the tensors, not the stored dN/dx
+                moved = nne * nd * 8 * (1 + scale) + scale * nip * 9 * 8
                 row[key].update(geometry="recomputed from the element coordinates",
                                 moved_bytes_per_element=moved, frac_moved=moved * E / t / 1e9 / HBM_PEAK_GBS)
         out[nm] = row
