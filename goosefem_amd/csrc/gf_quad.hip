@@ -644,6 +644,52 @@ __global__ void __launch_bounds__(PB3) k_int_tensor2_h8(int64_t nelem, int nip, 
     stage_out<T, PB3>(elemvec + e0 * 24, s_s, ne * 24);
 }
 
+// FP32 Hex8 from the stored geometry with everything staged: whole-wave streams of dN/dx, dV and the
+// tensors, one thread per (element, node) over the points.  The same order of sums.  Taken where the arrays
+// leave the caches behind: us with k_int_tensor2_h8 and staged, 110,592 elements 20.9 and 23.5; 394,831: 82.1
+// and 82.0; 884,736: 182 and 176; 2,097,152: 441 and 416.
+constexpr int EBS = 16; // elements per workgroup
+constexpr int64_t H8_STAGED = 400000;
+
+inline size_t int2_h8_staged_lds_bytes(int nip) { return (static_cast<size_t>(EBS) * nip * 34 + EBS * 24) * 4; }
+
+__global__ void __launch_bounds__(EBS * 8) k_int_tensor2_h8_staged(int64_t nelem, int nip, const float* __restrict__ dNx,
+                                                                   const float* __restrict__ vol,
+                                                                   const float* __restrict__ qtensor,
+                                                                   float* __restrict__ elemvec)
+{
+    constexpr int NT = EBS * 8;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * EBS;
+    const int ne = static_cast<int>(min<int64_t>(EBS, nelem - e0));
+    float* s_g = reinterpret_cast<float*>(smem); // [EBS nip][24]
+    float* s_s = s_g + EBS * nip * 24;           // [EBS nip][9]
+    float* s_o = s_s + EBS * nip * 9;            // [EBS][24]
+    float* s_v = s_o + EBS * 24;                 // [EBS nip]
+    stage_in<float, NT, 6>(s_g, dNx + e0 * nip * 24, ne * nip * 24);
+    stage_in<float, NT, 3>(s_s, qtensor + e0 * nip * 9, ne * nip * 9);
+    stage_in<float, NT, 1>(s_v, vol + e0 * nip, ne * nip);
+    __syncthreads();
+    const int el = threadIdx.x / 8, m = threadIdx.x % 8;
+    if (el < ne) {
+        float f[3] = {0.0f, 0.0f, 0.0f};
+        for (int q = 0; q < nip; ++q) {
+            const float *g = s_g + ((el * nip + q) * 8 + m) * 3, *sq = s_s + (el * nip + q) * 9;
+            const float v = s_v[el * nip + q];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                float a = g[0] * sq[j] + g[1] * sq[3 + j];
+                a = a + g[2] * sq[6 + j];
+                f[j] += a * v;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s_o[(el * 8 + m) * 3 + j] = f[j];
+    }
+    __syncthreads();
+    stage_out<float, NT>(elemvec + e0 * 24, s_o, ne * 24);
+}
+
 // (at least 9 values per point and 24 per element behind the contributions)
 inline size_t int2_h8_lds_bytes(int nip, size_t sz)
 {
@@ -1163,6 +1209,13 @@ int gf_quad_int_gradN_dot_tensor2_dV(gf_quad q, const void* qtensor, void* elemv
                 else {
                     gx = q->x.p;
                     gv = q->w_d.p;
+                }
+                if constexpr (std::is_same_v<T, float>) {
+                    if (E >= H8_STAGED && int2_h8_staged_lds_bytes(nip) <= 32768) {
+                        k_int_tensor2_h8_staged<<<nblocks(E, EBS), EBS * 8, int2_h8_staged_lds_bytes(nip), s>>>(E, nip, gx, gv,
+                                                                                                               in, o);
+                        return;
+                    }
                 }
                 k_int_tensor2_h8<T><<<nblocks(E, PB3 / nip), PB3, int2_h8_lds_bytes(nip, sz), s>>>(
                     E, nip, gx, q->dNxi_d.p, gv, in, o);

@@ -175,3 +175,19 @@ def test_vector_numberings(gf, et, numbering):
     for a in (torch.from_numpy(e32).cuda(), unaligned(e32)):
         assert np.array_equal(host(gv.AssembleDofs(a)), want_d)
         assert np.array_equal(host(gv.AssembleNode(a)), ov.AsNode(want_d))
+
+
+@pytest.mark.parametrize("nelem", [399999, 400000, 400007])
+def test_hex8_fp32_integral_of_large_arrays(gf, nelem):
+    """From 400,000 elements on the FP32 integral streams everything through LDS; the same bits as a few
+    elements at a time."""
+    import torch
+
+    x = elements(HEX8, 500, 3)
+    rng = np.random.default_rng(nelem)
+    qt = torch.from_numpy(rng.standard_normal((500, 8, 3, 3)).astype(np.float32)).cuda()
+    few = host(gf.Element.Hex8.Quadrature(x).Int_gradN_dot_tensor2_dV(qt))
+    idx = torch.arange(nelem, device="cuda") % 500
+    many = gf.Element.Hex8.Quadrature(torch.from_numpy(x).cuda()[idx].contiguous())
+    got = many.Int_gradN_dot_tensor2_dV(qt[idx].contiguous())
+    assert torch.equal(got, torch.from_numpy(few).cuda()[idx])
