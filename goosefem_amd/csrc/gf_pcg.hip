@@ -995,8 +995,24 @@ bool uniform_per_element(const double* data, int64_t nelem, int n, double* first
     return true;
 }
 
+// true if every unknown is the DOF of exactly one grid node and component: the structured kernels write
+// each node's sum to its unknown, so two nodes of one unknown would overwrite each other and an unknown
+// without a node would stay unwritten
+bool one_place_per_unknown(const std::vector<int32_t>& sidx, int64_t nnu)
+{
+    std::vector<char> seen(nnu, 0);
+    int64_t found = 0;
+    for (int32_t d : sidx) {
+        if (d < 0) continue;
+        if (seen[d]) return false;
+        seen[d] = 1;
+        ++found;
+    }
+    return found == nnu;
+}
+
 // Regular nx x ny Quad4 cell (at least 8 elements each way: a halo row wraps onto a line of its own)
-// whose dependent DOFs are periodic copies (C_du rows = one unit entry of the partner's u-DOF, or empty
+// with one unknown per free node and component, whose dependent DOFs are periodic copies (C_du rows = one unit entry of the partner's u-DOF, or empty
 // when the partner is prescribed) and whose elements share one geometry: then K' x_u is applied by
 // k_apply_periodic_q4.
 void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_col_h, const double* cdu_val_h)
@@ -1046,6 +1062,7 @@ void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_co
                 const int64_t d = dof(j * N1 + i, c);
                 sidx[(j * nx + i) * 2 + c] = d < P->nnu ? static_cast<int32_t>(d) : -1;
             }
+    if (!one_place_per_unknown(sidx, P->nnu)) return;
     P->sidx.alloc(sidx.size());
     GF_HIP(hipMemcpy(P->sidx.p, sidx.data(), sidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     for (int k = 0; k < 32; ++k) P->sh_g[k] = g[k];
@@ -1145,6 +1162,7 @@ void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* c
                     const int64_t d = dof(node(i, j, k), c);
                     sidx[((k * ny + j) * nx + i) * 3 + c] = d < P->nnu ? static_cast<int32_t>(d) : -1;
                 }
+    if (!one_place_per_unknown(sidx, P->nnu)) return;
     P->sidx.alloc(sidx.size());
     GF_HIP(hipMemcpy(P->sidx.p, sidx.data(), sidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     P->ke8.alloc(kkg.size());

@@ -258,3 +258,73 @@ def test_structured_operator_of_any_size(gf, size):
     assert res <= 1e-9 and np.linalg.norm(b - A @ host(sol)) <= 1e-9 * np.linalg.norm(b)
     again, it2, _ = P.solve(b, tol=1e-10)
     assert it2 == it and np.array_equal(host(again), host(sol))
+
+
+def tied_cell(gf, size, merge=(), spare=0):
+    """A Regular periodic cell (origin fixed) in the numbering [u | p | d], as a program may pass it:
+    unknowns of each group in merge are made one, and `spare` nodes that no element uses bring two or three
+    unknowns each.  (mesh, vector, quadrature, moduli, tyings, dense K' from the element matrices at coor)"""
+    from types import SimpleNamespace
+
+    nd = len(size)
+    mesh = gf.Mesh.Quad4.Regular(*size) if nd == 2 else gf.Mesh.Hex8.Regular(*size)
+    ctrl = gf.Tyings.Control(mesh.coor, mesh.dofs)
+    iip = np.concatenate((ctrl.controlDofs.ravel(), ctrl.dofs[mesh.nodesOrigin]))
+    ty = gf.Tyings.Periodic(ctrl.coor, ctrl.dofs, ctrl.controlDofs, mesh.nodesPeriodic, iip)
+    drop = np.sort([m for group in merge for m in group[1:]]).astype(np.int64)
+    new = np.arange(ty.nni + ty.nnd)
+    for group in merge:
+        new[list(group[1:])] = group[0]
+    new = new - np.searchsorted(drop, new)
+    nnu = ty.nnu - drop.size
+    new[ty.nnu:] += nd * spare
+    dofs = np.concatenate((new[ty.dofs], (nnu + np.arange(nd * spare)).reshape(spare, nd)))
+    rp, col, val = ty.Cdu_csr[:3]
+    tyings = SimpleNamespace(nnu=nnu + nd * spare, nnp=ty.nnp, nnd=ty.nnd, Cdu_csr=(rp, new[col], val),
+                             Cdp_csr=ty.Cdp_csr)
+    vec = gf.Vector(mesh.conn, dofs)
+    x = oracle.Vector(mesh.conn, oracle.dofs(mesh.nnode, nd)).AsElement(mesh.coor)
+    quad = gf.Element.Hex8.Quadrature(x) if nd == 3 else gf.Element.Quad4.QuadraturePlanar(x)
+    rng = np.random.default_rng(sum(size))
+    K, G = rng.uniform(5.0, 15.0, mesh.nelem), np.exp(0.4 * rng.standard_normal(mesh.nelem))
+
+    def dense(coor):
+        et = HEX8 if nd == 3 else QUAD4_PLANAR
+        oq = oracle.Quadrature(et, oracle.Vector(mesh.conn, oracle.dofs(mesh.nnode, nd)).AsElement(coor))
+        C = oracle.elastic_tangent(np.repeat(K[:, None], oq.nip, 1), np.repeat(G[:, None], oq.nip, 1))
+        Ke = oq.Int_gradN_dot_tensor4_dot_gradNT_dV(C)
+        nni = tyings.nnu + tyings.nnp
+        A = np.zeros((nni + tyings.nnd,) * 2)
+        for e in range(mesh.nelem):
+            d = dofs[mesh.conn[e]].ravel()
+            np.add.at(A, np.ix_(d, d), Ke[e])
+        T = np.zeros((tyings.nnd, tyings.nnu))
+        for r in range(tyings.nnd):
+            T[r, new[col[rp[r]:rp[r + 1]]]] += val[rp[r]:rp[r + 1]]
+        u, d = slice(0, tyings.nnu), slice(nni, nni + tyings.nnd)
+        return A[u, u] + A[u, d] @ T + T.T @ A[d, u] + T.T @ A[d, d] @ T
+
+    return mesh, vec, quad, K, G, tyings, dense
+
+
+@pytest.mark.parametrize("size", [(10, 9), (32, 8), (5, 4, 6)])
+@pytest.mark.parametrize("kind", ["merged", "spare"])
+def test_cells_whose_unknowns_are_not_one_per_node(gf, size, kind):
+    """A Regular cell in which unknowns of several nodes are one (rigid parts), and one with unknowns that no
+    element uses: the product sums every node of an unknown, and is zero where there is none (1e-13: FP64 sums
+    of some ten terms).  Such cells are no grid of unknowns, so the general operator takes them."""
+    nd = len(size)
+    merge = [(3 * nd, 3 * nd + nd, 3 * nd + 2 * nd), (1, 8 * nd + 1)] if kind == "merged" else []
+    mesh, vec, quad, K, G, ty, dense = tied_cell(gf, size, merge, 2 if kind == "spare" else 0)
+    P = gf.TyingsPCG(vec, quad, K, G, ty)
+    A = dense(mesh.coor)
+    rng = np.random.default_rng(3)
+    for _ in range(2):  # the second product finds the first one's result in the pool
+        xu = rng.standard_normal(ty.nnu)
+        y = host(P.apply(xu))
+        assert np.linalg.norm(y - A @ xu) <= 1e-13 * np.linalg.norm(A @ xu)
+    assert not P.structured
+    if kind == "merged":
+        b = A @ xu
+        x, _, res = P.solve(b, tol=1e-10)
+        assert res <= 1e-9 and np.linalg.norm(b - A @ host(x)) <= 1e-9 * np.linalg.norm(b)
