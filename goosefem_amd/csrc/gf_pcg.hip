@@ -31,6 +31,7 @@ const double* quad_vol(gf_quad q);
 int64_t quad_nelem(gf_quad q);
 int quad_nip(gf_quad q);
 int quad_etype(gf_quad q);
+uint64_t quad_version(gf_quad q);
 } // namespace gf
 
 namespace {
@@ -62,7 +63,9 @@ struct gf_pcg_s {
     DBuf<double> scal;     // [8]: rz (2 slots), bb, rr, tol2, ...
     DBuf<int32_t> state;   // [0] done, [1] iterations, [2] maxiter
     // structured periodic operator (Regular cell, periodic tyings, uniform geometry)
-    bool structured = false;
+    bool cell = false;       // the mesh, numbering and tyings are such a cell's
+    bool structured = false; // ... and the geometry of version `geom` of the quadrature is uniform
+    uint64_t geom = 0;
     int snx = 0, sny = 0, snz = 0, ntiles = 0, ntx = 0, per_xcd = 0;
     double sh_g[32] = {}, sh_v[4] = {};
     DBuf<int32_t> sidx; // [nodes of the cell * nd] u-DOF of grid node component c, or -1
@@ -895,7 +898,7 @@ void apply(gf_pcg_s* P, const double* xu, const double* xp, double* yu, bool xu_
            const double* w, double* partial, const int32_t* state)
 {
     auto v = P->v;
-    if (P->structured && !xp) {
+    if (P->structured && P->geom == quad_version(P->q) && !xp) {
         const double* xs = xu_in_full ? P->xfull.p : xu;
         if ((!w || w == xs) && P->et == GF_HEX8) {
             k_apply_periodic_h8<8, 8, 4><<<P->ntiles, 256, 0, s>>>(P->snx, P->sny, P->snz, P->ntx, P->nty, P->ke8.p,
@@ -1011,10 +1014,10 @@ bool one_place_per_unknown(const std::vector<int32_t>& sidx, int64_t nnu)
     return found == nnu;
 }
 
-// Regular nx x ny Quad4 cell (at least 8 elements each way: a halo row wraps onto a line of its own)
-// with one unknown per free node and component, whose dependent DOFs are periodic copies (C_du rows = one unit entry of the partner's u-DOF, or empty
-// when the partner is prescribed) and whose elements share one geometry: then K' x_u is applied by
-// k_apply_periodic_q4.
+// Regular nx x ny Quad4 cell (at least 8 elements each way: a halo row wraps onto a line of its own) with
+// one unknown per free node and component and periodic copies as dependent DOFs (C_du rows = one unit entry
+// of the partner's u-DOF, or empty when the partner is prescribed): K' x_u is applied by k_apply_periodic_q4
+// while the elements share one geometry (shared_geometry).
 void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_col_h, const double* cdu_val_h)
 {
     constexpr int TX = 32, TY = 8;
@@ -1050,11 +1053,6 @@ void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_co
                 else if (cnt != 0)
                     return;
             }
-    // uniform geometry: every element's dN/dx and dV equal element 0's to 1e-12 relative (a Regular
-    // mesh gives the same Jacobian everywhere up to the rounding of the coordinate sums, ~1e-16)
-    std::vector<double> g(32), vol(4);
-    if (!uniform_per_element(quad_dNx(P->q), P->nelem, 32, g.data())) return;
-    if (!uniform_per_element(quad_vol(P->q), P->nelem, 4, vol.data())) return;
     std::vector<int32_t> sidx(static_cast<size_t>(nx * ny * 2));
     for (int64_t j = 0; j < ny; ++j)
         for (int64_t i = 0; i < nx; ++i)
@@ -1065,33 +1063,15 @@ void detect_structured(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_co
     if (!one_place_per_unknown(sidx, P->nnu)) return;
     P->sidx.alloc(sidx.size());
     GF_HIP(hipMemcpy(P->sidx.p, sidx.data(), sidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    for (int k = 0; k < 32; ++k) P->sh_g[k] = g[k];
-    for (int k = 0; k < 4; ++k) P->sh_v[k] = vol[k];
     P->snx = static_cast<int>(nx);
     P->sny = static_cast<int>(ny);
     P->ntx = static_cast<int>((nx + TX - 1) / TX);
     P->ntiles = P->ntx * static_cast<int>((ny + TY - 1) / TY);
     P->per_xcd = P->ntiles % 8 == 0 ? P->ntiles / 8 : 0;
-    // K_e = k EK + g EG: EK(2m+j, 2n+l) = sum_q dV dNx(m,j) dNx(n,l), EG(2m+j, 2n+l) =
-    // sum_q dV [dNx(m,l) dNx(n,j) + delta_jl dNx(m).dNx(n) - 2/3 dNx(m,j) dNx(n,l)]
-    for (int q = 0; q < 4; ++q)
-        for (int m = 0; m < 4; ++m)
-            for (int o = 0; o < 4; ++o) {
-                const double *a = g.data() + q * 8 + 2 * m, *b = g.data() + q * 8 + 2 * o;
-                const double dot = a[0] * b[0] + a[1] * b[1];
-                for (int j = 0; j < 2; ++j)
-                    for (int l = 0; l < 2; ++l) {
-                        P->eq4.k[2 * m + j][2 * o + l] += vol[q] * a[j] * b[l];
-                        P->eq4.g[2 * m + j][2 * o + l] +=
-                            vol[q] * (a[l] * b[j] + (j == l ? dot : 0.0) - 2.0 / 3.0 * a[j] * b[l]);
-                    }
-            }
-    alloc_single_reduction(P);
-    P->structured = true;
+    P->cell = true;
 }
 
-// Hex8 Regular nx x ny x nz cell (at least 4 elements each way) with periodic copies as dependent DOFs
-// and identical element geometry (to 1e-12): K' x_u is applied by k_apply_periodic_h8 with
+// Hex8 Regular nx x ny x nz cell (at least 4 elements each way), likewise: k_apply_periodic_h8 with
 // K_e = K KK + G KG.
 void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* cdu_col_h, const double* cdu_val_h)
 {
@@ -1132,28 +1112,6 @@ void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* c
                     else if (cnt != 0)
                         return;
                 }
-    constexpr int NGE = 8 * 8 * 3;
-    std::vector<double> g(NGE), vol(8);
-    if (!uniform_per_element(quad_dNx(P->q), P->nelem, NGE, g.data())) return;
-    if (!uniform_per_element(quad_vol(P->q), P->nelem, 8, vol.data())) return;
-    // KK(m*3+j, n*3+k) = sum_q dV dNx(m,j) dNx(n,k)
-    // KG(m*3+j, n*3+k) = sum_q dV [dNx(m,k) dNx(n,j) + delta_jk dNx(m).dNx(n) - 2/3 dNx(m,j) dNx(n,k)]
-    std::vector<double> kkg(2 * 576, 0.0);
-    for (int q = 0; q < 8; ++q) {
-        const double* gq = g.data() + q * 24;
-        const double dv = vol[q];
-        for (int m = 0; m < 8; ++m)
-            for (int nn = 0; nn < 8; ++nn) {
-                const double dot = gq[m * 3] * gq[nn * 3] + gq[m * 3 + 1] * gq[nn * 3 + 1] + gq[m * 3 + 2] * gq[nn * 3 + 2];
-                for (int j = 0; j < 3; ++j)
-                    for (int k = 0; k < 3; ++k) {
-                        const int r = m * 3 + j, c = nn * 3 + k;
-                        kkg[r * 24 + c] += dv * gq[m * 3 + j] * gq[nn * 3 + k];
-                        kkg[576 + r * 24 + c] += dv * (gq[m * 3 + k] * gq[nn * 3 + j] + (j == k ? dot : 0.0) -
-                                                       2.0 / 3.0 * gq[m * 3 + j] * gq[nn * 3 + k]);
-                    }
-            }
-    }
     std::vector<int32_t> sidx(static_cast<size_t>(nx * ny * nz * 3));
     for (int64_t k = 0; k < nz; ++k)
         for (int64_t j = 0; j < ny; ++j)
@@ -1165,8 +1123,6 @@ void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* c
     if (!one_place_per_unknown(sidx, P->nnu)) return;
     P->sidx.alloc(sidx.size());
     GF_HIP(hipMemcpy(P->sidx.p, sidx.data(), sidx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    P->ke8.alloc(kkg.size());
-    GF_HIP(hipMemcpy(P->ke8.p, kkg.data(), kkg.size() * sizeof(double), hipMemcpyHostToDevice));
     P->snx = static_cast<int>(nx);
     P->sny = static_cast<int>(ny);
     P->snz = static_cast<int>(nz);
@@ -1174,6 +1130,61 @@ void detect_structured_hex8(gf_pcg P, const int64_t* cdu_ptr_h, const int64_t* c
     P->nty = static_cast<int>((ny + TY - 1) / TY);
     P->ntiles = P->ntx * P->nty * static_cast<int>((nz + TZ - 1) / TZ);
     P->per_xcd = 0;
+    P->cell = true;
+}
+
+// The shared element geometry of a cell, for the quadrature's coordinates in force: structured if every
+// element's dN/dx and dV equal element 0's to 1e-12 relative (a Regular mesh gives the same Jacobian
+// everywhere up to the rounding of the coordinate sums, ~1e-16).  The geometry on the device is complete.
+void shared_geometry(gf_pcg P)
+{
+    P->structured = false;
+    P->geom = quad_version(P->q);
+    const int nq = P->nne, ng = nq * P->nne * P->nd;
+    std::vector<double> g(ng), vol(nq);
+    if (!uniform_per_element(quad_dNx(P->q), P->nelem, ng, g.data())) return;
+    if (!uniform_per_element(quad_vol(P->q), P->nelem, nq, vol.data())) return;
+    if (P->et == GF_HEX8) {
+        // KK(m*3+j, n*3+k) = sum_q dV dNx(m,j) dNx(n,k)
+        // KG(m*3+j, n*3+k) = sum_q dV [dNx(m,k) dNx(n,j) + delta_jk dNx(m).dNx(n) - 2/3 dNx(m,j) dNx(n,k)]
+        std::vector<double> kkg(2 * 576, 0.0);
+        for (int q = 0; q < 8; ++q) {
+            const double* gq = g.data() + q * 24;
+            const double dv = vol[q];
+            for (int m = 0; m < 8; ++m)
+                for (int nn = 0; nn < 8; ++nn) {
+                    const double dot = gq[m * 3] * gq[nn * 3] + gq[m * 3 + 1] * gq[nn * 3 + 1] + gq[m * 3 + 2] * gq[nn * 3 + 2];
+                    for (int j = 0; j < 3; ++j)
+                        for (int k = 0; k < 3; ++k) {
+                            const int r = m * 3 + j, c = nn * 3 + k;
+                            kkg[r * 24 + c] += dv * gq[m * 3 + j] * gq[nn * 3 + k];
+                            kkg[576 + r * 24 + c] += dv * (gq[m * 3 + k] * gq[nn * 3 + j] + (j == k ? dot : 0.0) -
+                                                           2.0 / 3.0 * gq[m * 3 + j] * gq[nn * 3 + k]);
+                        }
+                }
+        }
+        P->ke8.upload(kkg);
+        P->structured = true;
+        return;
+    }
+    for (int k = 0; k < 32; ++k) P->sh_g[k] = g[k];
+    for (int k = 0; k < 4; ++k) P->sh_v[k] = vol[k];
+    P->eq4 = ElemQ4();
+    // K_e = k EK + g EG: EK(2m+j, 2n+l) = sum_q dV dNx(m,j) dNx(n,l), EG(2m+j, 2n+l) =
+    // sum_q dV [dNx(m,l) dNx(n,j) + delta_jl dNx(m).dNx(n) - 2/3 dNx(m,j) dNx(n,l)]
+    for (int q = 0; q < 4; ++q)
+        for (int m = 0; m < 4; ++m)
+            for (int o = 0; o < 4; ++o) {
+                const double *a = g.data() + q * 8 + 2 * m, *b = g.data() + q * 8 + 2 * o;
+                const double dot = a[0] * b[0] + a[1] * b[1];
+                for (int j = 0; j < 2; ++j)
+                    for (int l = 0; l < 2; ++l) {
+                        P->eq4.k[2 * m + j][2 * o + l] += vol[q] * a[j] * b[l];
+                        P->eq4.g[2 * m + j][2 * o + l] +=
+                            vol[q] * (a[l] * b[j] + (j == l ? dot : 0.0) - 2.0 / 3.0 * a[j] * b[l]);
+                    }
+            }
+    if (!P->sgrid.n) alloc_single_reduction(P);
     P->structured = true;
 }
 
@@ -1234,6 +1245,7 @@ int gf_pcg_create(gf_pcg* out, gf_vector v, gf_quad q, const double* K_e, const 
             P->state.alloc(4);
             detect_structured(P, cdu_ptr_h, cdu_col_h, cdu_val_h);
             detect_structured_hex8(P, cdu_ptr_h, cdu_col_h, cdu_val_h);
+            if (P->cell) shared_geometry(P);
             P->partial.alloc(3 * NBR + std::max(NBR, P->ntiles));
             compute_invdiag(P, nullptr);
             GF_HIP(hipDeviceSynchronize());
@@ -1267,7 +1279,7 @@ int gf_pcg_is_structured(gf_pcg P, int* structured)
 {
     return guard([&] {
         GF_REQUIRE(P && structured, "null argument");
-        *structured = P->structured ? 1 : 0;
+        *structured = P->structured && P->geom == quad_version(P->q) ? 1 : 0;
     });
 }
 
@@ -1318,6 +1330,10 @@ int gf_pcg_solve(gf_pcg P, const double* b_u, double* x_u, double tol, int64_t m
         if (check_every <= 0) check_every = 32;
         hipStream_t s = S(stream);
         const int64_t n = P->nnu;
+        if (P->cell && P->geom != quad_version(P->q)) { // update_x since: until here the general operator ran
+            GF_HIP(hipStreamSynchronize(s));
+            shared_geometry(P);
+        }
         // Initial residual of a start (nullptr: zero) -> host (||r0||^2, ||b||^2).  The start goes to
         // the u-part of x_full, where the search direction lives during the iteration.
         auto init = [&](const double* x0) {

@@ -26,6 +26,7 @@ struct gf_quad_s {
     DBuf<double> x, N_d, dNxi_d, w_d, dNx, vol;
     DBuf<float> dNx32, vol32;
     bool have32 = false;
+    uint64_t version = 0; // counts update_x: what was derived from dNx or vol is of one version
 };
 
 namespace {
@@ -1022,6 +1023,7 @@ const double* quad_vol(gf_quad q) { return q->vol.p; }
 int quad_etype(gf_quad q) { return q->et; }
 int64_t quad_nelem(gf_quad q) { return q->nelem; }
 int quad_nip(gf_quad q) { return q->nip; }
+uint64_t quad_version(gf_quad q) { return q->version; }
 } // namespace gf
 
 extern "C" {
@@ -1093,6 +1095,7 @@ int gf_quad_update_x(gf_quad q, const double* x, void* stream)
 {
     return guard([&] {
         GF_REQUIRE(q && x, "null argument");
+        ++q->version;
         if (q->x.n)
             GF_HIP(hipMemcpyAsync(q->x.p, x, q->x.n * sizeof(double), hipMemcpyDeviceToDevice, S(stream)));
         compute_geometry(q, S(stream));

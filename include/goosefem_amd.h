@@ -559,9 +559,10 @@ int gf_pcg_create(gf_pcg* out, gf_vector v, gf_quad q, const double* K_e, const 
                   const int64_t* cdp_ptr_h, const int64_t* cdp_col_h, const double* cdp_val_h);
 int gf_pcg_destroy(gf_pcg p);
 int gf_pcg_sizes(gf_pcg p, int64_t* nnu, int64_t* nnp, int64_t* nnd);
-/* 1 if K' x_u is applied by a fused structured kernel (Quad4 Regular n x n cell, n a multiple of 32,
- * or Hex8 Regular n^3 cell, n a multiple of 8; periodic tyings; identical element geometry), else 0
- * (general element + gather path) */
+/* 1 if K' x_u is applied by a fused structured kernel (Quad4 Regular cell of at least 8 elements each way,
+ * or Hex8 Regular cell of at least 4; periodic tyings; one unknown per free node and component; identical
+ * element geometry), else 0 (general element + gather path).  After gf_quad_update_x the products take the
+ * general path until the next gf_pcg_solve has looked at the new geometry. */
 int gf_pcg_is_structured(gf_pcg p, int* structured);
 /* replace the per-element moduli (device, FP64 [nelem] each) and recompute the Jacobi diagonal,
  * enqueued on stream: the tied operator of a new material field without rebuilding the tyings

@@ -328,3 +328,29 @@ def test_cells_whose_unknowns_are_not_one_per_node(gf, size, kind):
         b = A @ xu
         x, _, res = P.solve(b, tol=1e-10)
         assert res <= 1e-9 and np.linalg.norm(b - A @ host(x)) <= 1e-9 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("size", [(10, 9), (32, 8), (5, 4, 6)])
+def test_operator_follows_the_quadrature(gf, size):
+    """update_x on the quadrature of an operator: products and solves are those of the coordinates in force,
+    uneven ones (no shared geometry, so no structured kernel), even ones again, and stretched ones."""
+    mesh, vec, quad, K, G, ty, dense = tied_cell(gf, size)
+    P = gf.TyingsPCG(vec, quad, K, G, ty)
+    assert P.structured
+    nd = len(size)
+    rng = np.random.default_rng(4)
+    uneven = mesh.coor + 0.1 * np.sin(2.0 * np.pi * mesh.coor / np.array(size)[None, ::-1])
+    for coor, even in ((mesh.coor, True), (uneven, False), (mesh.coor, True), (mesh.coor * (1.5, 0.75, 2.0)[:nd], True)):
+        quad.update_x(oracle.Vector(mesh.conn, oracle.dofs(mesh.nnode, nd)).AsElement(coor))
+        A = dense(coor)
+        xu = rng.standard_normal(ty.nnu)
+        y = host(P.apply(xu))
+        assert np.linalg.norm(y - A @ xu) <= 1e-13 * np.linalg.norm(A @ xu)
+        P.set_moduli(K, G)
+        assert np.allclose(host(P.inverse_diagonal), 1.0 / np.diag(A), rtol=1e-13)
+        b = A @ xu
+        x, _, res = P.solve(b, tol=1e-10)
+        assert res <= 1e-9 and np.linalg.norm(b - A @ host(x)) <= 1e-9 * np.linalg.norm(b)
+        assert P.structured == even
+        y = host(P.apply(xu))
+        assert np.linalg.norm(y - A @ xu) <= 1e-13 * np.linalg.norm(A @ xu)
