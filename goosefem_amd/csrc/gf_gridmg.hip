@@ -30,6 +30,7 @@
 #include <cmath>
 #include <mutex>
 
+#include "gf_gridlines.hpp"
 #include "gf_gridmg.hpp"
 #include "gf_wave.hpp"
 
@@ -79,29 +80,10 @@ struct Level {
 
 __host__ __device__ inline bool is_line(int f, int n, int per) { return !(f & 1) || (!per && f == n); }
 
-// wrapped index of a line at most one direction's length out of range, or -1 outside an unwrapped
-// direction
-__device__ inline int wrap(int f, int m, int per)
-{
-    if (f < 0) return per ? f + m : -1;
-    if (f >= m) return per ? f - m : -1;
-    return f;
-}
-
-// ... of any line (a tile is wider than a small wrapped grid)
-__device__ inline int wrap_far(int f, int m, int per)
-{
-    if (per && m < 64) {
-        f %= m;
-        return f < 0 ? f + m : f;
-    }
-    return wrap(f, m, per);
-}
-
 // weights with which fine lines f - 1, f, f + 1 contribute to the coarse line that lies on f
 __device__ inline void restrict_weights(int f, int n, int m, int per, int c, double (&w)[3])
 {
-    const int a = wrap(f - 1, m, per), b = wrap(f + 1, m, per);
+    const int a = wrap_line(f - 1, m, per), b = wrap_line(f + 1, m, per);
     w[0] = c && a >= 0 && !is_line(a, n, per) ? 0.5 : 0.0;
     w[1] = 1.0;
     w[2] = c && b >= 0 && !is_line(b, n, per) ? 0.5 : 0.0;
@@ -116,7 +98,7 @@ __device__ inline double weight(int f, int k, int n, int m, int per, int c)
     const int p = line_of(k, n, c);
     if (f == p) return 1.0;
     if (!c || is_line(f, n, per)) return 0.0;
-    return f == wrap(p - 1, m, per) || f == wrap(p + 1, m, per) ? 0.5 : 0.0;
+    return f == wrap_line(p - 1, m, per) || f == wrap_line(p + 1, m, per) ? 0.5 : 0.0;
 }
 
 __device__ inline void load_stencil(const Level& L, int node, double (&S)[36])
@@ -172,7 +154,7 @@ __global__ void __launch_bounds__(BS) k_mg_galerkin(Level L, Level C)
     const int s = t / C.n, I = t - s * C.n;
     const int ky = I / C.mx, kx = I - ky * C.mx;
     double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    const int jx = wrap(kx + s % 3 - 1, C.mx, C.perx), jy = wrap(ky + s / 3 - 1, C.my, C.pery);
+    const int jx = wrap_line(kx + s % 3 - 1, C.mx, C.perx), jy = wrap_line(ky + s / 3 - 1, C.my, C.pery);
     if (jx >= 0 && jy >= 0) {
         const int px = line_of(kx, L.nx, L.cx), py = line_of(ky, L.ny, L.cy);
         double rx[3], ry[3];
@@ -181,11 +163,11 @@ __global__ void __launch_bounds__(BS) k_mg_galerkin(Level L, Level C)
         for (int i = 0; i < 9; ++i) {
             const double w = rx[i % 3] * ry[i / 3];
             if (w == 0.0) continue;
-            const int fx = wrap(px + i % 3 - 1, L.mx, L.perx), fy = wrap(py + i / 3 - 1, L.my, L.pery);
+            const int fx = wrap_line(px + i % 3 - 1, L.mx, L.perx), fy = wrap_line(py + i / 3 - 1, L.my, L.pery);
             double vx[3], vy[3]; // weights of the fine neighbours of (fx, fy) from (jx, jy)
 #pragma unroll
             for (int o = 0; o < 3; ++o) {
-                const int gx = wrap(fx + o - 1, L.mx, L.perx), gy = wrap(fy + o - 1, L.my, L.pery);
+                const int gx = wrap_line(fx + o - 1, L.mx, L.perx), gy = wrap_line(fy + o - 1, L.my, L.pery);
                 vx[o] = gx < 0 ? 0.0 : weight(gx, jx, L.nx, L.mx, L.perx, L.cx);
                 vy[o] = gy < 0 ? 0.0 : weight(gy, jy, L.ny, L.my, L.pery, L.cy);
             }
@@ -225,7 +207,7 @@ __global__ void __launch_bounds__(DT) k_mg_dense(Level C, double* __restrict__ i
     __syncthreads();
     for (int t = threadIdx.x; t < 9 * C.n; t += DT) {
         const int s = t / C.n, I = t - s * C.n, ky = I / C.mx, kx = I - ky * C.mx;
-        const int jx = wrap(kx + s % 3 - 1, C.mx, C.perx), jy = wrap(ky + s / 3 - 1, C.my, C.pery);
+        const int jx = wrap_line(kx + s % 3 - 1, C.mx, C.perx), jy = wrap_line(ky + s / 3 - 1, C.my, C.pery);
         if (jx < 0 || jy < 0) continue;
         const int J = jy * C.mx + jx;
         for (int a = 0; a < 2; ++a)
@@ -313,8 +295,8 @@ __global__ void __launch_bounds__(NT) k_mg_down(Level L, Level C, Cheb ch, Fine 
     if (state[0]) return;
     __shared__ double2 s_d[NT];
     const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
-    const int ux = blockIdx.x * DX + lx - HD, uy = blockIdx.y * DY + ly - HD;
-    const int gx = wrap_far(ux, L.mx, L.perx), gy = wrap_far(uy, L.my, L.pery);
+    const int ux = tile_raw<TX, HD>(blockIdx.x, lx), uy = tile_raw<TY, HD>(blockIdx.y, ly);
+    const int gx = tile_line<TX, HD>(blockIdx.x, lx, L.mx, L.perx), gy = tile_line<TY, HD>(blockIdx.y, ly, L.my, L.pery);
     const bool in = gx >= 0 && gy >= 0;
     const int node = in ? gy * L.mx + gx : 0;
     const bool own = lx >= HD && lx < TX - HD && ly >= HD && ly < TY - HD && ux < L.mx && uy < L.my;
@@ -403,8 +385,8 @@ __global__ void __launch_bounds__(NT) k_mg_up(Level L, Level C, Cheb ch, const d
     if (state[0]) return;
     __shared__ double2 s_d[NT];
     const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
-    const int ux = blockIdx.x * UX + lx - HU, uy = blockIdx.y * UY + ly - HU;
-    const int gx = wrap_far(ux, L.mx, L.perx), gy = wrap_far(uy, L.my, L.pery);
+    const int ux = tile_raw<TX, HU>(blockIdx.x, lx), uy = tile_raw<TY, HU>(blockIdx.y, ly);
+    const int gx = tile_line<TX, HU>(blockIdx.x, lx, L.mx, L.perx), gy = tile_line<TY, HU>(blockIdx.y, ly, L.my, L.pery);
     const bool in = gx >= 0 && gy >= 0;
     const int node = in ? gy * L.mx + gx : 0;
     const bool own = lx >= HU && lx < TX - HU && ly >= HU && ly < TY - HU && ux < L.mx && uy < L.my;
@@ -475,8 +457,8 @@ __global__ void __launch_bounds__(CT) k_mg_coarse(CoarseArgs A, Cheb ch, const i
         int at[3], dy[3];
 #pragma unroll
         for (int o = 0; o < 3; ++o) {
-            at[o] = max(wrap(gx + o - 1, L.mx, L.perx), 0);
-            dy[o] = max(wrap(gy + o - 1, L.my, L.pery), 0) * L.mx;
+            at[o] = max(wrap_line(gx + o - 1, L.mx, L.perx), 0);
+            dy[o] = max(wrap_line(gy + o - 1, L.my, L.pery), 0) * L.mx;
         }
         double2 r = s_b[off + node];
         double2 d = make_double2(ch.it * (di.x * r.x), ch.it * (di.y * r.y)), x = d;
@@ -507,8 +489,8 @@ __global__ void __launch_bounds__(CT) k_mg_coarse(CoarseArgs A, Cheb ch, const i
             int fx[3], fy[3];
 #pragma unroll
             for (int o = 0; o < 3; ++o) {
-                fx[o] = max(wrap(px + o - 1, L.mx, L.perx), 0);
-                fy[o] = max(wrap(py + o - 1, L.my, L.pery), 0) * L.mx;
+                fx[o] = max(wrap_line(px + o - 1, L.mx, L.perx), 0);
+                fy[o] = max(wrap_line(py + o - 1, L.my, L.pery), 0) * L.mx;
             }
             double2 c = make_double2(0.0, 0.0);
 #pragma unroll
@@ -553,8 +535,8 @@ __global__ void __launch_bounds__(CT) k_mg_coarse(CoarseArgs A, Cheb ch, const i
         int at[3], dy[3];
 #pragma unroll
         for (int o = 0; o < 3; ++o) {
-            at[o] = max(wrap(gx + o - 1, L.mx, L.perx), 0);
-            dy[o] = max(wrap(gy + o - 1, L.my, L.pery), 0) * L.mx;
+            at[o] = max(wrap_line(gx + o - 1, L.mx, L.perx), 0);
+            dy[o] = max(wrap_line(gy + o - 1, L.my, L.pery), 0) * L.mx;
         }
         const double2 pe = prolong(L, C, s_x + coff, gx, gy);
         double2 x = s_x[off + node], r = s_b[off + node];
@@ -603,8 +585,8 @@ __global__ void __launch_bounds__(ANT) k_mg_apply(Level L, const double2* __rest
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int t = min(static_cast<int>(threadIdx.x) + j * ANT, HX * HY - 1);
-        const int hx = wrap(static_cast<int>(blockIdx.x) * AX + t % HX - 1, L.mx, L.perx),
-                  hy = wrap(static_cast<int>(blockIdx.y) * AY + t / HX - 1, L.my, L.pery);
+        const int hx = tile_line_ring<HX, 1>(blockIdx.x, t % HX, L.mx, L.perx),
+                  hy = tile_line_ring<HY, 1>(blockIdx.y, t / HX, L.my, L.pery);
         const bool ok = hx >= 0 && hy >= 0;
         const int h = ok ? hy * L.mx + hx : 0;
         hz[j] = z[h];
@@ -670,7 +652,7 @@ __global__ void __launch_bounds__(BS) k_mg_residual(Level L, const double2* __re
     const int gy = t / L.mx, gx = t - gy * L.mx;
     double2 v = rhs[t];
     for (int s = 0; s < 9; ++s) {
-        const int jx = wrap(gx + s % 3 - 1, L.mx, L.perx), jy = wrap(gy + s / 3 - 1, L.my, L.pery);
+        const int jx = wrap_line(gx + s % 3 - 1, L.mx, L.perx), jy = wrap_line(gy + s / 3 - 1, L.my, L.pery);
         if (jx < 0 || jy < 0) continue;
         const double2 p = x[jy * L.mx + jx];
         const double* S = L.st + static_cast<int64_t>(4 * s) * L.n + t;
