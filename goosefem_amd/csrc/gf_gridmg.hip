@@ -289,10 +289,14 @@ struct Fine {
 // the latency of a launch and its dependent loads, not the 2.7 times redundant halo.
 // FINE: b is the residual after the conjugate-gradient update, formed on the halo too (r and q are read
 // there), and written with x and the partials of r.r for the tile's own nodes.
+//
+// (*) Workgroup 0 may raise the flag in this launch while waves of others are still to read it.  A wave that
+// reads it early must not leave the reduction's barriers to the rest of its workgroup: every wave goes
+// through the reduction, and those that read no flag come to the same decision from the same sum.
 template <bool FINE>
 __global__ void __launch_bounds__(NT) k_mg_down(Level L, Level C, Cheb ch, Fine F, const int32_t* __restrict__ state)
 {
-    if (state[0]) return;
+    const int done = state[0];
     __shared__ double2 s_d[NT];
     const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
     const int ux = tile_raw<TX, HD>(blockIdx.x, lx), uy = tile_raw<TY, HD>(blockIdx.y, ly);
@@ -310,6 +314,7 @@ __global__ void __launch_bounds__(NT) k_mg_down(Level L, Level C, Cheb ch, Fine 
             double pq = 0.0;
             for (int i = threadIdx.x; i < F.npq; i += NT) pq += F.pq[i];
             pq = block_sum<NT>(pq);
+            if (done) return; // (*)
             const double alpha = F.scal[(F.it - 1) & 1] / pq;
             if (!(pq > 0.0)) { // not positive definite (or not a number): the same in every workgroup
                 if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) F.state[0] = 4;
@@ -325,12 +330,15 @@ __global__ void __launch_bounds__(NT) k_mg_down(Level L, Level C, Cheb ch, Fine 
                 F.xsol[node] = x;
             }
         }
+        else if (done) return;
         if (own) F.rnew[node] = r;
         const double rr = block_sum<NT>(own ? r.x * r.x + r.y * r.y : 0.0);
         if (threadIdx.x == 0) F.part[blockIdx.y * gridDim.x + blockIdx.x] = rr;
     }
-    else
+    else {
+        if (done) return;
         r = L.b[node];
+    }
     if (!in) {
         r = make_double2(0.0, 0.0);
         di = r;
@@ -564,7 +572,8 @@ __global__ void __launch_bounds__(CT) k_mg_coarse(CoarseArgs A, Cheb ch, const i
 }
 
 // p = z + beta p_prev on the tile and its ring, q = A p, partials of p.q; block 0 records r.z and the
-// iteration count and raises done at convergence (r.r <= tol^2 b.b) or at a breakdown.
+// iteration count and raises done at convergence (r.r <= tol^2 b.b) or at a breakdown.  The flag is tested
+// behind the reduction, as in k_mg_down (*).
 __global__ void __launch_bounds__(ANT) k_mg_apply(Level L, const double2* __restrict__ z,
                                                   const double2* __restrict__ pold, double2* __restrict__ pnew,
                                                   double2* __restrict__ q, const double* __restrict__ rr_part, int nrr,
@@ -572,7 +581,7 @@ __global__ void __launch_bounds__(ANT) k_mg_apply(Level L, const double2* __rest
                                                   double* __restrict__ pq_part, double* __restrict__ scal,
                                                   int32_t* __restrict__ state, int it)
 {
-    if (state[0]) return;
+    const int done = state[0];
     constexpr int HX = AX + 2, HY = AY + 2;
     __shared__ double2 s_p[HX * HY];
     const int lx = threadIdx.x % AX, ly = threadIdx.x / AX;
@@ -597,6 +606,7 @@ __global__ void __launch_bounds__(ANT) k_mg_apply(Level L, const double2* __rest
     for (int i = threadIdx.x; i < nrr; i += ANT) rr += rr_part[i];
     for (int i = threadIdx.x; i < nrz; i += ANT) rz += rz_part[i];
     block_sum3<ANT>(rr, rz, none);
+    if (done) return;
     const bool first = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
     if (first) state[1] = it;
     if (rr <= scal[4] || !(rz > 0.0) || !isfinite(rz)) {

@@ -164,3 +164,24 @@ def test_tied_cell(gf, nx, ny):
     ref = (T @ xi)[ty.dofs]
     assert np.linalg.norm(got - ref) <= 1e6 * solver.tol * np.linalg.norm(ref)
     assert np.array_equal(got, host(solver.Solve(A, b, x)))
+
+
+def test_breakdown_on_the_way(gf):
+    # an indefinite matrix whose negative modes show after some iterations, on a grid of many workgroups: the
+    # method stops in all of them at once and hands over, the same way every time
+    rng = np.random.default_rng(7)
+    coor, conn = oracle.quad4_regular(130, 60)
+    dofs = np.arange(coor.size).reshape(coor.shape)
+    A = gf.MatrixPartitioned(conn, dofs, dofs[:131].ravel())
+    A.assemble(stiffness(conn, coor, rng) - 2e-3 * np.eye(8))
+    b_u = rng.standard_normal(A.nnu)
+    solver = gf.MatrixPartitionedSolver(tol=1e-8, maxiter=400)
+    seen = []
+    for _ in range(3):
+        try:
+            seen.append(("solved", host(solver.Solve_u(A, b_u, np.zeros(A.nnp))).tobytes()))
+            assert solver.relres <= 10 * solver.tol
+        except gf.GooseFEMError as e:
+            assert e.code == gf.GF_ENOTCONV
+            seen.append(str(e))
+    assert seen[0] == seen[1] == seen[2]
