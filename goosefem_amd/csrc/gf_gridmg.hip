@@ -196,12 +196,14 @@ __global__ void __launch_bounds__(BS) k_mg_galerkin(Level L, Level C)
         for (int b = 0; b < 2; ++b) C.st[static_cast<int64_t>((s * 2 + a) * 2 + b) * C.n + I] = acc[a][b];
 }
 
-// dense inverse of the coarsest operator (prescribed components: the identity), Gauss-Jordan without
-// pivoting (symmetric positive definite) in one workgroup
-__global__ void __launch_bounds__(DT) k_mg_dense(Level C, double* __restrict__ inv)
+// Dense inverse of the coarsest operator (prescribed components: the identity), Gauss-Jordan without
+// pivoting (symmetric positive definite) in one workgroup.  *unfit = 1 where a pivot is lost to rounding, that
+// is below 1e-12 of its diagonal entry (72 rows of sums leave about 1e-14): the operator of a plate or cell
+// that is free to move or turn.  Its "inverse" would add a motion of any size to the solution.
+__global__ void __launch_bounds__(DT) k_mg_dense(Level C, double* __restrict__ inv, int32_t* __restrict__ unfit)
 {
     constexpr int N = 2 * CMAX;
-    __shared__ double A[N][N + 1];
+    __shared__ double A[N][N + 1], diag[N];
     const int m = 2 * C.n;
     for (int t = threadIdx.x; t < m * m; t += DT) A[t / m][t % m] = 0.0;
     __syncthreads();
@@ -214,10 +216,17 @@ __global__ void __launch_bounds__(DT) k_mg_dense(Level C, double* __restrict__ i
             for (int b = 0; b < 2; ++b) A[2 * I + a][2 * J + b] = C.st[static_cast<int64_t>((s * 2 + a) * 2 + b) * C.n + I];
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < m; t += DT)
+    for (int t = threadIdx.x; t < m; t += DT) {
         if (A[t][t] == 0.0) A[t][t] = 1.0;
+        diag[t] = A[t][t];
+    }
+    if (threadIdx.x == 0) *unfit = 0;
     __syncthreads();
     for (int k = 0; k < m; ++k) {
+        if (!(A[k][k] > 1e-12 * diag[k])) { // the same for every thread
+            if (threadIdx.x == 0) *unfit = 1;
+            return;
+        }
         const double pv = 1.0 / A[k][k];
         double v[(N * N + DT - 1) / DT];
 #pragma unroll
@@ -680,7 +689,7 @@ __global__ void __launch_bounds__(BS) k_mg_scalars(const double* __restrict__ bb
     bb = block_sum<BS>(bb);
     if (threadIdx.x != 0) return;
     scal[4] = tol * tol * (bb > 0.0 ? bb : 1.0);
-    state[0] = isfinite(bb) ? 0 : 2;
+    state[0] = !isfinite(bb) ? 2 : state[2] ? 4 : 0; // state[2]: k_mg_dense
     state[1] = 0;
 }
 
@@ -903,7 +912,7 @@ static void refresh(GridMG* M, const double* val, hipStream_t s)
         if (l) k_mg_galerkin<<<nblocks(9 * static_cast<int64_t>(M->L[l].n), BS), BS, 0, s>>>(M->L[l - 1], M->L[l]);
         k_mg_diag<<<nblocks(M->L[l].n, BS), BS, 0, s>>>(M->L[l]);
     }
-    k_mg_dense<<<1, DT, 0, s>>>(M->L[M->nlev - 1], M->inv.p);
+    k_mg_dense<<<1, DT, 0, s>>>(M->L[M->nlev - 1], M->inv.p, M->state.p + 2);
     check_launch();
     M->stale = false;
 }

@@ -185,3 +185,36 @@ def test_breakdown_on_the_way(gf):
             assert e.code == gf.GF_ENOTCONV
             seen.append(str(e))
     assert seen[0] == seen[1] == seen[2]
+
+
+def free_plate(nx, ny, pinned):
+    """A plate with node 0 pinned (free to turn about it) or not held at all, and its rigid motions."""
+    coor, conn = oracle.quad4_regular(nx, ny)
+    dofs = np.arange(coor.size).reshape(coor.shape)
+    turn = np.stack((-coor[:, 1], coor[:, 0]), 1)
+    modes = [turn] if pinned else [np.tile((1.0, 0.0), (coor.shape[0], 1)), np.tile((0.0, 1.0), (coor.shape[0], 1)), turn]
+    fixed = dofs[0] if pinned else dofs[0, :0]
+    return coor, conn, dofs, fixed, np.stack([m.ravel() for m in modes], 1)[np.setdiff1d(dofs, fixed)]
+
+
+@pytest.mark.parametrize("nx,ny,pinned", [(24, 20, True), (24, 20, False), (17, 40, True), (64, 31, False)])
+def test_rigid_motions_are_left_alone(gf, nx, ny, pinned):
+    # Singular but consistent: the Jacobi iteration from zero returns the solution without rigid motion (orthogonal to
+    # the motions in the diagonal's metric, to rounding times iterations); the cycle, whose coarsest inverse is
+    # that of a singular matrix, would add one of any size.
+    coor, conn, dofs, fixed, N = free_plate(nx, ny, pinned)
+    rng = np.random.default_rng(nx)
+    A = gf.MatrixPartitioned(conn, dofs, fixed)
+    A.assemble(stiffness(conn, coor, rng))
+    b_u = rng.standard_normal(A.nnu)
+    Q = np.linalg.qr(N)[0]
+    for _ in range(2):
+        b_u -= Q @ (Q.T @ b_u)
+    rp, cl, v = (host(t) for t in A.csr(0))
+    M = sp.csr_matrix((v, cl, rp), shape=(A.nnu, A.nnu))
+    D = M.diagonal()
+    solver = gf.MatrixPartitionedSolver(tol=1e-10)
+    x = host(solver.Solve_u(A, b_u, np.zeros(A.nnp)))
+    assert np.linalg.norm(b_u - M @ x) <= 10 * solver.tol * np.linalg.norm(b_u)
+    part = np.abs(N.T @ (D * x)) / np.linalg.norm(np.sqrt(D)[:, None] * N, axis=0) / np.linalg.norm(np.sqrt(D) * x)
+    assert part.max() <= 1e-10
