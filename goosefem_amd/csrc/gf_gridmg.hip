@@ -662,7 +662,7 @@ __global__ void __launch_bounds__(BS) k_mg_begin(int n, const int32_t* __restric
     if (threadIdx.x == 0) bb_part[blockIdx.x] = bb;
 }
 
-// r = b - A x (x: the start, null for zero) and the first scalars
+// r = b - A x of a start x
 __global__ void __launch_bounds__(BS) k_mg_residual(Level L, const double2* __restrict__ rhs,
                                                     const double2* __restrict__ x, double2* __restrict__ r)
 {
@@ -704,8 +704,6 @@ __global__ void __launch_bounds__(BS) k_mg_end(int n, const int32_t* __restrict_
     if (u1 >= 0) x[u1] = v.y;
 }
 
-int coarse_lines(int n, int per) { return (n + 1) / 2 + (per ? 0 : 1); }
-
 } // namespace
 
 namespace gf {
@@ -719,28 +717,35 @@ struct GridMG {
     DBuf<int32_t> uidx, src, more_at, more_ptr, more_src, state;
     DBuf<double> part, scal, inv;
     double2 *rhs = nullptr, *xsol = nullptr, *r[2] = {}, *p[2] = {}, *q = nullptr;
-    StatePipe pipe;
+    std::unique_ptr<StatePipe> pipe;
     dim3 gdown[MAXLEV], gup[MAXLEV], gapp;
     int nrr = 0, nrz = 0, npq = 0, nbb = 0;
 };
 
 void GridMGDelete::operator()(GridMG* m) const { delete m; }
 
-GridMGPtr gridmg_create(const gf_vector_s* v, int64_t nnu, const std::function<int64_t(int64_t, int)>& u_of,
-                        const std::vector<int32_t>& rp, const std::vector<int32_t>& cl,
-                        const std::vector<int64_t>& u_of_row)
+bool gridmg_mesh(const gf_vector_s* v)
 {
-    if (v->nne != 4 || v->ndim != 2 || v->nelem < 1 || nnu < 1) return nullptr;
-    // the grid: conn of Mesh::Quad4::Regular (rows of nx elements, nodes left to right, bottom to top)
+    if (v->nne != 4 || v->ndim != 2 || v->nelem < 1) return false;
+    // conn of Mesh::Quad4::Regular (rows of nx elements, nodes left to right, bottom to top)
     const int64_t N1 = v->conn_h[3], nx = N1 - 1;
-    if (nx < 1 || v->nelem % nx != 0) return nullptr;
-    const int64_t ny = v->nelem / nx;
-    if (N1 * (ny + 1) < GRIDMG_MIN_NODES || N1 * (ny + 1) > (int64_t(1) << 26) || v->nnode < N1 * (ny + 1)) return nullptr;
+    if (nx < 1 || v->nelem % nx != 0) return false;
+    const int64_t ny = v->nelem / nx, n = N1 * (ny + 1);
+    // 36 n in 32 bits (the stencil's entries); a column of tiles as the y dimension of a launch
+    if (n < GRIDMG_MIN_NODES || 36 * n >= INT32_MAX || ny + 1 > 65535 * static_cast<int64_t>(DY) || v->nnode < n) return false;
     for (int64_t e = 0; e < v->nelem; ++e) {
         const int64_t a = (e / nx) * N1 + e % nx, want[4] = {a, a + 1, a + N1 + 1, a + N1};
         for (int m = 0; m < 4; ++m)
-            if (v->conn_h[4 * e + m] != want[m]) return nullptr;
+            if (v->conn_h[4 * e + m] != want[m]) return false;
     }
+    return true;
+}
+
+static GridMGPtr build(const gf_vector_s* v, int64_t nnu, const std::function<int64_t(int64_t, int)>& u_of,
+                       const std::function<GridMGMatrix()>& matrix, const std::vector<int64_t>& u_of_row)
+{
+    if (nnu < 1 || !gridmg_mesh(v)) return nullptr;
+    const int64_t N1 = v->conn_h[3], nx = N1 - 1, ny = v->nelem / nx;
     // opposite edges stand for the same unknowns: the direction is wrapped
     auto same = [&](int64_t count, int64_t a0, int64_t b0, int64_t step) {
         bool any = false;
@@ -774,10 +779,11 @@ GridMGPtr gridmg_create(const gf_vector_s* v, int64_t nnu, const std::function<i
         if (at[u] < 0) return nullptr;
     auto M = GridMGPtr(new GridMG());
     M->nnu = nnu;
+    const GridMGMatrix K = matrix();
+    const auto &rp = K.rowptr, &cl = K.col;
     // the CSR entry (or entries) behind every stencil entry; rows that stand for different unknowns
     // write different entries, so only rows that share one are kept off the threads
     const int64_t n0 = static_cast<int64_t>(mx) * my;
-    if (36 * n0 >= INT32_MAX) return nullptr;
     struct Place {
         int32_t x, y, t; // grid line numbers, 2 node + component
     };
@@ -893,7 +899,23 @@ GridMGPtr gridmg_create(const gf_vector_s* v, int64_t nnu, const std::function<i
     M->more_at.upload(mat);
     M->more_ptr.upload(mptr);
     M->more_src.upload(msrc);
+    M->pipe = std::make_unique<StatePipe>();
     return M;
+}
+
+GridMGPtr gridmg_create(const gf_vector_s* v, int64_t nnu, const std::function<int64_t(int64_t, int)>& u_of,
+                        const std::function<GridMGMatrix()>& matrix, const std::vector<int64_t>& u_of_row)
+{
+    try {
+        return build(v, nnu, u_of, matrix, u_of_row);
+    }
+    catch (const Error& e) {
+        if (e.code != GF_ENOMEM) throw;
+        (void)hipGetLastError(); // the failed allocation's, which the next launch check would find
+    }
+    catch (const std::bad_alloc&) {
+    }
+    return nullptr;
 }
 
 void gridmg_invalidate(GridMG* m)
@@ -937,7 +959,7 @@ GridMGStatus gridmg_solve(GridMG* M, const double* val, const double* b, double*
     const int cap = static_cast<int>(std::min<int64_t>(maxiter, 1000));
     constexpr int check_every = 4;
     int32_t st[2] = {0, 0};
-    StatePipe& pipe = M->pipe;
+    StatePipe& pipe = *M->pipe;
     int chunk = 0;
     for (int it = 0; it <= cap && !st[0];) {
         for (int k = 0; k < check_every && it <= cap; ++k, ++it) {

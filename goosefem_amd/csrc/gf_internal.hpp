@@ -8,6 +8,8 @@
 #include <cstdio>
 #include <algorithm>
 #include <cstring>
+#include <exception>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <thread>
@@ -135,7 +137,8 @@ __device__ inline double ordered_gather_sum(int32_t b, int32_t e, const int32_t*
     return s;
 }
 
-// Host-side parallel loop over [0, n) in contiguous chunks (set-up code only).
+// Host-side parallel loop over [0, n) in contiguous chunks (set-up code only).  An exception in a chunk is
+// thrown again here; a chunk whose thread does not start is run by the caller.
 template <class F>
 inline void parallel_for(int64_t n, F&& f)
 {
@@ -144,16 +147,32 @@ inline void parallel_for(int64_t n, F&& f)
         for (int64_t i = 0; i < n; ++i) f(i);
         return;
     }
+    std::exception_ptr err;
+    std::mutex err_mu;
+    auto run = [&](int64_t b, int64_t e) {
+        try {
+            for (int64_t i = b; i < e; ++i) f(i);
+        }
+        catch (...) {
+            std::lock_guard<std::mutex> lock(err_mu);
+            if (!err) err = std::current_exception();
+        }
+    };
     std::vector<std::thread> th;
+    th.reserve(nt);
     int64_t chunk = (n + nt - 1) / nt;
     for (int t = 0; t < nt; ++t) {
-        int64_t b = t * chunk, e = std::min(n, b + chunk);
+        const int64_t b = t * chunk, e = std::min(n, b + chunk);
         if (b >= e) break;
-        th.emplace_back([b, e, &f] {
-            for (int64_t i = b; i < e; ++i) f(i);
-        });
+        try {
+            th.emplace_back(run, b, e);
+        }
+        catch (const std::exception&) {
+            run(b, e);
+        }
     }
     for (auto& t : th) t.join();
+    if (err) std::rethrow_exception(err);
 }
 
 // Hex8 stiffness on MFMA (BF16 hi/lo split, FP32 accumulation), gf_stiffness.hip

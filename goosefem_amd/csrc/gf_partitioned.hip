@@ -41,7 +41,8 @@ struct gf_matpart_s {
     DBuf<double> work; // x_u, x_p, b_u, b_p, then the PCG vectors
     DBuf<double> red;  // reduction partials and scalars
     DBuf<int32_t> state;
-    GridMGPtr mg; // multigrid on A_uu where the mesh is a Regular Quad4 grid (else null)
+    GridMGPtr mg; // multigrid on A_uu where the mesh is a Regular Quad4 grid (else null), by the first solve
+    bool mg_tried = false;
 };
 
 // MatrixPartitionedTyings: the unpartitioned CSR K over the tied DOF numbering [u | p | d] and the
@@ -55,7 +56,9 @@ struct gf_mattyings_s {
     DBuf<double> work; // x, r, z, p, q, invd, rhs [nnu]; xfull, yfull, kdiag [ndof]; p2 [nnu]
     DBuf<double> red;
     DBuf<int32_t> state;
-    GridMGPtr mg; // multigrid on the condensed operator where the cell is a Regular Quad4 grid (else null)
+    GridMGPtr mg; // multigrid on the condensed operator where the cell is a Regular Quad4 grid (else null), by
+                  // the first solve
+    bool mg_tried = false;
 };
 
 namespace {
@@ -928,7 +931,68 @@ void vecpart_as_dofs(gf_vecpart p, int kind, const double* in, double* u, double
     if (rc != GF_OK) throw Error(rc, gf_last_error());
 }
 
-// x_u = A_uu^-1 rhs by Jacobi-PCG from the x_u given (warm) or from zero
+template <class T>
+std::vector<T> host_copy(const DBuf<T>& d)
+{
+    std::vector<T> h(d.n);
+    if (d.n) GF_HIP(hipMemcpy(h.data(), d.p, d.n * sizeof(T), hipMemcpyDeviceToHost));
+    return h;
+}
+
+// the multigrid of A_uu, or null (gridmg_create)
+GridMG* multigrid(gf_matpart A)
+{
+    if (A->mg_tried) return A->mg.get();
+    A->mg_tried = true;
+    const gf_vector v = A->p->v;
+    if (!gridmg_mesh(v)) return nullptr;
+    const int64_t nu = A->nrows[0];
+    std::vector<int64_t> u_of(v->ndof, -1), same(nu);
+    for (int64_t u = 0; u < nu; ++u) u_of[A->p->iiu_h[u]] = same[u] = u;
+    A->mg = gridmg_create(
+        v, nu, [&](int64_t node, int c) { return u_of[v->dofs_h[node * v->ndim + c]]; },
+        [&] { return GridMGMatrix{host_copy(A->rowptr[0]), host_copy(A->col[0])}; }, same);
+    return A->mg.get();
+}
+
+// ... of the condensed operator
+GridMG* multigrid(gf_mattyings A)
+{
+    if (A->mg_tried) return A->mg.get();
+    A->mg_tried = true;
+    const gf_vector v = A->v;
+    if (!gridmg_mesh(v)) return nullptr;
+    // the unknown that a DOF stands for in the condensed system: itself, its partner's if it is a copy of that
+    // one (plus prescribed terms), -1 for none, -2 for a combination
+    const auto rp = host_copy(A->du_rp), cl = host_copy(A->du_cl);
+    const auto val = host_copy(A->du_v);
+    const int64_t nni = A->nnu + A->nnp;
+    std::vector<int64_t> u_of(A->ndof);
+    for (int64_t d = 0; d < A->ndof; ++d) {
+        if (d < nni) u_of[d] = d < A->nnu ? d : -1;
+        else {
+            const int64_t k = rp[d - nni], cnt = rp[d - nni + 1] - k;
+            u_of[d] = cnt == 0 ? -1 : cnt == 1 && val[k] == 1.0 ? cl[k] : -2;
+        }
+    }
+    A->mg = gridmg_create(
+        v, A->nnu, [&](int64_t node, int c) { return u_of[v->dofs_h[node * v->ndim + c]]; },
+        [&] {
+            int64_t n = 0, nnz = 0;
+            const int32_t *krp = nullptr, *kcl = nullptr;
+            const double* kv = nullptr;
+            gf_matrix_sizes(A->K, &n, &nnz);
+            gf_matrix_csr(A->K, &krp, &kcl, &kv);
+            GridMGMatrix K{std::vector<int32_t>(n + 1), std::vector<int32_t>(nnz)};
+            GF_HIP(hipMemcpy(K.rowptr.data(), krp, K.rowptr.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            if (nnz) GF_HIP(hipMemcpy(K.col.data(), kcl, K.col.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+            return K;
+        },
+        u_of);
+    return A->mg.get();
+}
+
+// x_u = A_uu^-1 rhs by PCG from the x_u given (warm) or from zero
 void matpart_cg(gf_matpart A, const double* rhs, double* xu, bool warm, double tol, int64_t maxiter, int64_t* iterations,
                 double* relres, hipStream_t s)
 {
@@ -960,11 +1024,11 @@ void matpart_cg(gf_matpart A, const double* rhs, double* xu, bool warm, double t
         if (relres) *relres = res;
         return res;
     };
-    if (A->mg) {
+    if (GridMG* mg = multigrid(A)) {
         // a Regular Quad4 grid: multigrid-preconditioned iterations, independent of the grid's size
         if (warm) GF_HIP(hipMemcpyAsync(W.cx, xu, n * sizeof(double), hipMemcpyDeviceToDevice, s));
         int64_t its = 0;
-        const GridMGStatus g = gridmg_solve(A->mg.get(), vl, rhs, W.cx, warm, tol, maxiter, &its, s);
+        const GridMGStatus g = gridmg_solve(mg, vl, rhs, W.cx, warm, tol, maxiter, &its, s);
         if (g == GRIDMG_BAD_RHS) throw Error(GF_EINVAL, "non-finite right-hand side");
         // otherwise, and where rounding keeps the true residual from following, the Jacobi iteration below
         if (g == GRIDMG_CONVERGED && finish(its) <= 10.0 * tol) return;
@@ -1092,16 +1156,6 @@ int gf_matpart_create(gf_matpart* out, gf_vecpart p)
                 A->src[b].upload(bsrc[b]);
                 A->val[b].alloc(A->nnz[b]);
             }
-            std::vector<int64_t> same(nu);
-            for (int64_t u = 0; u < nu; ++u) same[u] = u;
-            const auto& dofs = p->v->dofs_h;
-            A->mg = gridmg_create(
-                p->v, nu,
-                [&](int64_t node, int c) {
-                    const int64_t r = renum[dofs[node * p->v->ndim + c]];
-                    return r < nu ? r : int64_t(-1);
-                },
-                brp[0], bcl[0], same);
             A->work.alloc(2 * (nu + np) + 8 * nu);
             A->red.alloc(3 * NPB + 8 + nblocks(LPR * nu, PB));
             A->state.alloc(4);
@@ -1312,28 +1366,6 @@ int gf_mattyings_create(gf_mattyings* out, gf_vector v, int64_t nnu, int64_t nnp
             A->ud_rp.upload(trp);
             A->ud_cl.upload(tcl);
             A->ud_v.upload(tv);
-            // the unknown that a DOF stands for in the condensed system: itself, its partner's if it is a
-            // copy of that one (plus prescribed terms), -1 for none, -2 for a combination
-            const int64_t nni = nnu + nnp;
-            std::vector<int64_t> u_of(A->ndof);
-            for (int64_t d = 0; d < A->ndof; ++d) {
-                if (d < nni) u_of[d] = d < nnu ? d : -1;
-                else {
-                    const int64_t k = du_rp[d - nni], cnt = du_rp[d - nni + 1] - k;
-                    u_of[d] = cnt == 0 ? -1 : cnt == 1 && du_v[k] == 1.0 ? du_cl[k] : -2;
-                }
-            }
-            int64_t knr = 0, knz = 0;
-            gf_matrix_sizes(A->K, &knr, &knz);
-            const int32_t *krp = nullptr, *kcl = nullptr;
-            const double* kv = nullptr;
-            gf_matrix_csr(A->K, &krp, &kcl, &kv);
-            rp.resize(knr + 1);
-            cl.resize(knz);
-            GF_HIP(hipMemcpy(rp.data(), krp, rp.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-            if (knz) GF_HIP(hipMemcpy(cl.data(), kcl, cl.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-            A->mg = gridmg_create(
-                v, nnu, [&](int64_t node, int c) { return u_of[v->dofs_h[node * v->ndim + c]]; }, rp, cl, u_of);
             A->work.alloc(8 * nnu + 3 * A->ndof);
             A->red.alloc(3 * NPB + 8 + nblocks(LPR * nnu, PB)); // + the fused product's p.q partials
             A->state.alloc(4);
@@ -1439,12 +1471,12 @@ int gf_mattyings_solve(gf_mattyings A, const double* b, double* x, double tol, i
         int64_t its = 0;
         double res = 0.0;
         bool solved = nu == 0;
-        if (A->mg) {
+        if (GridMG* mg = nu ? multigrid(A) : nullptr) {
             // a Regular Quad4 cell: multigrid-preconditioned iterations, independent of the grid's size
             const int32_t *krp = nullptr, *kcl = nullptr;
             const double* kv = nullptr;
             gf_matrix_csr(A->K, &krp, &kcl, &kv);
-            const GridMGStatus g = gridmg_solve(A->mg.get(), kv, rhs, cx, false, tol, maxiter, &its, s);
+            const GridMGStatus g = gridmg_solve(mg, kv, rhs, cx, false, tol, maxiter, &its, s);
             if (g == GRIDMG_BAD_RHS) throw Error(GF_EINVAL, "non-finite right-hand side");
             // otherwise, and where rounding keeps the true residual from following, the Jacobi iteration
             if (g == GRIDMG_CONVERGED) {

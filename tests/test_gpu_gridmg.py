@@ -218,3 +218,37 @@ def test_rigid_motions_are_left_alone(gf, nx, ny, pinned):
     assert np.linalg.norm(b_u - M @ x) <= 10 * solver.tol * np.linalg.norm(b_u)
     part = np.abs(N.T @ (D * x)) / np.linalg.norm(np.sqrt(D)[:, None] * N, axis=0) / np.linalg.norm(np.sqrt(D) * x)
     assert part.max() <= 1e-10
+
+
+@pytest.mark.parametrize("tied", [False, True])
+def test_storage_comes_with_the_first_solve(gf, tied):
+    # a matrix that is assembled and multiplied has no multigrid storage (above 500 bytes per node, of which the
+    # allocator's pages leave at least half visible); a solve adds it once
+    import torch
+
+    n = 300
+    mesh = gf.Mesh.Quad4.Regular(n, n)
+    em = torch.eye(8, dtype=torch.float64, device="cuda").expand(mesh.nelem, 8, 8).contiguous()
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    if tied:
+        control = gf.Tyings.Control(mesh.coor, mesh.dofs)
+        iip = np.concatenate((control.controlDofs.ravel(), control.dofs[mesh.nodesOrigin].ravel()))
+        ty = gf.Tyings.Periodic(control.coor, control.dofs, control.controlDofs, mesh.nodesPeriodic, iip)
+        A = gf.MatrixPartitionedTyings(mesh.conn, ty.dofs, ty.Cdu_csr, ty.Cdp_csr)
+        b = torch.ones(control.coor.shape, dtype=torch.float64, device="cuda")
+        solver = gf.MatrixPartitionedTyingsSolver(tol=1e-9)
+    else:
+        A = gf.MatrixPartitioned(mesh.conn, mesh.dofs, mesh.dofs[mesh.nodesBottomEdge].ravel())
+        b = torch.ones(mesh.coor.shape, dtype=torch.float64, device="cuda")
+        solver = gf.MatrixPartitionedSolver(tol=1e-9)
+    at = [free()]
+    for _ in range(2):
+        A.assemble(em)
+        solver.Solve(A, b, torch.zeros_like(b))
+        at.append(free())
+    half = 250 * mesh.nnode
+    assert at[0] - at[1] > half and at[1] - at[2] < half

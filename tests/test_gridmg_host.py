@@ -15,3 +15,7 @@ def run(name):
 
 def test_tiles_read_lines_of_the_grid():
     run("test_gridlines")
+
+
+def test_set_up_without_storage():
+    run("test_gridmg_host")
