@@ -51,6 +51,8 @@ constexpr int CMAX = 36;          // nodes of the coarsest grid
 constexpr int DT = 1024;          // threads of its inversion
 constexpr int CLEV = 8;           // grids that the coarse kernel walks
 constexpr int BS = 256;
+constexpr int NFOLD = 256;        // partial sums that are left of more than these:
+constexpr int FOLD_R = 2048, FOLD_PQ = 1024; // of r.r and r.z; of p.q (k_mg_fold)
 
 // Chebyshev coefficients of the smoother: d = M^-1 r / theta; then d = c1[i] d + c2[i] M^-1 r
 struct Cheb {
@@ -644,6 +646,24 @@ __global__ void __launch_bounds__(ANT) k_mg_apply(Level L, const double2* __rest
     if (threadIdx.x == 0) pq_part[blockIdx.y * gridDim.x + blockIdx.x] = c;
 }
 
+// Partial sums a (y = 0) and b (y = 1) to NFOLD each, every one of a contiguous share in a fixed order.
+// Each workgroup of the kernels that need a sum adds all its partials, so that no launch is spent on it; their
+// number and that of the workgroups both grow with the grid, so large grids fold them first.  us per iteration
+// of an n x n plate without and with it: n = 500 (5,208 partials of r.r and r.z, 1,008 of p.q) 414-418 and 414,
+// folding p.q too 415-418; 600: 467 and 451, with p.q 440; 700: 561 and 530; 1,000: 1,454 and 1,287; 1,500:
+// 3,136 and 2,220; 2,000: 8,372 and 5,035.  300 and below: no difference.
+__global__ void __launch_bounds__(BS) k_mg_fold(const double* __restrict__ a, int na, const double* __restrict__ b, int nb,
+                                                double* __restrict__ out, const int32_t* __restrict__ state)
+{
+    if (state[0]) return;
+    const double* p = blockIdx.y ? b : a;
+    const int n = blockIdx.y ? nb : na, share = (n + NFOLD - 1) / NFOLD, e = min((static_cast<int>(blockIdx.x) + 1) * share, n);
+    double v = 0.0;
+    for (int i = blockIdx.x * share + threadIdx.x; i < e; i += BS) v += p[i];
+    v = block_sum<BS>(v);
+    if (threadIdx.x == 0) out[blockIdx.y * NFOLD + blockIdx.x] = v;
+}
+
 // right-hand side and start on the grid; partials of b.b
 __global__ void __launch_bounds__(BS) k_mg_begin(int n, const int32_t* __restrict__ uidx, const double* __restrict__ b,
                                                  const double* __restrict__ x0, double2* __restrict__ rhs,
@@ -890,7 +910,7 @@ static GridMGPtr build(const gf_vector_s* v, int64_t nnu, const std::function<in
     M->nrz = M->gup[0].x * M->gup[0].y;
     M->npq = M->gapp.x * M->gapp.y;
     M->nbb = nblocks(n0, BS);
-    M->part.alloc(M->nrr + M->nrz + M->npq + M->nbb);
+    M->part.alloc(M->nrr + M->nrz + M->npq + M->nbb + 3 * NFOLD);
     M->scal.alloc(8);
     M->state.alloc(4);
     M->inv.alloc(4 * CMAX * CMAX);
@@ -944,7 +964,8 @@ GridMGStatus gridmg_solve(GridMG* M, const double* val, const double* b, double*
 {
     const int n0 = M->L[0].n, fc = M->first_coarse;
     if (M->stale) refresh(M, val, s);
-    double *rr = M->part.p, *rz = rr + M->nrr, *pq = rz + M->nrz, *bb = pq + M->npq;
+    double *rr = M->part.p, *rz = rr + M->nrr, *pq = rz + M->nrz, *bb = pq + M->npq, *fold = bb + M->nbb;
+    const bool fold_r = M->nrr + M->nrz > FOLD_R, fold_pq = M->npq > FOLD_PQ;
     int32_t* state = M->state.p;
     static const Cheb ch;
     CoarseArgs ca;
@@ -969,8 +990,8 @@ GridMGStatus gridmg_solve(GridMG* M, const double* val, const double* b, double*
             F.p = M->p[(it + 1) & 1];
             F.rnew = M->r[it & 1];
             F.xsol = M->xsol;
-            F.pq = pq;
-            F.npq = M->npq;
+            F.pq = fold_pq ? fold + 2 * NFOLD : pq;
+            F.npq = fold_pq ? NFOLD : M->npq;
             F.part = rr;
             F.scal = M->scal.p;
             F.state = state;
@@ -985,8 +1006,11 @@ GridMGStatus gridmg_solve(GridMG* M, const double* val, const double* b, double*
                 e = M->L[l].y;
             }
             k_mg_up<true><<<M->gup[0], NT, 0, s>>>(M->L[0], M->L[1], ch, M->r[it & 1], e, M->L[0].y, rz, state);
-            k_mg_apply<<<M->gapp, ANT, 0, s>>>(M->L[0], M->L[0].y, M->p[(it + 1) & 1], M->p[it & 1], M->q, rr, M->nrr,
-                                               rz, M->nrz, pq, M->scal.p, state, it);
+            if (fold_r) k_mg_fold<<<dim3(NFOLD, 2), BS, 0, s>>>(rr, M->nrr, rz, M->nrz, fold, state);
+            k_mg_apply<<<M->gapp, ANT, 0, s>>>(M->L[0], M->L[0].y, M->p[(it + 1) & 1], M->p[it & 1], M->q,
+                                               fold_r ? fold : rr, fold_r ? NFOLD : M->nrr, fold_r ? fold + NFOLD : rz,
+                                               fold_r ? NFOLD : M->nrz, pq, M->scal.p, state, it);
+            if (fold_pq) k_mg_fold<<<NFOLD, BS, 0, s>>>(pq, M->npq, nullptr, 0, fold + 2 * NFOLD, state);
         }
         check_launch();
         pipe.post(state, chunk, s);

@@ -252,3 +252,27 @@ def test_storage_comes_with_the_first_solve(gf, tied):
         at.append(free())
     half = 250 * mesh.nnode
     assert at[0] - at[1] > half and at[1] - at[2] < half
+
+
+@pytest.mark.parametrize("nx,ny", [(300, 300), (310, 312), (500, 500), (495, 517), (30, 4100)])
+def test_many_partial_sums(gf, nx, ny):
+    # grids on either side of where the partial sums are folded first (above 2,048 of r.r and r.z, above 1,024 of
+    # p.q; here 1,930 and 380, 2,059 and 390, 5,208 and 1,008, 5,251 and 1,040, 3,420 and 513): the residual
+    # of the CSR is of the tolerance, and the solution repeats bit for bit
+    rng = np.random.default_rng(nx)
+    coor, conn = oracle.quad4_regular(nx, ny)
+    dofs = np.arange(coor.size).reshape(coor.shape)
+    A = gf.MatrixPartitioned(conn, dofs, dofs[: nx + 1].ravel() if ny < 1000 else dofs[:: nx + 1].ravel())
+    import torch
+
+    G = torch.from_numpy(np.exp(0.4 * rng.standard_normal((conn.shape[0], 1)))).cuda().expand(-1, 4).contiguous()
+    quad = gf.Element.Quad4.QuadraturePlanar(coor[conn])
+    A.assemble(quad.Int_gradN_dot_tensor4_dot_gradNT_dV(gf.elastic_tangent(torch.full_like(G, 10.0), G)))
+    b_u = rng.standard_normal(A.nnu)
+    solver = gf.MatrixPartitionedSolver(tol=1e-10)
+    x = host(solver.Solve_u(A, b_u, np.zeros(A.nnp)))
+    rp, cl, v = (host(t) for t in A.csr(0))
+    M = sp.csr_matrix((v, cl, rp), shape=(A.nnu, A.nnu))
+    assert np.linalg.norm(b_u - M @ x) <= 10 * solver.tol * np.linalg.norm(b_u)
+    assert solver.iterations <= 60
+    assert np.array_equal(x, host(solver.Solve_u(A, b_u, np.zeros(A.nnp))))
