@@ -975,9 +975,16 @@ GridMGStatus gridmg_solve(GridMG* M, const double* val, const double* b, double*
     k_mg_begin<<<M->nbb, BS, 0, s>>>(n0, M->uidx.p, b, warm ? x : nullptr, M->rhs, M->xsol, bb);
     k_mg_scalars<<<1, BS, 0, s>>>(bb, M->nbb, tol, M->scal.p, state);
     if (warm) k_mg_residual<<<M->nbb, BS, 0, s>>>(M->L[0], M->rhs, M->xsol, M->r[1]);
-    // The count is a few ten wherever the method is worth it; past the cap the caller's Jacobi
-    // iteration is the better one.  The flag is looked at every 4 iterations, one look behind.
-    const int cap = static_cast<int>(std::min<int64_t>(maxiter, 1000));
+    // The cycle smooths ten times with a scaled diagonal, so an iteration does the work of at least some seven of the
+    // Jacobi iteration and takes the time of about seven, however badly the matrix is scaled: there is no count from
+    // which the caller's iteration would be the better one.  128 x 112 plate, iterations and ms, here / Jacobi:
+    // one phase 10, 1.0 / 1,389, 13.7; K/G = 10^4 261, 18 / 30,572, 297; log-normal moduli over four decades (one
+    // sigma two) to 1e-7 2,111, 146 / 127,284, 1,257; stripes of contrast 10^6 across the load 1,034, 72 /
+    // 9,093, 90; elements 100 times as wide as high 165, 12 / 1,331, 13.  The least favourable: such stripes on
+    // 64 x 64, 223, 14.0 / 1,408, 13.1.  The cap is for matrices that rounding keeps from converging, on which
+    // the caller's iteration mostly fails too: an eighth of its own count.
+    // The flag is looked at every 4 iterations, one look behind.
+    const int cap = static_cast<int>(std::min<int64_t>(maxiter, std::max<int64_t>(1000, maxiter / 8)));
     constexpr int check_every = 4;
     int32_t st[2] = {0, 0};
     StatePipe& pipe = *M->pipe;

@@ -276,3 +276,35 @@ def test_many_partial_sums(gf, nx, ny):
     assert np.linalg.norm(b_u - M @ x) <= 10 * solver.tol * np.linalg.norm(b_u)
     assert solver.iterations <= 60
     assert np.array_equal(x, host(solver.Solve_u(A, b_u, np.zeros(A.nnp))))
+
+
+@pytest.mark.parametrize("case,tol,most", [("stripes", 1e-10, 3000), ("decades", 1e-7, 6000), ("incompressible", 1e-10, 600)])
+def test_badly_scaled_plates(gf, case, tol, most):
+    # the cycle goes on where it converges slowly: stripes of contrast 1e6 across the load (1,034 iterations
+    # against 9,093 of the Jacobi iteration), moduli over many decades (about 1,800 against 49,000), a bulk
+    # modulus 1e4 times the shear modulus (260 against 30,000)
+    import torch
+
+    nx, ny = (64, 64) if case == "decades" else (128, 112)
+    rng = np.random.default_rng(0)
+    coor, conn = oracle.quad4_regular(nx, ny)
+    dofs = np.arange(coor.size).reshape(coor.shape)
+    cx = coor[conn, 0].mean(1)
+    c = np.where((cx // 3).astype(int) % 2 == 0, 1e6, 1.0) if case == "stripes" else np.ones(conn.shape[0])
+    if case == "decades":
+        c = 10.0 ** (2 * rng.standard_normal(conn.shape[0]))
+    K = 1e4 if case == "incompressible" else 10.0
+
+    def dev(a):
+        return torch.from_numpy(np.repeat(a[:, None], 4, 1)).cuda()
+
+    A = gf.MatrixPartitioned(conn, dofs, np.concatenate((dofs[: nx + 1].ravel(), dofs[-nx - 1:].ravel())))
+    quad = gf.Element.Quad4.QuadraturePlanar(coor[conn])
+    A.assemble(quad.Int_gradN_dot_tensor4_dot_gradNT_dV(gf.elastic_tangent(dev(K * c), dev(c))))
+    b_u = rng.standard_normal(A.nnu)
+    solver = gf.MatrixPartitionedSolver(tol=tol)
+    x = host(solver.Solve_u(A, b_u, np.zeros(A.nnp)))
+    rp, cl, v = (host(t) for t in A.csr(0))
+    M = sp.csr_matrix((v, cl, rp), shape=(A.nnu, A.nnu))
+    assert np.linalg.norm(b_u - M @ x) <= 10 * tol * np.linalg.norm(b_u)
+    assert solver.iterations <= most
