@@ -314,6 +314,20 @@ void spmv(gf_matrix_s* A, const double* x, double* y, hipStream_t s)
 
 } // namespace
 
+namespace {
+
+// the product on nodevecs that do not overlap: one kernel, no workspace
+bool dot_disjoint(gf_matrix_s* A, const double* x, double* b, hipStream_t s)
+{
+    const int64_t n = A->v->nnode * A->v->ndim;
+    if (!(b + n <= x || x + n <= b)) return false;
+    if (A->v->identity) spmv<false>(A, x, b, s);
+    else spmv<true>(A, x, b, s);
+    return true;
+}
+
+} // namespace
+
 // exported for the solver translation units
 namespace gf {
 void matrix_spmv(gf_matrix A, const double* x, double* y, hipStream_t s) { spmv<false>(A, x, y, s); }
@@ -602,12 +616,7 @@ int gf_matrix_dot_nodevec(gf_matrix A, const double* x, double* b, void* stream)
         GF_REQUIRE(A && x && b, "null argument");
         if (!A->assembled) throw Error(GF_ESTATE, "matrix not assembled");
         // Matrix.h:804-809: b = AsNode(A * AsDofs(x)) with AsDofs overwriting (last node wins)
-        const int64_t n = A->v->nnode * A->v->ndim;
-        if (b + n <= x || x + n <= b) {
-            if (A->v->identity) spmv<false>(A, x, b, S(stream));
-            else spmv<true>(A, x, b, S(stream));
-            return;
-        }
+        if (dot_disjoint(A, x, b, S(stream))) return;
         // a result written over the operand: through copies
         DBuf<double> xd(A->nrows), bd(A->nrows);
         int rc = gf_vector_as_dofs_nodevec(A->v, x, xd.p, stream);
@@ -656,9 +665,10 @@ int gf_matrix_dot_nodevec_noalloc(gf_matrix A, const double* x, double* b, void*
             throw Error(GF_EINVAL, "gf_matrix_dot_nodevec_noalloc: " + std::to_string(A->nrows) +
                                        " DOFs exceed the static staging of " + std::to_string(NOALLOC_MAX_DOFS) +
                                        " (use gf_matrix_dot_nodevec)");
+        if (dot_disjoint(A, x, b, S(stream))) return;
         double* xd = scratch_ptr();
         double* bd = xd + NOALLOC_MAX_DOFS;
-        // three kernels for the one product of gf_matrix_dot_nodevec; k_row_last writes every DOF of xd, and
+        // a result written over the operand, through the static copies; k_row_last writes every DOF of xd, and
         // the product every row of bd, so nothing left by an earlier call is read
         int rc = gf_vector_as_dofs_nodevec(A->v, x, xd, stream);
         if (rc) throw Error(rc, gf_last_error());

@@ -72,3 +72,25 @@ def test_dot_nodevec_noalloc_rejects_oversize(gf):
     with pytest.raises(gf.GooseFEMError) as e:
         gf._call("gf_matrix_dot_nodevec_noalloc", A._h, gf._dp(x), gf._dp(out), gf._stream())
     assert e.value.code == gf.GF_EINVAL and "exceed" in str(e.value)
+
+
+def test_dot_nodevec_noalloc_on_two_streams(gf):
+    # products that overlap in time on one GPU, and a result written over its operand
+    import torch
+
+    systems = [_system(gf, 60, 45, 1), _system(gf, 61, 44, 2)]
+    refs = [A.Dot(x).cpu().numpy() for A, x in systems]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [[torch.full_like(x, np.nan) for _ in range(50)] for _, x in systems]
+    torch.cuda.synchronize()
+    for k in range(50):
+        for (A, x), s, out in zip(systems, streams, outs):
+            with torch.cuda.stream(s):
+                gf._call("gf_matrix_dot_nodevec_noalloc", A._h, gf._dp(x), gf._dp(out[k]), gf._stream())
+    torch.cuda.synchronize()
+    for ref, out in zip(refs, outs):
+        assert all(np.array_equal(o.cpu().numpy(), ref) for o in out)
+    for (A, x), ref in zip(systems, refs):
+        y = x.clone()
+        gf._call("gf_matrix_dot_nodevec_noalloc", A._h, gf._dp(y), gf._dp(y), gf._stream())
+        assert np.array_equal(y.cpu().numpy(), ref)
