@@ -46,7 +46,7 @@ def test_operand_forms(gf):
 def test_work_goes_to_the_current_stream(gf):
     import torch
 
-    assert gf._stream().value == torch.cuda.current_stream().cuda_stream or torch.cuda.current_stream().cuda_stream == 0
+    assert (gf._stream().value or 0) == torch.cuda.current_stream().cuda_stream  # ctypes: None for a null pointer
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
         assert gf._stream().value == s.cuda_stream
