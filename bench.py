@@ -656,9 +656,11 @@ def bench_statics(args):
     nnu = vector.nnu
     cg_its = sum(its)
     t_it = t_solve / max(cg_its, 1)
-    # per CG iteration: three passes over the fine grid's nine 2 x 2 stencil blocks (down, up, product) and two
-    # over the coarse grids' (a third of the nodes in all), 288 bytes a node each, and 12 vector passes; the
-    # solve's share of the whole (t_solve) also holds the residual, its norms and the host's part
+    # what a CG iteration cannot do without: three passes over the fine grid's nine 2 x 2 stencil blocks (down,
+    # up, product) and two over the coarse grids' (a third of the nodes in all), 288 bytes a node each, and 12
+    # vector passes.  The smoothing tiles read their halo's stencils too (6.4 times on the way down, 3.9 on the
+    # way up: about 290 instead of 82 MB at 256^2, mostly from the caches).  The solve's share of the whole
+    # (t_solve) also holds the residual, its norms and the host's part.
     b_it = mesh.nnode * (3 * 288 + 2 * 288 / 3 + 12 * 16)
     ach = b_it / t_it / 1e9
     res = {
@@ -1019,9 +1021,10 @@ def explicit_general(nx, ny, steps, warmup):
 def api_kernels(kind, n):
     """The unfused quadrature calls of the reference's API (SymGradN_vector, GradN_vector,
     Int_gradN_dot_tensor2_dV; Element.h:634-717, 807-825) on Quad4 planar n x n or Hex8 n^3, FP64
-    and FP32 element data, each timed with HIP events.  Algorithmic bytes per element (FP64; half
-    for FP32): Quad4 gradient dN/dx 256 + elemvec 64 read, qtensor 288 written; integral dN/dx 256 +
-    dV 32 + qtensor 288 read, elemvec 64 written.  Hex8: 1536 + 192 / 576 and 1536 + 64 + 576 / 192."""
+    and FP32 element data, each timed with HIP events.  The bytes per element that a call cannot do without,
+    and moves: the geometry, elemvec (Quad4 64, Hex8 192 in FP64) and qtensor (288, 576).  The geometry is
+    the FP64 element coordinates (64, 192), from which the kernels form dN/dx and dV; FP32 Hex8 reads its stored
+    FP32 dN/dx (768) and, for the integral, dV (32)."""
     import torch
 
     import goosefem_amd as gf
@@ -1032,10 +1035,8 @@ def api_kernels(kind, n):
     quad = gf.Element.Hex8.Quadrature(x) if kind == "hex8" else gf.Element.Quad4.QuadraturePlanar(x)
     del x
     E, nip, nne, nd = mesh.nelem, quad.nip, quad.nne, quad.ndim
-    bytes_grad = nip * nne * nd * 8 + nne * nd * 8 + nip * 9 * 8
-    bytes_int = nip * nne * nd * 8 + nip * 8 + nip * 9 * 8 + nne * nd * 8
     out = {"workload": f"{'Hex8 ' + str(n) + '^3' if kind == 'hex8' else 'Quad4 planar ' + str(n) + '^2'}",
-           "nelem": E, "bytes_per_element_f64": {"gradient": bytes_grad, "integral": bytes_int}}
+           "nelem": E}
     u = torch.from_numpy(gf.randn(11, E * nne * nd)).cuda().reshape(E, nne, nd)
     for dt, nm, scale in ((torch.float64, "f64", 1.0), (torch.float32, "f32", 0.5)):
         ue = u.to(dt)
@@ -1045,16 +1046,13 @@ def api_kernels(kind, n):
         t_grad = _timed(lambda: quad.GradN_vector(ue, out=eps), 10)
         t_int = _timed(lambda: quad.Int_gradN_dot_tensor2_dV(eps, out=fe), 10)
         row = {}
-        for key, t, b in (("SymGradN_vector", t_sym, bytes_grad), ("GradN_vector", t_grad, bytes_grad),
-                          ("Int_gradN_dot_tensor2_dV", t_int, bytes_int)):
-            gbs = scale * b * E / t / 1e9
-            row[key] = {"us": t * 1e6, "achieved_GBs": gbs, "frac": gbs / HBM_PEAK_GBS}
-            if kind == "quad4" or nm == "f64":
-                # the Quad4 kernels and the FP64 Hex8 ones form dN/dx from the FP64 element coordinates: they
-                # move those (64 or 192 B per element), the element vector and the tensors, not the stored dN/dx
-                moved = nne * nd * 8 * (1 + scale) + scale * nip * 9 * 8
-                row[key].update(geometry="recomputed from the element coordinates",
-                                moved_bytes_per_element=moved, frac_moved=moved * E / t / 1e9 / HBM_PEAK_GBS)
+        for key, t in (("SymGradN_vector", t_sym), ("GradN_vector", t_grad), ("Int_gradN_dot_tensor2_dV", t_int)):
+            stored = kind == "hex8" and nm == "f32"
+            geometry = nip * (nne * nd + (key[0] == "I")) * 4 if stored else nne * nd * 8
+            moved = geometry + scale * (nne * nd * 8 + nip * 9 * 8)
+            gbs = moved * E / t / 1e9
+            row[key] = {"us": t * 1e6, "bytes_per_element": moved, "achieved_GBs": gbs, "frac": gbs / HBM_PEAK_GBS,
+                        "geometry": "stored FP32 dN/dx" if stored else "recomputed from the element coordinates"}
         out[nm] = row
         del eps, fe, ue
     del u, quad, vec

@@ -45,3 +45,19 @@ def test_default_line_contract():
     ndof = d["config"].get("ndof")
     if ndof:
         assert abs(d["value"] * d["ms_per_step"] * 1e-3 / ndof - 1.0) < 0.05
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,n,geometry", [("quad4", 700, (64, 64, 64, 64)), ("hex8", 48, (192, 192, 768, 800))])
+def test_quadrature_rows_count_the_bytes_they_move(kind, n, geometry):
+    # geometry + elemvec + qtensor per element: what the kernels move, not the stored geometry they no longer read
+    import bench
+
+    blk = bench.api_kernels(kind, n)
+    vec, ten = (64, 288) if kind == "quad4" else (192, 576)
+    for nm, scale, geo in (("f64", 1.0, geometry[:2]), ("f32", 0.5, geometry[2:])):
+        for key, g in (("SymGradN_vector", geo[0]), ("GradN_vector", geo[0]), ("Int_gradN_dot_tensor2_dV", geo[1])):
+            row = blk[nm][key]
+            assert row["bytes_per_element"] == g + scale * (vec + ten)
+            gbs = row["bytes_per_element"] * blk["nelem"] / row["us"] * 1e-3
+            assert abs(row["achieved_GBs"] / gbs - 1.0) < 1e-9 and abs(row["frac"] * bench.HBM_PEAK_GBS / gbs - 1.0) < 1e-9
