@@ -576,7 +576,7 @@ def bench_newton(args):
     # algorithmic bytes per element (FP64): reads dNx 256, dV 32, u_e 64, (K, G, sigy0, H) 128,
     # Epsp_t 288, epsp_t 32; writes Epsp 288, epsp 32, f_e 64, K_e 512
     b_el = 1696
-    b_plain = 8576  # the unfused chain: Eps, Sig and C written and read back
+    b_plain = 8160  # the unfused chain: Eps, Sig and C written and read back, geometry from the coordinates
     ach = b_el * ne / t_fused / 1e9
     res = {
         "metric": "J2 Newton pass throughput (fused strain + return map + f_e + K_e)",
