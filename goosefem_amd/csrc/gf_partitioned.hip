@@ -218,6 +218,10 @@ __global__ void k_node_from_part_sel(int64_t n, int64_t nnu, int which, const in
 // the NPB partials in the same fixed order.  scal: [0], [1] rz by iteration parity, [2] rr, [3] bb,
 // [4] tol^2 bb.  state: [0] done, [1] iterations, [2] iteration cap.  Every kernel returns at once
 // when done is set, so launches queued past convergence leave the result alone.
+// (*) The kernel that raises done also reads it, so the waves of a workgroup may read it differently.  They
+// count those that saw it raised in their first reduction and leave as a whole, or go on as a whole: what
+// a workgroup does on its own after that (a search direction that nobody uses) is complete, and no wave leaves
+// the barriers to the others.
 constexpr int PB = 256, NPB = 256;
 
 // the workgroup's sum (DPP wavefront sums, waves added in order) stored by thread 0
@@ -316,9 +320,11 @@ __global__ void __launch_bounds__(PB)
                    double* __restrict__ pnew, double* __restrict__ q, const double* __restrict__ rz_rr,
                    double* __restrict__ scal, double* __restrict__ partial, int32_t* __restrict__ state, int64_t it)
 {
-    if (state[0]) return;
+    double rz_new = 0.0, rr_unused = 0.0, done = state[0] ? 1.0 : 0.0;
+    for (int b = threadIdx.x; b < NPB; b += PB) rz_new += rz_rr[b];
+    block_sum3<PB>(rz_new, rr_unused, done);
+    if (done != 0.0) return; // (*)
     const double rz_old = scal[(it - 1) & 1];
-    const double rz_new = block_sum_partials(rz_rr, NPB);
     const double beta = rz_old != 0.0 ? rz_new / rz_old : 0.0;
     if (blockIdx.x == 0) {
         const double rr = block_sum_partials(rz_rr + NPB, NPB);
@@ -579,9 +585,13 @@ __global__ void __launch_bounds__(PB) k_ty_expand_dir(int64_t nnu, int64_t nnp, 
                                                       double* __restrict__ xfull, const double* __restrict__ partial,
                                                       double* __restrict__ scal, int32_t* __restrict__ state, int64_t it)
 {
-    if (state[0]) return;
-    const double rz_new = block_sum_partials(partial, NPB);
-    const double rr = block_sum_partials(partial + NPB, NPB);
+    double rz_new = 0.0, rr = 0.0, done = state[0] ? 1.0 : 0.0;
+    for (int b = threadIdx.x; b < NPB; b += PB) {
+        rz_new += partial[b];
+        rr += partial[NPB + b];
+    }
+    block_sum3<PB>(rz_new, rr, done);
+    if (done != 0.0) return; // (*)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         scal[2] = rr;
         state[1] = static_cast<int32_t>(it); // the updates done

@@ -685,13 +685,14 @@ __global__ void k_expand_dir(int64_t nnu, int64_t nnp, int64_t nnd, const double
                              const double* __restrict__ rz_rr, double* __restrict__ scal, int32_t* __restrict__ state,
                              int64_t it)
 {
-    if (state[0]) return;
-    double rz_new = 0.0, rr = 0.0, unused = 0.0;
+    // every wave passes the reduction's barriers; a workgroup leaves if any of its waves saw the flag raised
+    double rz_new = 0.0, rr = 0.0, done = state[0] ? 1.0 : 0.0;
     for (int i = threadIdx.x; i < NBR; i += BS) {
         rz_new += rz_rr[i];
         rr += rz_rr[NBR + i];
     }
-    block_sum3<BS>(rz_new, rr, unused);
+    block_sum3<BS>(rz_new, rr, done);
+    if (done != 0.0) return;
     if (rr <= scal[4]) { // converged after `it` iterations
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             scal[3] = rr;
@@ -812,8 +813,13 @@ __global__ void __launch_bounds__(BS) k_pcg_direction(int64_t n, const double* _
                                                       double* __restrict__ scal, const double* __restrict__ z,
                                                       double* __restrict__ p, int32_t* __restrict__ state, int64_t it)
 {
-    if (state[0]) return;
-    const double rz_new = reduce_partials(partial), rr = reduce_partials(partial + NBR);
+    double rz_new = 0.0, rr = 0.0, done = state[0] ? 1.0 : 0.0;
+    for (int i = threadIdx.x; i < NBR; i += BS) {
+        rz_new += partial[i];
+        rr += partial[NBR + i];
+    }
+    block_sum3<BS>(rz_new, rr, done);
+    if (done != 0.0) return; // a workgroup as a whole
     const double beta = rz_new / scal[it & 1];
     for (int64_t i = blockIdx.x * static_cast<int64_t>(BS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * BS)
         p[i] = z[i] + beta * p[i];
