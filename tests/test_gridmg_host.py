@@ -8,7 +8,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 def run(name):
     path = os.path.join(ROOT, "tests", "cpp", "_build", name)
-    assert os.path.exists(path), "build it first: __graft_entry__.build() (make -C tests/cpp)"
+    if not os.path.exists(path):
+        subprocess.run(["make", "-s", "-C", os.path.join(ROOT, "tests", "cpp"), f"_build/{name}"], check=True)
     r = subprocess.run([path], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "ALL OK" in r.stdout, (r.returncode, r.stdout, r.stderr)
 
