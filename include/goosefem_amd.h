@@ -283,8 +283,10 @@ int gf_material_elastic_tangent_f32(int64_t nq, int tdim, const double* K_q, con
  * FP64 preconditioned CG instead of an LDLT factorisation, so K'_uu must be symmetric positive
  * definite.  The preconditioner is a multigrid V-cycle where the cell is a Regular Quad4 grid of at
  * least 64 nodes whose dependent DOFs are copies of u DOFs (plus prescribed terms), which makes the
- * iteration count independent of the grid, else (and should that not converge) the diagonal.  C_du [nnd, nnu] and C_dp [nnd, nnp] are host CSR (int64 rowptr / col, FP64
- * values), as Tyings::Periodic::Cdu() / Cdp() (TyingsPeriodic.h:244-256).
+ * iteration count independent of the grid (its storage, some 700 bytes per node, comes with the first
+ * solve); else, and should that not converge or its storage not be had, the diagonal.  C_du [nnd, nnu] and
+ * C_dp [nnd, nnp] are host CSR (int64 rowptr / col, FP64 values), as Tyings::Periodic::Cdu() / Cdp()
+ * (TyingsPeriodic.h:244-256).
  * ============================================================================================== */
 int gf_mattyings_create(gf_mattyings* out, gf_vector v, int64_t nnu, int64_t nnp, int64_t nnd, const int64_t* du_rowptr,
                         const int64_t* du_col, const double* du_val, const int64_t* dp_rowptr, const int64_t* dp_col,
@@ -471,8 +473,9 @@ int gf_matrix_todense(gf_matrix A, double* out, void* stream);
  * (FP64, deterministic reductions), so A_uu must be symmetric positive definite (the reference's
  * SimplicialLDLT also takes indefinite symmetric matrices).  The preconditioner is a multigrid V-cycle
  * where the mesh is a Regular Quad4 grid of at least 64 nodes with one DOF per node and component
- * (opposite edges may share theirs), else (and should that not converge) the diagonal.  set() / add() of dense sub-matrices
- * are not provided (the sparsity pattern is the mesh's).
+ * (opposite edges may share theirs; its storage, some 700 bytes per node, comes with the first solve); else,
+ * and should that not converge or its storage not be had, the diagonal.  set() / add() of dense
+ * sub-matrices are not provided (the sparsity pattern is the mesh's).
  * ============================================================================================== */
 
 /* MatrixPartitioned(conn, dofs, iip)  (MatrixPartitioned.h:87-121) over p's Vector and iip.  Holds
